@@ -592,6 +592,7 @@ void append_table(std::vector<StepEntry>& out, const icarion_domain_desc& d, boo
         } else {
             e.c0 = e.ch = e.c1 = 0.0;
         }
+        fill_fast_entry(e);
         t = t + dt;
     }
 }

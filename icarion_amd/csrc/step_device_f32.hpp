@@ -18,6 +18,10 @@ __device__ __forceinline__ void kahan_add(float& hi, float& lo, float d) {
     hi = t;
 }
 
+// Keeps a wave-uniform branch a branch: without it the compiler computes both
+// sides in every step and selects.
+__device__ __forceinline__ void keep_branch() { asm volatile(""); }
+
 // hardware transcendentals: v_log_f32 (log2), v_exp_f32 (exp2), v_sin/cos_f32
 // (argument in revolutions), v_sqrt_f32, v_rcp_f32
 __device__ __forceinline__ float fast_ln(float u) { return __builtin_amdgcn_logf(u) * 0.69314718056f; }
@@ -27,10 +31,9 @@ __device__ __forceinline__ float fast_sqrt(float x) { return __builtin_amdgcn_sq
 
 
 // c: the stage's RF coefficient (analytic fields) or the stage time (field
-// arrays), in FP64 as the step table holds it.
-template <int FIELD>
-__device__ __forceinline__ f3 field_f32(const StepParams& P, const FastConst& C, f3 p, double c,
-                                        double ez) {
+// arrays, always in FP64); T: float where the caller holds rounded values.
+template <int FIELD, class T>
+__device__ __forceinline__ f3 field_f32(const StepParams& P, const FastConst& C, f3 p, T c, T ez) {
     if constexpr (FIELD == FIELD_LINEAR) {
         const float c_rf = (float)c;
         f3 E{0.0f, 0.0f, (float)ez};
@@ -43,6 +46,7 @@ __device__ __forceinline__ f3 field_f32(const StepParams& P, const FastConst& C,
         const f3 s{p.x - C.ox, p.y - C.oy, p.z - C.oz};
         f3 l = s;
         if (!P.rot_identity) {
+            keep_branch();
             l = f3{C.g2l[0] * s.x + C.g2l[1] * s.y + C.g2l[2] * s.z,
                    C.g2l[3] * s.x + C.g2l[4] * s.y + C.g2l[5] * s.z,
                    C.g2l[6] * s.x + C.g2l[7] * s.y + C.g2l[8] * s.z};
@@ -51,6 +55,7 @@ __device__ __forceinline__ f3 field_f32(const StepParams& P, const FastConst& C,
         const float Cf = 1.0f - C.R_char_sq * __builtin_amdgcn_rcpf(r_sq);
         f3 E{C.orbi_hk * l.x * Cf, C.orbi_hk * l.y * Cf, -C.orbi_k * l.z};
         if (!P.rot_identity) {
+            keep_branch();
             E = f3{C.l2g[0] * E.x + C.l2g[1] * E.y + C.l2g[2] * E.z,
                    C.l2g[3] * E.x + C.l2g[4] * E.y + C.l2g[5] * E.z,
                    C.l2g[6] * E.x + C.l2g[7] * E.y + C.l2g[8] * E.z};
@@ -141,6 +146,7 @@ __device__ __forceinline__ bool contains_f32(const StepParams& P, const FastCons
     const f3 s{px - C.ox, py - C.oy, pz - C.oz};
     f3 l = s;
     if (!P.rot_identity) {
+        keep_branch();
         l = f3{C.g2l[0] * s.x + C.g2l[1] * s.y + C.g2l[2] * s.z,
                C.g2l[3] * s.x + C.g2l[4] * s.y + C.g2l[5] * s.z,
                C.g2l[6] * s.x + C.g2l[7] * s.y + C.g2l[8] * s.z};
@@ -156,8 +162,7 @@ __device__ __forceinline__ bool contains_f32(const StepParams& P, const FastCons
         const float f_out = z2 - 0.5f * (r2 - C.R_out * C.R_out) - C.R_char_sq * (C.ln_R_out - ln_r);
         return f_in >= 0.0f && f_out <= 0.0f;
     }
-    if (l.z < 0.0f || l.z >= C.L) return false;
-    return r2 <= C.R_eps_sq;
+    return !(l.z < 0.0f) & !(l.z >= C.L) & (r2 <= C.R_eps_sq);
 }
 
 __device__ __forceinline__ f3 iso_dir_f32(PhiloxStream& rng) {
@@ -296,9 +301,9 @@ __device__ __forceinline__ f3 gas_velocity_f32(const StepParams& P, const FastCo
 }
 
 // FLOW: the gas velocity at p (gas_velocity_f32), else the constant one.
-template <int FIELD, int COLL, bool FLOW = false>
+template <int FIELD, int COLL, bool FLOW = false, class T>
 __device__ __forceinline__ f3 accel_f32(const StepParams& P, const FastConst& C, f3 p, f3 v,
-                                        double c, double ez, float qm, float lpre) {
+                                        T c, T ez, float qm, float lpre) {
     f3 a = field_f32<FIELD>(P, C, p, c, ez) * qm;
     if constexpr (COLL == COLL_DAMPING) {
         const float g = (P.damping_model == 3) ? lpre / fmaxf(1e-6f, fast_sqrt(dot(v, v))) : lpre;
@@ -308,6 +313,70 @@ __device__ __forceinline__ f3 accel_f32(const StepParams& P, const FastConst& C,
         }
     }
     return a;
+}
+
+// One RK4 or Boris push of the FP32 path: position and velocity increments of
+// the step from (p0, v0).
+template <int INTEG, int FIELD, int COLL, bool FLOW = false>
+__device__ __forceinline__ void push_f32(const StepParams& P, const FastConst& C, const StepEntry& te, f3 p0, f3 v0,
+                                         float qm, float lp, float dt, float half_dt, float h6, f3& dpos, f3& dvel) {
+    if constexpr (INTEG == 0) {
+        if constexpr (FIELD == FIELD_LINEAR && COLL != COLL_DAMPING) {
+            if (!P.has_rf) {
+                // E = (0, 0, E_z(t)) everywhere: the general stages below with
+                // x and y accelerations of zero, whose velocities stay v0
+                const float az1 = te.e0f * qm;
+                const float az2 = te.ehf * qm;
+                const float az4 = te.e1f * qm;
+                const float k2z = v0.z + az1 * half_dt;
+                const float k3z = v0.z + az2 * half_dt;
+                const float k4z = v0.z + az2 * dt;
+                dpos.x = (v0.x + v0.x * 2.0f + v0.x * 2.0f + v0.x) * h6;
+                dpos.y = (v0.y + v0.y * 2.0f + v0.y * 2.0f + v0.y) * h6;
+                dpos.z = (v0.z + k2z * 2.0f + k3z * 2.0f + k4z) * h6;
+                dvel = f3{0.0f, 0.0f, (az1 + az2 * 2.0f + az2 * 2.0f + az4) * h6};
+                return;
+            }
+        }
+        if constexpr (FIELD == FIELD_ARRAY_X) {   // stage times in FP64
+            const f3 k1a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, te.c0, te.e0, qm, lp);
+            const f3 k2v = v0 + k1a * half_dt;
+            const f3 k2a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + v0 * half_dt, k2v, te.ch, te.eh, qm, lp);
+            const f3 k3v = v0 + k2a * half_dt;
+            const f3 k3a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + k2v * half_dt, k3v, te.ch, te.eh, qm, lp);
+            const f3 k4v = v0 + k3a * dt;
+            const f3 k4a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + k3v * dt, k4v, te.c1, te.e1, qm, lp);
+            dpos = (v0 + k2v * 2.0f + k3v * 2.0f + k4v) * h6;
+            dvel = (k1a + k2a * 2.0f + k3a * 2.0f + k4a) * h6;
+        } else {
+            const f3 k1a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, te.c0f, te.e0f, qm, lp);
+            const f3 k2v = v0 + k1a * half_dt;
+            const f3 k2a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + v0 * half_dt, k2v, te.chf, te.ehf, qm, lp);
+            const f3 k3v = v0 + k2a * half_dt;
+            const f3 k3a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + k2v * half_dt, k3v, te.chf, te.ehf, qm, lp);
+            const f3 k4v = v0 + k3a * dt;
+            const f3 k4a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + k3v * dt, k4v, te.c1f, te.e1f, qm, lp);
+            dpos = (v0 + k2v * 2.0f + k3v * 2.0f + k4v) * h6;
+            dvel = (k1a + k2a * 2.0f + k3a * 2.0f + k4a) * h6;
+        }
+    } else {
+        f3 a;
+        if constexpr (FIELD == FIELD_ARRAY_X)
+            a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, te.c0, te.e0, qm, lp);
+        else
+            a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, te.c0f, te.e0f, qm, lp);
+        const f3 vm = v0 + a * half_dt;
+        f3 rot{0.0f, 0.0f, 0.0f};
+        if (P.magnetic) {
+            const f3 tv = f3{(float)P.B[0], (float)P.B[1], (float)P.B[2]} * (qm * half_dt);
+            const float s_f = 2.0f / (1.0f + dot(tv, tv));
+            const f3 vprime = vm + cross(vm, tv);
+            rot = cross(vprime, tv * s_f);
+        }
+        // x += v+ dt, v = v+ + a dt/2 = v0 + a dt + rot (no cancellation)
+        dpos = (vm + rot) * dt;
+        dvel = a * dt + rot;
+    }
 }
 
 }  // namespace icarion

@@ -596,115 +596,98 @@ __device__ __forceinline__ void f32_ion(const StepParams& P, const IonPtrs& S, c
         }
         lpre = (float)l;
     }
-    bool checked = false;
+    // 0: done, 1: stepping, 2: unborn, 3: stepping, position not yet known to
+    // be inside.  A register rather than lane masks, which the compiler would
+    // merge with the execution mask on every path through the loop.
+    uint32_t state = !born ? 2u : active ? 3u : 0u;
     const float dt = (float)P.dt;
     const float half_dt = 0.5f * dt;
     const float h6 = dt * (1.0f / 6.0f);
+    // The loop is wave-uniform and its body one masked region; lanes that leave
+    // one by one cost the scalar unit a third of the step's instructions.  With
+    // the uniform-field push and the FP32 table values this took 200,003 ions x
+    // 10,000 HSS steps from 23.6 to 19.0 ms and 1M ions x 20,000 Boris + kick
+    // steps from 123 to 103 ms (bound by vector issue, 3-4 wavefronts per SIMD).
     for (uint32_t k = 0; k < P.n_steps; ++k) {
-        const StepEntry te = P.table[k];
+        if (__ballot(state != 0u) == 0ull) break;
+        const StepEntry& te = P.table[k];
         const double t = te.t;
-        if (!born) {
-            if (t >= birth) {
+        if (__ballot(state > 1u) != 0ull) {   // before an ion's first step only
+            if (state == 2u && t >= birth) {
                 born = true;
-                active = true;
-                checked = false;
-            } else {
-                continue;
+                state = 3u;
             }
-        }
-        if (!active) break;
-        if (!checked && !contains_f32(P, C, hi[0], hi[1], hi[2])) {
-            active = false;
-            death = t;
-            break;
-        }
-        const float z_before = hi[2];
-        const float z_before_lo = lo[2];
-        // the step's gas density over the domain's (scales gamma and the rates)
-        const float nrel = (float)te.nrel;
-        const float lp = lpre * nrel;
-        const f3 p0{hi[0], hi[1], hi[2]};
-        const f3 v0{hi[3], hi[4], hi[5]};
-        f3 dpos, dvel;
-        if constexpr (INTEG == 0) {
-            const f3 k1a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, te.c0, te.e0, qm, lp);
-            const f3 k2v = v0 + k1a * half_dt;
-            const f3 k2a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + v0 * half_dt, k2v, te.ch, te.eh, qm, lp);
-            const f3 k3v = v0 + k2a * half_dt;
-            const f3 k3a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + k2v * half_dt, k3v, te.ch, te.eh, qm, lp);
-            const f3 k4v = v0 + k3a * dt;
-            const f3 k4a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + k3v * dt, k4v, te.c1, te.e1, qm, lp);
-            dpos = (v0 + k2v * 2.0f + k3v * 2.0f + k4v) * h6;
-            dvel = (k1a + k2a * 2.0f + k3a * 2.0f + k4a) * h6;
-        } else {
-            const f3 a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, te.c0, te.e0, qm, lp);
-            const f3 vm = v0 + a * half_dt;
-            f3 rot{0.0f, 0.0f, 0.0f};
-            if (P.magnetic) {
-                const f3 tv = f3{(float)P.B[0], (float)P.B[1], (float)P.B[2]} * (qm * half_dt);
-                const float s_f = 2.0f / (1.0f + dot(tv, tv));
-                const f3 vprime = vm + cross(vm, tv);
-                rot = cross(vprime, tv * s_f);
-            }
-            // x += v+ dt, v = v+ + a dt/2 = v0 + a dt + rot (no cancellation)
-            dpos = (vm + rot) * dt;
-            dvel = a * dt + rot;
-        }
-        kahan_add(hi[0], lo[0], dpos.x);
-        kahan_add(hi[1], lo[1], dpos.y);
-        kahan_add(hi[2], lo[2], dpos.z);
-        kahan_add(hi[3], lo[3], dvel.x);
-        kahan_add(hi[4], lo[4], dvel.y);
-        kahan_add(hi[5], lo[5], dvel.z);
-        ++pushed;
-        if constexpr (COLL != COLL_NONE) {
-            PhiloxStream rng(P.seed, i, P.step0 + k);
-            f3 v{hi[3], hi[4], hi[5]};
-            const f3 vin = v;
-            // collision substeps: dt / n_sub each, one continuing stream, in the
-            // SUB instantiation (the loop costs the one-stage kernels a
-            // wavefront per SIMD)
-            const int ns = SUB ? P.n_sub : 1;
-            const float sub = SUB ? 1.0f / static_cast<float>(P.n_sub) : 1.0f;
-            const float dtc = SUB ? static_cast<float>(P.dt / static_cast<double>(P.n_sub)) : dt;
-            uint32_t hits = 0;
-            const f3 ug = FLOW ? gas_velocity_f32(P, C, f3{hi[0], hi[1], hi[2]}) : f3{0.0f, 0.0f, 0.0f};
-            for (int s = 0; s < ns; ++s)
-                hits += collide_f32<COLL, FLOW>(P, C, sp, sidx, m, inv_m_plus, lp, kbt2_dt_over_m * sub, v, rng,
-                                                dtc * nrel, C.n_dt * sub * nrel, ug) ? 1u : 0u;
-            if (COLL == COLL_HSS || COLL == COLL_HSS_MIX) {
-                if (hits) {
-                    // a collision replaces the velocity: restart its compensation
-                    hi[3] = v.x; hi[4] = v.y; hi[5] = v.z;
-                    lo[3] = 0.0f; lo[4] = 0.0f; lo[5] = 0.0f;
-                    nc += hits;
-                    ncoll_launch += hits;
+            if (state == 3u) {
+                state = 1u;
+                if (!contains_f32(P, C, hi[0], hi[1], hi[2])) {
+                    state = 0u;
+                    death = t;
                 }
-            } else {
-                kahan_add(hi[3], lo[3], v.x - vin.x);
-                kahan_add(hi[4], lo[4], v.y - vin.y);
-                kahan_add(hi[5], lo[5], v.z - vin.z);
             }
         }
-        if (P.detect && isnan(arrival)) {
-            const double zb = (double)z_before + (double)z_before_lo;
-            const double za = (double)hi[2] + (double)lo[2];
-            if (zb < P.det_z && za >= P.det_z)
-                arrival = t + P.dt * (P.det_z - zb) / (za - zb);
-        }
-        if (!contains_f32(P, C, hi[0], hi[1], hi[2])) {
-            active = false;
-            death = t;
-            break;
-        }
-        checked = true;
-        if (!(isfinite(hi[0]) && isfinite(hi[1]) && isfinite(hi[2]) && isfinite(hi[3]) &&
-              isfinite(hi[4]) && isfinite(hi[5]))) {
-            active = false;
-            death = t;
-            break;
+        if (state == 1u) {
+            const float z_before = hi[2];
+            const float z_before_lo = lo[2];
+            // the step's gas density over the domain's (scales gamma and the rates)
+            const float nrel = te.nrelf;
+            const float lp = lpre * nrel;
+            const f3 p0{hi[0], hi[1], hi[2]};
+            const f3 v0{hi[3], hi[4], hi[5]};
+            f3 dpos, dvel;
+            push_f32<INTEG, FIELD, COLL, FLOW>(P, C, te, p0, v0, qm, lp, dt, half_dt, h6, dpos, dvel);
+            kahan_add(hi[0], lo[0], dpos.x);
+            kahan_add(hi[1], lo[1], dpos.y);
+            kahan_add(hi[2], lo[2], dpos.z);
+            kahan_add(hi[3], lo[3], dvel.x);
+            kahan_add(hi[4], lo[4], dvel.y);
+            kahan_add(hi[5], lo[5], dvel.z);
+            ++pushed;
+            if constexpr (COLL != COLL_NONE) {
+                PhiloxStream rng(P.seed, i, P.step0 + k);
+                f3 v{hi[3], hi[4], hi[5]};
+                const f3 vin = v;
+                // collision substeps: dt / n_sub each, one continuing stream, in the
+                // SUB instantiation (the loop costs the one-stage kernels a
+                // wavefront per SIMD)
+                const int ns = SUB ? P.n_sub : 1;
+                const float sub = SUB ? 1.0f / static_cast<float>(P.n_sub) : 1.0f;
+                const float dtc = SUB ? static_cast<float>(P.dt / static_cast<double>(P.n_sub)) : dt;
+                uint32_t hits = 0;
+                const f3 ug = FLOW ? gas_velocity_f32(P, C, f3{hi[0], hi[1], hi[2]}) : f3{0.0f, 0.0f, 0.0f};
+                for (int s = 0; s < ns; ++s)
+                    hits += collide_f32<COLL, FLOW>(P, C, sp, sidx, m, inv_m_plus, lp, kbt2_dt_over_m * sub, v, rng,
+                                                    dtc * nrel, C.n_dt * sub * nrel, ug) ? 1u : 0u;
+                if (COLL == COLL_HSS || COLL == COLL_HSS_MIX) {
+                    if (hits) {
+                        // a collision replaces the velocity: restart its compensation
+                        hi[3] = v.x; hi[4] = v.y; hi[5] = v.z;
+                        lo[3] = 0.0f; lo[4] = 0.0f; lo[5] = 0.0f;
+                        nc += hits;
+                        ncoll_launch += hits;
+                    }
+                } else {
+                    kahan_add(hi[3], lo[3], v.x - vin.x);
+                    kahan_add(hi[4], lo[4], v.y - vin.y);
+                    kahan_add(hi[5], lo[5], v.z - vin.z);
+                }
+            }
+            if (P.detect) {
+                keep_branch();
+                if (isnan(arrival)) {
+                    const double zb = (double)z_before + (double)z_before_lo;
+                    const double za = (double)hi[2] + (double)lo[2];
+                    if (zb < P.det_z && za >= P.det_z)
+                        arrival = t + P.dt * (P.det_z - zb) / (za - zb);
+                }
+            }
+            if (!(contains_f32(P, C, hi[0], hi[1], hi[2]) & isfinite(hi[0]) & isfinite(hi[1]) & isfinite(hi[2]) &
+                  isfinite(hi[3]) & isfinite(hi[4]) & isfinite(hi[5]))) {
+                state = 0u;
+                death = t;
+            }
         }
     }
+    if (state != 2u) active = state != 0u;
     S.x[i] = (double)hi[0] + (double)lo[0];
     S.y[i] = (double)hi[1] + (double)lo[1];
     S.z[i] = (double)hi[2] + (double)lo[2];
@@ -798,29 +781,7 @@ __device__ __forceinline__ void surr_ion(const StepParams& P, const IonPtrs& S, 
             const f3 p0{hi[0], hi[1], hi[2]};
             const f3 v0{hi[3], hi[4], hi[5]};
             f3 dpos, dvel;
-            if constexpr (INTEG == 0) {
-                const f3 k1a = accel_f32<FIELD, COLL_NONE>(P, C, p0, v0, te.c0, te.e0, qm, 0.f);
-                const f3 k2v = v0 + k1a * half_dt;
-                const f3 k2a = accel_f32<FIELD, COLL_NONE>(P, C, p0 + v0 * half_dt, k2v, te.ch, te.eh, qm, 0.f);
-                const f3 k3v = v0 + k2a * half_dt;
-                const f3 k3a = accel_f32<FIELD, COLL_NONE>(P, C, p0 + k2v * half_dt, k3v, te.ch, te.eh, qm, 0.f);
-                const f3 k4v = v0 + k3a * dt;
-                const f3 k4a = accel_f32<FIELD, COLL_NONE>(P, C, p0 + k3v * dt, k4v, te.c1, te.e1, qm, 0.f);
-                dpos = (v0 + k2v * 2.0f + k3v * 2.0f + k4v) * h6;
-                dvel = (k1a + k2a * 2.0f + k3a * 2.0f + k4a) * h6;
-            } else {
-                const f3 a = accel_f32<FIELD, COLL_NONE>(P, C, p0, v0, te.c0, te.e0, qm, 0.f);
-                const f3 vmid = v0 + a * half_dt;
-                f3 rot{0.0f, 0.0f, 0.0f};
-                if (P.magnetic) {
-                    const f3 tv = f3{(float)P.B[0], (float)P.B[1], (float)P.B[2]} * (qm * half_dt);
-                    const float s_f = 2.0f / (1.0f + dot(tv, tv));
-                    const f3 vprime = vmid + cross(vmid, tv);
-                    rot = cross(vprime, tv * s_f);
-                }
-                dpos = (vmid + rot) * dt;
-                dvel = a * dt + rot;
-            }
+            push_f32<INTEG, FIELD, COLL_NONE>(P, C, te, p0, v0, qm, 0.f, dt, half_dt, h6, dpos, dvel);
             kahan_add(hi[0], lo[0], dpos.x);
             kahan_add(hi[1], lo[1], dpos.y);
             kahan_add(hi[2], lo[2], dpos.z);
@@ -841,7 +802,7 @@ __device__ __forceinline__ void surr_ion(const StepParams& P, const IonPtrs& S, 
                 vm = fast_sqrt(dot(vrel, vrel));
                 if (vm >= (float)kMinRelativeVelocity) {
                     // n dt of the step (the density ratio of a pressure waveform)
-                    const float x = C.n_dt * (float)te.nrel * sigma * vm;
+                    const float x = C.n_dt * te.nrelf * sigma * vm;
                     const float Pc = x < 1e-3f ? x * (1.0f - 0.5f * x * (1.0f - x * (1.0f / 3.0f)))
                                                : 1.0f - __builtin_amdgcn_exp2f(-x * 1.44269504089f);
                     if (rng.uniform_f32() < Pc) {

@@ -67,7 +67,20 @@ struct StepEntry {
     double eh;
     double e1;
     double nrel;
+    // c0, ch, c1, e0, eh, e1, nrel rounded once for the FP32 kernels, whose
+    // waves would otherwise convert each of them on the vector pipe every step
+    float c0f, chf, c1f, e0f, ehf, e1f, nrelf, padf;
 };
+inline void fill_fast_entry(StepEntry& e) {
+    e.c0f = static_cast<float>(e.c0);
+    e.chf = static_cast<float>(e.ch);
+    e.c1f = static_cast<float>(e.c1);
+    e.e0f = static_cast<float>(e.e0);
+    e.ehf = static_cast<float>(e.eh);
+    e.e1f = static_cast<float>(e.e1);
+    e.nrelf = static_cast<float>(e.nrel);
+    e.padf = 0.0f;
+}
 
 struct IonPtrs {
     double *x, *y, *z, *vx, *vy, *vz;
