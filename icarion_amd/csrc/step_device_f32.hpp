@@ -30,10 +30,22 @@ __device__ __forceinline__ float fast_sin_rev(float r) { return __builtin_amdgcn
 __device__ __forceinline__ float fast_sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 
 
+// The corner values of the grid cell an ion is in.  An ion crosses a cell in
+// hundreds to thousands of steps, so a caller that keeps this across the stages
+// and steps reloads the eight corners only when the cell changes (24 registers
+// more).  Gathering them at every stage, the RK4 kernel waited on four dependent
+// gathers per step: 1M ions x 2000 HSS steps on a 96 x 96 x 192 grid took 71 ms
+// of kernel time, now 29 ms (82 -> 41 ms for the whole call), bound by vector
+// issue.
+struct CellF32 {
+    uint64_t node = ~0ull;   // the cell's first node
+    f3 e[8];                 // corner 4 dx + 2 dy + dz
+};
+
 // c: the stage's RF coefficient (analytic fields) or the stage time (field
 // arrays, always in FP64); T: float where the caller holds rounded values.
 template <int FIELD, class T>
-__device__ __forceinline__ f3 field_f32(const StepParams& P, const FastConst& C, f3 p, T c, T ez) {
+__device__ __forceinline__ f3 field_f32(const StepParams& P, const FastConst& C, f3 p, T c, T ez, CellF32& cell) {
     if constexpr (FIELD == FIELD_LINEAR) {
         const float c_rf = (float)c;
         f3 E{0.0f, 0.0f, (float)ez};
@@ -64,16 +76,13 @@ __device__ __forceinline__ f3 field_f32(const StepParams& P, const FastConst& C,
     } else {
         // trilinear on float4 nodes; the axis search of the FP64 path on
         // non-uniform axes
+        // (branch-free: the clamped ends are selected over the interior value)
         auto loc = [](float v, float v0, float vl, float inv_d, int n, int& i0, float& a) {
-            if (v <= v0) { i0 = 0; a = 0.0f; }
-            else if (v >= vl) { i0 = n - 2; a = 1.0f; }
-            else {
-                const float f = (v - v0) * inv_d;
-                int i = static_cast<int>(f);
-                i = i > n - 2 ? n - 2 : (i < 0 ? 0 : i);
-                i0 = i;
-                a = f - static_cast<float>(i);
-            }
+            const float f = (v - v0) * inv_d;
+            const int i = min(static_cast<int>(f), n - 2);   // negative only below v0
+            const bool below = v <= v0, above = v >= vl;
+            a = below ? 0.0f : above ? 1.0f : f - static_cast<float>(i);
+            i0 = below ? 0 : above ? n - 2 : i;
         };
         auto loc_axis = [](const float* __restrict__ ax, int n, float v, int& i0, float& a) {
             if (v <= ax[0]) { i0 = 0; a = 0.0f; }
@@ -98,26 +107,41 @@ __device__ __forceinline__ f3 field_f32(const StepParams& P, const FastConst& C,
             loc_axis(P.axf_y, P.ny, p.y, iy, ay);
             loc_axis(P.axf_z, P.nz, p.z, iz, az);
         } else {
-            loc(p.x, (float)P.x0, (float)P.x_last, (float)P.inv_dx, P.nx, ix, ax);
-            loc(p.y, (float)P.y0, (float)P.y_last, (float)P.inv_dy, P.ny, iy, ay);
-            loc(p.z, (float)P.z0, (float)P.z_last, (float)P.inv_dz, P.nz, iz, az);
+            loc(p.x, C.fa_first[0], C.fa_last[0], C.fa_inv[0], P.nx, ix, ax);
+            loc(p.y, C.fa_first[1], C.fa_last[1], C.fa_inv[1], P.ny, iy, ay);
+            loc(p.z, C.fa_first[2], C.fa_last[2], C.fa_inv[2], P.nz, iz, az);
         }
-        const size_t sy = static_cast<size_t>(P.nx), sz = static_cast<size_t>(P.nx) * P.ny;
-        const size_t base = ix + sy * iy + sz * iz;
         f3 r{0.0f, 0.0f, 0.0f};
+        const size_t sy = static_cast<size_t>(P.nx), sz = static_cast<size_t>(P.nx) * P.ny;
         if (!GEN || P.n_terms <= 1) {
+            // the cell's first node by two 32 x 32 -> 64-bit multiply-adds, the
+            // other three rows by one 64-bit add each; the second node of a
+            // row is an offset of the load
+            const uint32_t row = static_cast<uint32_t>(iy) + static_cast<uint32_t>(P.ny) * static_cast<uint32_t>(iz);
+            const uint64_t node = static_cast<uint64_t>(row) * static_cast<uint32_t>(P.nx) + static_cast<uint32_t>(ix);
+            const char* const p00 = reinterpret_cast<const char*>(P.fa_f32) + 16 * node;
+            if (node != cell.node) {
+                cell.node = node;
+#pragma unroll
+                for (int c4 = 0; c4 < 4; ++c4) {
+                    const float4* const q = reinterpret_cast<const float4*>(p00 + 16 * ((c4 >> 1) * sy + (c4 & 1) * sz));
+                    const float4 lo4 = q[0], hi4 = q[1];
+                    cell.e[c4] = f3{lo4.x, lo4.y, lo4.z};
+                    cell.e[4 + c4] = f3{hi4.x, hi4.y, hi4.z};
+                }
+            }
 #pragma unroll
             for (int c8 = 0; c8 < 8; ++c8) {
                 const int dx = c8 >> 2, dy = (c8 >> 1) & 1, dzz = c8 & 1;
                 const float w = (dx ? ax : 1.0f - ax) * (dy ? ay : 1.0f - ay) * (dzz ? az : 1.0f - az);
-                const float4 e = P.fa_f32[base + dx + dy * sy + dzz * sz];
-                r.x += w * e.x;
-                r.y += w * e.y;
-                r.z += w * e.z;
+                r.x += w * cell.e[c8].x;
+                r.y += w * cell.e[c8].y;
+                r.z += w * cell.e[c8].z;
             }
         } else {
             // the time factors in FP64 (phase never in FP32), applied in FP32
             const int nt = P.n_terms;
+            const size_t base = ix + sy * iy + sz * iz;
             for (int j = 0; j < nt; ++j) {
                 const float sj = (float)term_scale_f64(P, j, c);
                 f3 e{0.0f, 0.0f, 0.0f};
@@ -133,7 +157,7 @@ __device__ __forceinline__ f3 field_f32(const StepParams& P, const FastConst& C,
                 r = r + e * sj;
             }
         }
-        const float s = (float)P.fa_scale;
+        const float s = C.fa_scale;
         if (s != 1.0f) r = r * s;
         return r;
     }
@@ -303,8 +327,8 @@ __device__ __forceinline__ f3 gas_velocity_f32(const StepParams& P, const FastCo
 // FLOW: the gas velocity at p (gas_velocity_f32), else the constant one.
 template <int FIELD, int COLL, bool FLOW = false, class T>
 __device__ __forceinline__ f3 accel_f32(const StepParams& P, const FastConst& C, f3 p, f3 v,
-                                        T c, T ez, float qm, float lpre) {
-    f3 a = field_f32<FIELD>(P, C, p, c, ez) * qm;
+                                        T c, T ez, float qm, float lpre, CellF32& cell) {
+    f3 a = field_f32<FIELD>(P, C, p, c, ez, cell) * qm;
     if constexpr (COLL == COLL_DAMPING) {
         const float g = (P.damping_model == 3) ? lpre / fmaxf(1e-6f, fast_sqrt(dot(v, v))) : lpre;
         if (g > 0.0f) {
@@ -315,11 +339,19 @@ __device__ __forceinline__ f3 accel_f32(const StepParams& P, const FastConst& C,
     return a;
 }
 
+template <int FIELD, int COLL, bool FLOW = false, class T>
+__device__ __forceinline__ f3 accel_f32(const StepParams& P, const FastConst& C, f3 p, f3 v,
+                                        T c, T ez, float qm, float lpre) {
+    CellF32 cell;
+    return accel_f32<FIELD, COLL, FLOW>(P, C, p, v, c, ez, qm, lpre, cell);
+}
+
 // One RK4 or Boris push of the FP32 path: position and velocity increments of
 // the step from (p0, v0).
 template <int INTEG, int FIELD, int COLL, bool FLOW = false>
 __device__ __forceinline__ void push_f32(const StepParams& P, const FastConst& C, const StepEntry& te, f3 p0, f3 v0,
-                                         float qm, float lp, float dt, float half_dt, float h6, f3& dpos, f3& dvel) {
+                                         float qm, float lp, float dt, float half_dt, float h6, CellF32& cell, f3& dpos,
+                                         f3& dvel) {
     if constexpr (INTEG == 0) {
         if constexpr (FIELD == FIELD_LINEAR && COLL != COLL_DAMPING) {
             if (!P.has_rf) {
@@ -339,32 +371,32 @@ __device__ __forceinline__ void push_f32(const StepParams& P, const FastConst& C
             }
         }
         if constexpr (FIELD == FIELD_ARRAY_X) {   // stage times in FP64
-            const f3 k1a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, te.c0, te.e0, qm, lp);
+            const f3 k1a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, te.c0, te.e0, qm, lp, cell);
             const f3 k2v = v0 + k1a * half_dt;
-            const f3 k2a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + v0 * half_dt, k2v, te.ch, te.eh, qm, lp);
+            const f3 k2a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + v0 * half_dt, k2v, te.ch, te.eh, qm, lp, cell);
             const f3 k3v = v0 + k2a * half_dt;
-            const f3 k3a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + k2v * half_dt, k3v, te.ch, te.eh, qm, lp);
+            const f3 k3a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + k2v * half_dt, k3v, te.ch, te.eh, qm, lp, cell);
             const f3 k4v = v0 + k3a * dt;
-            const f3 k4a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + k3v * dt, k4v, te.c1, te.e1, qm, lp);
+            const f3 k4a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + k3v * dt, k4v, te.c1, te.e1, qm, lp, cell);
             dpos = (v0 + k2v * 2.0f + k3v * 2.0f + k4v) * h6;
             dvel = (k1a + k2a * 2.0f + k3a * 2.0f + k4a) * h6;
         } else {
-            const f3 k1a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, te.c0f, te.e0f, qm, lp);
+            const f3 k1a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, te.c0f, te.e0f, qm, lp, cell);
             const f3 k2v = v0 + k1a * half_dt;
-            const f3 k2a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + v0 * half_dt, k2v, te.chf, te.ehf, qm, lp);
+            const f3 k2a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + v0 * half_dt, k2v, te.chf, te.ehf, qm, lp, cell);
             const f3 k3v = v0 + k2a * half_dt;
-            const f3 k3a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + k2v * half_dt, k3v, te.chf, te.ehf, qm, lp);
+            const f3 k3a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + k2v * half_dt, k3v, te.chf, te.ehf, qm, lp, cell);
             const f3 k4v = v0 + k3a * dt;
-            const f3 k4a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + k3v * dt, k4v, te.c1f, te.e1f, qm, lp);
+            const f3 k4a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + k3v * dt, k4v, te.c1f, te.e1f, qm, lp, cell);
             dpos = (v0 + k2v * 2.0f + k3v * 2.0f + k4v) * h6;
             dvel = (k1a + k2a * 2.0f + k3a * 2.0f + k4a) * h6;
         }
     } else {
         f3 a;
         if constexpr (FIELD == FIELD_ARRAY_X)
-            a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, te.c0, te.e0, qm, lp);
+            a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, te.c0, te.e0, qm, lp, cell);
         else
-            a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, te.c0f, te.e0f, qm, lp);
+            a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, te.c0f, te.e0f, qm, lp, cell);
         const f3 vm = v0 + a * half_dt;
         f3 rot{0.0f, 0.0f, 0.0f};
         if (P.magnetic) {

@@ -600,6 +600,7 @@ __device__ __forceinline__ void f32_ion(const StepParams& P, const IonPtrs& S, c
     // be inside.  A register rather than lane masks, which the compiler would
     // merge with the execution mask on every path through the loop.
     uint32_t state = !born ? 2u : active ? 3u : 0u;
+    CellF32 cell;
     const float dt = (float)P.dt;
     const float half_dt = 0.5f * dt;
     const float h6 = dt * (1.0f / 6.0f);
@@ -634,7 +635,7 @@ __device__ __forceinline__ void f32_ion(const StepParams& P, const IonPtrs& S, c
             const f3 p0{hi[0], hi[1], hi[2]};
             const f3 v0{hi[3], hi[4], hi[5]};
             f3 dpos, dvel;
-            push_f32<INTEG, FIELD, COLL, FLOW>(P, C, te, p0, v0, qm, lp, dt, half_dt, h6, dpos, dvel);
+            push_f32<INTEG, FIELD, COLL, FLOW>(P, C, te, p0, v0, qm, lp, dt, half_dt, h6, cell, dpos, dvel);
             kahan_add(hi[0], lo[0], dpos.x);
             kahan_add(hi[1], lo[1], dpos.y);
             kahan_add(hi[2], lo[2], dpos.z);
@@ -755,6 +756,7 @@ __device__ __forceinline__ void surr_ion(const StepParams& P, const IonPtrs& S, 
     const float dt = (float)P.dt;
     const float half_dt = 0.5f * dt;
     const float h6 = dt * (1.0f / 6.0f);
+    CellF32 cell;
     // the next step's table entry is loaded one step ahead
     StepEntry te_next = P.n_steps ? P.table[0] : StepEntry{};
     for (uint32_t k = 0; k < P.n_steps; ++k) {
@@ -781,7 +783,7 @@ __device__ __forceinline__ void surr_ion(const StepParams& P, const IonPtrs& S, 
             const f3 p0{hi[0], hi[1], hi[2]};
             const f3 v0{hi[3], hi[4], hi[5]};
             f3 dpos, dvel;
-            push_f32<INTEG, FIELD, COLL_NONE>(P, C, te, p0, v0, qm, 0.f, dt, half_dt, h6, dpos, dvel);
+            push_f32<INTEG, FIELD, COLL_NONE>(P, C, te, p0, v0, qm, 0.f, dt, half_dt, h6, cell, dpos, dvel);
             kahan_add(hi[0], lo[0], dpos.x);
             kahan_add(hi[1], lo[1], dpos.y);
             kahan_add(hi[2], lo[2], dpos.z);

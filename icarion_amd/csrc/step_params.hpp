@@ -133,6 +133,8 @@ struct FastConst {
     float m_gas;
     float L, half_L, R_eps_sq, R_in_sq, R_out, R_out_sq, ln_R_in, ln_R_out;
     float g2l[9], l2g[9];
+    // field array: first and last node and reciprocal spacing per axis, scale
+    float fa_first[3], fa_last[3], fa_inv[3], fa_scale;
 };
 
 struct StepParams {
@@ -281,6 +283,14 @@ inline void fill_fast_const(StepParams& P) {
         C.g2l[c] = (float)P.g2l[c];
         C.l2g[c] = (float)P.l2g[c];
     }
+    const double first[3] = {P.x0, P.y0, P.z0}, last[3] = {P.x_last, P.y_last, P.z_last};
+    const double inv[3] = {P.inv_dx, P.inv_dy, P.inv_dz};
+    for (int c = 0; c < 3; ++c) {
+        C.fa_first[c] = (float)first[c];
+        C.fa_last[c] = (float)last[c];
+        C.fa_inv[c] = (float)inv[c];
+    }
+    C.fa_scale = (float)P.fa_scale;
 }
 
 // ---- several domains ---------------------------------------------------------
