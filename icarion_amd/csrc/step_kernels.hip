@@ -166,24 +166,31 @@ __global__ void __launch_bounds__(256) step_f64_kernel(const StepParams P, const
 
 // ======================= FP64 geometry EHSS, wave-cooperative ===============
 //
-// The plain EHSS method of ehss_f64 / ehss_core_f64 with the work of one
-// collision spread over the whole wavefront.  Each lane pushes its own ion and
-// runs its own collision test (the handler's Maxwellian neutral and
-// P = 1 - exp(-n sigma_eff |v_rel| dt)); then the wavefront takes the ions that
-// collide one after another, and for each of them:
-//   * its random stream is handed to every lane (the stream is counter-based,
-//     so every lane draws the same numbers the ion's own lane would);
-//   * atom j of its cluster is handled by lane j mod 64: b_max is a wave max
-//     over the rotated atoms' radial extents, and for each impact parameter
-//     the first contact is a wave min over (s_hit, j) - the smallest s_hit,
-//     the lowest atom index among equal ones, which is the sequential loop's
-//     choice (CollisionKernels.cpp:283-381);
-//   * every lane forms the contact normal of the winning atom with the
-//     sequential loop's arithmetic, and the reflected velocity; the ion's lane
-//     keeps it.
-// So the wavefront spends the atoms x attempts work of the collisions it has,
-// instead of waiting on its slowest lane while the lanes without a collision
-// idle.
+// The plain EHSS method of ehss_f64 / ehss_core_f64 with a collision's atoms
+// spread over the wavefront and everything else done by all lanes at once.
+// A wavefront owns P.ions_per_wave ions (lanes below that number).  Per step:
+//   * every owner lane pushes its ion and runs its collision test (the
+//     handler's Maxwellian neutral, P = 1 - exp(-n sigma_eff |v_rel| dt)), and
+//     forms its random orientation, all lanes together;
+//   * the first impact parameters of every ion are drawn by all lanes together
+//     too: the stream is counter-based (attempt a is Philox block 5 + a), so
+//     lane g * ions_per_wave + l draws attempt g of ion l;
+//   * then the colliding ions one after another: the orientation goes to
+//     scalar registers, atom j of the cluster is handled by lane j mod 64.
+//     The method's geometry is taken in the collision frame, in which the
+//     relative velocity is the z axis and the rotation is the orientation
+//     alone: b_max is a wave max over the atoms' extents about the axis; for
+//     each impact parameter the first contact is a wave min over (s_hit, atom
+//     index), the sequential loop's choice (CollisionKernels.cpp:283-381);
+//   * the contact normals of all ions are turned to the global frame and the
+//     velocities reflected by all lanes together.
+// What bounds it: FP64 issue in the atom loops and the chain of one collision.
+// Done once per collision, the orientation, the draws and the reflection were
+// two thirds of the instructions; a row of atoms was waited for at a time; and
+// 64 ions on every wavefront left SIMDs idle below 131,072 ions (launch_step
+// picks ions_per_wave).  Before and now: 701 ions x 200 steps 55.5 and 2.0 ms,
+// 9001 x 200 57.7 and 7.5 ms, 40,000 x 300 93 and 32 ms, 250,000 x 40 33.9 and
+// 26.2 ms.
 
 __device__ __forceinline__ uint32_t readlane_u32(uint32_t x, int lane) {
     return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), lane));
@@ -195,202 +202,82 @@ __device__ __forceinline__ double readlane_f64(double x, int lane) {
     return __hiloint2double(hi, lo);
 }
 
-__device__ __forceinline__ d3 readlane_d3(d3 v, int lane) {
-    return d3{readlane_f64(v.x, lane), readlane_f64(v.y, lane), readlane_f64(v.z, lane)};
+// x moved between lanes by a DPP control; lanes without a source keep x.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_f64(double x) {
+    const int lo = __double2loint(x), hi = __double2hiint(x);
+    return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, ROWS, 0xf, false),
+                            __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROWS, 0xf, false));
 }
 
-__device__ __forceinline__ double wave_max_f64(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
-    return v;
-}
-
-// (s, j) <- the lexicographic minimum over the wavefront, on every lane
-__device__ __forceinline__ void wave_min_contact(double& s, uint32_t& j) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const double so = __shfl_xor(s, off, 64);
-        const uint32_t jo = __shfl_xor(j, off, 64);
-        if (so < s || (so == s && jo < j)) {
-            s = so;
-            j = jo;
-        }
-    }
+// The maximum / minimum over the wavefront (all 64 lanes active), wave-uniform:
+// row shifts within 16 lanes, then row broadcasts, read from lane 63.
+template <class Op>
+__device__ __forceinline__ double wave_reduce_f64(double v, Op&& op) {
+    v = op(v, dpp_f64<0x111, 0xf>(v));
+    v = op(v, dpp_f64<0x112, 0xf>(v));
+    v = op(v, dpp_f64<0x114, 0xf>(v));
+    v = op(v, dpp_f64<0x118, 0xf>(v));
+    v = op(v, dpp_f64<0x142, 0xa>(v));
+    v = op(v, dpp_f64<0x143, 0xc>(v));
+    return readlane_f64(v, 63);
 }
 
 // Rotated atoms of the collision in progress, per wavefront: the first
-// kWaveAtoms atoms of a cluster (x, y, z in the collision frame and
-// (r_atom + r_gas)^2), each written and read by its own lane; atoms past that
-// are rotated again from the table on every impact parameter.
-constexpr uint32_t kWaveAtoms = 512;
+// kWaveAtoms atoms of a cluster, (x, y) and (z, (r_atom + r_gas)^2) in the
+// collision frame, each written and read by its own lane; atoms past that are
+// rotated again from the table on every impact parameter.
+constexpr int kWaveRows = 8;
+constexpr uint32_t kWaveAtoms = 64 * kWaveRows;
+struct WaveAtoms {
+    double2 xy[kWaveAtoms];
+    double2 zr[kWaveAtoms];
+};
 
-// A per-(ion, step) stream whose state is wave-uniform: the draws of one ion
-// replayed by every lane, with its state and the Philox rounds held in scalar
-// registers (the same sequence as PhiloxStream).
-struct WaveStream {
-    uint32_t k0, k1, ion, s_lo, s_hi, block;
-    uint32_t buf[4];
-    int pos;
+// Impact parameters of an ion drawn ahead, in units of b_max, per pass over the
+// lanes (64 / ions_per_wave attempts each).
+constexpr int kAheadPasses = 3;
 
-    __device__ __forceinline__ void refill() {
-        const u32x4 o = philox4x32_10(__builtin_amdgcn_readfirstlane(block), __builtin_amdgcn_readfirstlane(ion),
-                                      __builtin_amdgcn_readfirstlane(s_lo), __builtin_amdgcn_readfirstlane(s_hi),
-                                      __builtin_amdgcn_readfirstlane(k0), __builtin_amdgcn_readfirstlane(k1));
-#pragma unroll
-        for (int c = 0; c < 4; ++c) buf[c] = __builtin_amdgcn_readfirstlane(o.v[c]);
-        ++block;
-        pos = 0;
+// The draws of the step's streams by block number: pair(b, ion) is draws 2 b and
+// 2 b + 1 of the ion's stream (0-5 the neutral, 6 the test, 7-9 the orientation,
+// 10 + 2 a and 11 + 2 a impact parameter a).
+struct EhssDraws {
+    uint32_t k0, k1, s_lo, s_hi;
+    __device__ __forceinline__ EhssDraws(uint64_t seed, uint64_t step)
+        : k0(static_cast<uint32_t>(seed)), k1(static_cast<uint32_t>(seed >> 32)), s_lo(static_cast<uint32_t>(step)),
+          s_hi(static_cast<uint32_t>(step >> 32)) {
+        // the round keys as scalar adds in each use (see PhiloxStream::refill)
+        k0 = __builtin_amdgcn_readfirstlane(k0);
+        k1 = __builtin_amdgcn_readfirstlane(k1);
+        asm("" : "+s"(k0), "+s"(k1) : "s"(__builtin_amdgcn_readfirstlane(s_lo)));
     }
-    // pos is 0 or 2: the words are selected, not indexed, so that the block
-    // stays in (scalar) registers instead of a private-memory array
-    __device__ __forceinline__ double uniform_f64() {
-        if (pos >= 4) refill();
-        const bool second = pos != 0;
-        const double u = uniform53(second ? buf[2] : buf[0], second ? buf[3] : buf[1]);
-        pos += 2;
-        return u;
+    __device__ __forceinline__ void pair(uint32_t block, uint32_t ion, double& u1, double& u2) const {
+        const u32x4 o = philox4x32_10(block, ion, s_lo, s_hi, k0, k1);
+        u1 = uniform53(o.v[0], o.v[1]);
+        u2 = uniform53(o.v[2], o.v[3]);
+    }
+    // the impact point of one attempt over b_max: sqrt(u1) (cos 2 pi u2, sin 2 pi u2)
+    __device__ __forceinline__ void impact(uint32_t attempt, uint32_t ion, double& ux, double& uy) const {
+        double u1, u2, sn, cs;
+        pair(5u + attempt, ion, u1, u2);
+        const double b = sqrt(u1);
+        sincos(2.0 * kPi * u2, &sn, &cs);
+        ux = b * cs;
+        uy = b * sn;
     }
 };
 
-// ehss_f64 of one ion, called by every lane of the wavefront with the same
-// (wave-uniform) arguments; returns the ion's new velocity on every lane.
-// lds: this wavefront's kWaveAtoms-entry staging area.
-__device__ d3 ehss_wave_f64(const StepParams& P, d3 v_ion, d3 v_n, double mi, double mn, double r_gas,
-                            uint32_t a0, uint32_t nat, WaveStream& rng, uint32_t lane, double4* lds) {
-    const double u1 = rng.uniform_f64();
-    const double u2 = rng.uniform_f64();
-    const double u3 = rng.uniform_f64();
-    if (nat == 0) return v_ion;
-    double s2, c2, s3, c3;
-    sincos(2.0 * kPi * u2, &s2, &c2);
-    sincos(2.0 * kPi * u3, &s3, &c3);
-    const double q1 = sqrt(1.0 - u1) * s2;
-    const double q2 = sqrt(1.0 - u1) * c2;
-    const double q3 = sqrt(u1) * s3;
-    const double q4 = sqrt(u1) * c3;
-    const double x = q1, y = q2, z = q3, w = q4;
-    double O[9];
-    O[0] = 1 - 2 * (y * y + z * z); O[1] = 2 * (x * y - z * w);     O[2] = 2 * (x * z + y * w);
-    O[3] = 2 * (x * y + z * w);     O[4] = 1 - 2 * (x * x + z * z); O[5] = 2 * (y * z - x * w);
-    O[6] = 2 * (x * z - y * w);     O[7] = 2 * (y * z + x * w);     O[8] = 1 - 2 * (x * x + y * y);
-    d3 vrel = v_ion - v_n;
-    double vrel_mag = sqrt(dot(vrel, vrel));
-    if (vrel_mag <= kMinVelocityMag) {
-        // iso_dir_f64 on the wave-uniform stream
-        const double w1 = rng.uniform_f64();
-        const double w2 = rng.uniform_f64();
-        const double cosT = 2.0 * w1 - 1.0;
-        const double sinT = sqrt(fmax(0.0, 1.0 - cosT * cosT));
-        double sp, cp;
-        sincos(2.0 * kPi * w2, &sp, &cp);
-        vrel = d3{sinT * cp, sinT * sp, cosT} * kMinVelocityMag;
-        vrel_mag = kMinVelocityMag;
-    }
-    const d3 ax{vrel.x / vrel_mag, vrel.y / vrel_mag, vrel.z / vrel_mag};
-    d3 t1, t2;
-    ortho_basis_f64(ax, t1, t2);
-    const double Bm[3][3] = {{t1.x, t2.x, ax.x}, {t1.y, t2.y, ax.y}, {t1.z, t2.z, ax.z}};
-    double Rm[9];
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-        for (int b = 0; b < 3; ++b)
-            Rm[3 * a + b] = Bm[a][0] * O[b] + Bm[a][1] * O[3 + b] + Bm[a][2] * O[6 + b];
-    const float4* __restrict__ atoms = P.atoms + a0;
-    double bm = 0.0;
-    for (uint32_t j = lane; j < nat; j += 64) {
-        const float4 f = atoms[j];
-        const d3 ra = mat_mul(Rm, d3{f.x, f.y, f.z});
-        const double sra = dot(ax, ra);
-        const d3 rp = ra - ax * sra;
-        const double cur = sqrt(dot(rp, rp)) + static_cast<double>(f.w);
-        bm = fmax(bm, cur);
-        if (j < kWaveAtoms) {
-            const double Rsum = static_cast<double>(f.w) + r_gas;
-            lds[j] = make_double4(ra.x, ra.y, ra.z, Rsum * Rsum);
-        }
-    }
-    double b_max = wave_max_f64(bm) + r_gas;
-    for (int attempt = 0; attempt < kEhssMaxAttempts; ++attempt) {
-        const double uA = rng.uniform_f64();
-        const double uB = rng.uniform_f64();
-        const double b = b_max * sqrt(uA);
-        double sphi, cphi;
-        sincos(2.0 * kPi * uB, &sphi, &cphi);
-        const d3 off = t1 * (b * cphi) + t2 * (b * sphi);
-        double best_s = INFINITY;
-        uint32_t best_j = 0xFFFFFFFFu;
-        for (uint32_t j = lane; j < nat; j += 64) {
-            d3 ra;
-            double Rsum2;
-            if (j < kWaveAtoms) {
-                const double4 a = lds[j];
-                ra = d3{a.x, a.y, a.z};
-                Rsum2 = a.w;
-            } else {
-                const float4 f = atoms[j];
-                ra = mat_mul(Rm, d3{f.x, f.y, f.z});
-                const double Rsum = static_cast<double>(f.w) + r_gas;
-                Rsum2 = Rsum * Rsum;
-            }
-            const d3 rel = off - ra;
-            const double sstar = dot(ax, rel);
-            const d3 dv = rel - ax * sstar;
-            const double dmin2 = dot(dv, dv);
-            if (dmin2 <= Rsum2) {
-                const double s_hit = sstar - sqrt(fmax(0.0, Rsum2 - dmin2));
-                if (s_hit < best_s) {
-                    best_s = s_hit;
-                    best_j = j;
-                }
-            }
-        }
-        // no lane found a contact: the next impact parameter (wave-uniform)
-        if (__ballot(best_j != 0xFFFFFFFFu) == 0ull) {
-            if (attempt == kBmaxExpansionAttempt) b_max *= kBmaxExpansionFactor;
-            continue;
-        }
-        wave_min_contact(best_s, best_j);
-        {
-            // the contact normal of the first atom hit, as the sequential loop forms it
-            const float4 f = atoms[best_j];
-            const d3 ra = mat_mul(Rm, d3{f.x, f.y, f.z});
-            const double Rsum = static_cast<double>(f.w) + r_gas;
-            const double Rsum2 = Rsum * Rsum;
-            const d3 rel = off - ra;
-            const double sstar = dot(ax, rel);
-            const d3 dv = rel - ax * sstar;
-            const double dmin2 = dot(dv, dv);
-            const double h = sqrt(fmax(0.0, Rsum2 - dmin2));
-            const double s_hit = sstar - h;
-            const d3 ph = rel - ax * s_hit;
-            const double phr2 = dot(ph, ph);
-            d3 nb;
-            if (phr2 <= kMinContactDistSq) {
-                nb = ax * -1.0;
-            } else {
-                nb = ph * (1.0 / sqrt(phr2));
-                if (dot(ax, nb) > 0.0) nb = nb * -1.0;
-            }
-            const double vdn = dot(vrel, nb);
-            const d3 vr = vrel - nb * (2.0 * vdn);
-            const double inv_mt = 1.0 / (mi + mn);
-            const d3 Vcom = (v_ion * mi + v_n * mn) * inv_mt;
-            return Vcom + vr * (mn * inv_mt);
-        }
-    }
-    return v_ion;
-}
-
-// step_f64_kernel<INTEG, FIELD, COLL_EHSS> with the geometry method run by
-// the wavefront (above).  Every lane stays in the step loop until no lane of
-// its wavefront has an ion left to step (lanes past the last ion, dead ions
-// and ions done are carried along), so the wave-wide parts see all 64 lanes.
 template <int INTEG, int FIELD>
 __global__ void __launch_bounds__(256) step_f64_ehss_kernel(const StepParams P, const IonPtrs S) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t lane = threadIdx.x & 63u;
-    const bool have = i < P.n_ions;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t G = P.ions_per_wave;
+    const uint32_t first = (blockIdx.x * (blockDim.x >> 6) + wave) * G;
+    const uint32_t ahead = lane / G, owner = lane - ahead * G;   // the attempt and ion this lane draws for
+    const uint32_t reps = 64u / G;                               // attempts drawn per pass
+    const uint32_t passes = reps >= 3u ? 1u : reps == 2u ? 2u : 3u;
+    const uint32_t i = first + lane;
+    const bool have = lane < G && i < P.n_ions;
     d3 pos{0.0, 0.0, 0.0}, vel{0.0, 0.0, 0.0};
     double m = 1.0, q = 0.0, birth = -INFINITY, death = -1.0, arrival = NAN;
     uint32_t sidx = 0, nc = 0;
@@ -415,8 +302,8 @@ __global__ void __launch_bounds__(256) step_f64_ehss_kernel(const StepParams P, 
     bool checked = false;
     const double dt = P.dt;
     const double half_dt = dt * 0.5;
-    __shared__ double4 s_atoms[4][kWaveAtoms];   // 256 threads = 4 wavefronts
-    double4* const lds = s_atoms[threadIdx.x >> 6];
+    __shared__ WaveAtoms s_atoms[4];   // 256 threads = 4 wavefronts
+    WaveAtoms& lds = s_atoms[threadIdx.x >> 6];
     // the next step's table entry is loaded one step ahead
     StepEntry te_next = P.n_steps ? P.table[0] : StepEntry{};
     for (uint32_t k = 0; k < P.n_steps; ++k) {
@@ -476,46 +363,197 @@ __global__ void __launch_bounds__(256) step_f64_ehss_kernel(const StepParams P, 
         }
         // the collision test of each lane (collide_f64<COLL_EHSS> up to the
         // geometry method)
-        PhiloxStream rng(P.seed, i, P.step0 + k);
+        const EhssDraws rng(P.seed, P.step0 + k);
         bool hit = false;
-        d3 vn{0.0, 0.0, 0.0};
+        d3 vn{0.0, 0.0, 0.0}, vrel{0.0, 0.0, 0.0};
+        double vrel_mag = 1.0, u_first = 0.0;   // u_first: the orientation's first draw
         if (live && sp.sigma_ehss > 0.0) {
-            double u1 = rng.uniform_f64(), u2 = rng.uniform_f64();
+            double u1, u2;
+            rng.pair(0u, i, u1, u2);
             vn.x = P.sigma_neutral * sqrt(-2.0 * log(u1)) * cos(2.0 * kPi * u2);
-            u1 = rng.uniform_f64(); u2 = rng.uniform_f64();
+            rng.pair(1u, i, u1, u2);
             vn.y = P.sigma_neutral * sqrt(-2.0 * log(u1)) * cos(2.0 * kPi * u2);
-            u1 = rng.uniform_f64(); u2 = rng.uniform_f64();
+            rng.pair(2u, i, u1, u2);
             vn.z = P.sigma_neutral * sqrt(-2.0 * log(u1)) * cos(2.0 * kPi * u2);
             vn = vn + d3{P.u_gas[0], P.u_gas[1], P.u_gas[2]};
-            const d3 vrel = vel - vn;
-            const double vrel_mag = sqrt(dot(vrel, vrel));
+            vrel = vel - vn;
+            vrel_mag = sqrt(dot(vrel, vrel));
             if (vrel_mag >= kMinRelativeVelocity) {
                 const double Pc = 1.0 - exp(-P.n * sp.sigma_ehss * vrel_mag * (dt * te.nrel));
-                hit = rng.uniform_f64() < Pc;
+                rng.pair(3u, i, u1, u_first);
+                hit = u1 < Pc;
             }
         }
-        // the geometry method of each colliding ion, on the whole wavefront
         uint64_t pending = __ballot(hit);
-        while (pending) {
-            const int L = __builtin_amdgcn_readfirstlane(static_cast<int>(__builtin_ctzll(pending)));
-            pending &= pending - 1ull;
-            WaveStream r;
-            r.k0 = rng.k0;
-            r.k1 = rng.k1;
-            r.s_lo = rng.s_lo;
-            r.s_hi = rng.s_hi;
-            r.ion = readlane_u32(i, L);
-            r.block = readlane_u32(rng.block, L);
+        if (pending) {
+            // the random orientation (CollisionGeometry::generate_random_rotation)
+            double O[9];
+            {
+                const double u1 = u_first;
+                double u2, u3;
+                rng.pair(4u, i, u2, u3);
+                double s2, c2, s3, c3;
+                sincos(2.0 * kPi * u2, &s2, &c2);
+                sincos(2.0 * kPi * u3, &s3, &c3);
+                const double x = sqrt(1.0 - u1) * s2;
+                const double y = sqrt(1.0 - u1) * c2;
+                const double z = sqrt(u1) * s3;
+                const double w = sqrt(u1) * c3;
+                O[0] = 1 - 2 * (y * y + z * z); O[1] = 2 * (x * y - z * w);     O[2] = 2 * (x * z + y * w);
+                O[3] = 2 * (x * y + z * w);     O[4] = 1 - 2 * (x * x + z * z); O[5] = 2 * (y * z - x * w);
+                O[6] = 2 * (x * z - y * w);     O[7] = 2 * (y * z + x * w);     O[8] = 1 - 2 * (x * x + y * y);
+            }
+            // the first impact points: pass p draws attempts p * reps .. + reps - 1
+            double ux[kAheadPasses], uy[kAheadPasses];
 #pragma unroll
-            for (int c = 0; c < 4; ++c) r.buf[c] = readlane_u32(rng.buf[c], L);
-            r.pos = static_cast<int>(readlane_u32(static_cast<uint32_t>(rng.pos), L));
-            const d3 v_new = ehss_wave_f64(P, readlane_d3(vel, L), readlane_d3(vn, L), readlane_f64(m, L),
-                                           P.m_gas, P.r_gas, readlane_u32(sp.atom_offset, L),
-                                           readlane_u32(sp.atom_count, L), r, lane, lds);
-            if (static_cast<int>(lane) == L) {
-                vel = v_new;
+            for (int p = 0; p < kAheadPasses; ++p) {
+                ux[p] = uy[p] = 0.0;
+                if (static_cast<uint32_t>(p) < passes) rng.impact(p * reps + ahead, first + owner, ux[p], uy[p]);
+            }
+            bool contact = false;
+            double nx = 0.0, ny = 0.0, nz = 1.0;   // the contact point about the atom, collision frame
+            // The cluster of the first colliding ion; each later one is loaded
+            // while the impact parameters of the ion before it are tried.  Rows of
+            // 64 atoms; lanes past the last atom read it again.
+            float4 row[kWaveRows];
+            auto fetch = [&](int L) {
+                const uint32_t nat = readlane_u32(sp.atom_count, L);
+                const float4* __restrict__ atoms = P.atoms + readlane_u32(sp.atom_offset, L);
+#pragma unroll
+                for (int r = 0; r < kWaveRows; ++r)
+                    if (64u * r < nat) row[r] = atoms[min(lane + 64u * r, nat - 1u)];
+            };
+            fetch(__builtin_amdgcn_readfirstlane(static_cast<int>(__builtin_ctzll(pending))));
+            while (pending) {
+                const int L = __builtin_amdgcn_readfirstlane(static_cast<int>(__builtin_ctzll(pending)));
+                pending &= pending - 1ull;
+                const uint32_t nat = readlane_u32(sp.atom_count, L);
+                const float4* __restrict__ atoms = P.atoms + readlane_u32(sp.atom_offset, L);
+                double Q[9];
+#pragma unroll
+                for (int c = 0; c < 9; ++c) Q[c] = readlane_f64(O[c], L);
+                const double r_gas = P.r_gas;
+                auto rotated = [&](float4 f, double2& xy, double2& zr) {
+                    const d3 r = mat_mul(Q, d3{f.x, f.y, f.z});
+                    const double Rsum = static_cast<double>(f.w) + r_gas;
+                    xy = make_double2(r.x, r.y);
+                    zr = make_double2(r.z, Rsum * Rsum);
+                };
+                double bm = 0.0;
+#pragma unroll
+                for (int r = 0; r < kWaveRows; ++r) {
+                    if (64u * r < nat) {
+                        double2 xy, zr;
+                        rotated(row[r], xy, zr);
+                        // (a lane past the last atom repeats it: the same extent)
+                        const double ext = sqrt(xy.x * xy.x + xy.y * xy.y) + static_cast<double>(row[r].w);
+                        bm = ext > bm ? ext : bm;
+                        if (lane + 64u * r >= nat) zr.y = -1.0;   // never a contact
+                        lds.xy[lane + 64u * r] = xy;
+                        lds.zr[lane + 64u * r] = zr;
+                    }
+                }
+                for (uint32_t j = kWaveAtoms + lane; j < nat; j += 64) {
+                    const float4 f = atoms[j];
+                    double2 xy, zr;
+                    rotated(f, xy, zr);
+                    bm = fmax(bm, sqrt(xy.x * xy.x + xy.y * xy.y) + static_cast<double>(f.w));
+                }
+                if (pending) fetch(__builtin_amdgcn_readfirstlane(static_cast<int>(__builtin_ctzll(pending))));
+                if (nat == 0) continue;
+                double b_max = wave_reduce_f64(bm, [](double a, double b) { return a > b ? a : b; }) + r_gas;
+                // the first contact of impact point (bx, by); true: found
+                auto first_contact = [&](double bx, double by) -> bool {
+                    double best_s = INFINITY, cx = 0.0, cy = 0.0, ch = 0.0;
+                    uint32_t best_j = 0;
+                    auto test = [&](uint32_t j, double2 xy, double2 zr) {
+                        const double dx = bx - xy.x, dy = by - xy.y;
+                        const double dmin2 = dx * dx + dy * dy;
+                        if (dmin2 <= zr.y) {
+                            const double h = sqrt(zr.y - dmin2);
+                            const double s_hit = -zr.x - h;
+                            if (s_hit < best_s) {
+                                best_s = s_hit;
+                                best_j = j;
+                                cx = dx;
+                                cy = dy;
+                                ch = h;
+                            }
+                        }
+                    };
+                    const uint32_t staged = min(nat, kWaveAtoms);
+#pragma unroll 2
+                    for (uint32_t base = 0; base < staged; base += 64)
+                        test(base + lane, lds.xy[base + lane], lds.zr[base + lane]);
+                    for (uint32_t j = kWaveAtoms + lane; j < nat; j += 64) {
+                        double2 xy, zr;
+                        rotated(atoms[j], xy, zr);
+                        test(j, xy, zr);
+                    }
+                    if (__ballot(best_s < INFINITY) == 0ull) return false;
+                    const double s_min = wave_reduce_f64(best_s, [](double a, double b) { return a < b ? a : b; });
+                    uint64_t at = __ballot(best_s == s_min);
+                    int W = __builtin_amdgcn_readfirstlane(static_cast<int>(__builtin_ctzll(at)));
+                    // equal s_hit: the lowest atom index
+                    for (at &= at - 1ull; at; at &= at - 1ull) {
+                        const int V = __builtin_amdgcn_readfirstlane(static_cast<int>(__builtin_ctzll(at)));
+                        if (readlane_u32(best_j, V) < readlane_u32(best_j, W)) W = V;
+                    }
+                    const double wx = readlane_f64(cx, W), wy = readlane_f64(cy, W), wh = readlane_f64(ch, W);
+                    if (static_cast<int>(lane) == L) {
+                        contact = true;
+                        nx = wx;
+                        ny = wy;
+                        nz = wh;
+                    }
+                    return true;
+                };
+                // the attempts drawn ahead, then 64 at a time drawn for this ion alone
+                const uint32_t drawn = passes * reps;
+                double sx = ux[0], sy = uy[0];
+                uint32_t from = static_cast<uint32_t>(L), last = from + (reps - 1u) * G;
+                for (uint32_t attempt = 0; attempt < kEhssMaxAttempts; ++attempt) {
+                    if (attempt >= drawn && ((attempt - drawn) & 63u) == 0u) {
+                        rng.impact(attempt + lane, first + L, sx, sy);
+                        from = 0;
+                    }
+                    if (attempt == kBmaxExpansionAttempt + 1) b_max *= kBmaxExpansionFactor;
+                    if (first_contact(b_max * readlane_f64(sx, static_cast<int>(from)),
+                                      b_max * readlane_f64(sy, static_cast<int>(from))))
+                        break;
+                    if (attempt + 1 >= drawn) {
+                        ++from;
+                    } else if (from == last) {   // the next pass
+                        from = static_cast<uint32_t>(L);
+                        const bool second = attempt + 1 == reps;
+                        sx = second ? ux[1] : ux[2];
+                        sy = second ? uy[1] : uy[2];
+                    } else {
+                        from += G;
+                    }
+                }
+            }
+            if (hit) {
                 ++nc;
                 ++ncoll_launch;
+            }
+            if (contact) {
+                // reflection about the contact normal, which points against the axis
+                d3 nb{0.0, 0.0, -1.0};
+                const double phr2 = nx * nx + ny * ny + nz * nz;
+                if (phr2 > kMinContactDistSq) {
+                    nb = d3{nx, ny, nz} * (1.0 / sqrt(phr2));
+                    if (nb.z > 0.0) nb = nb * -1.0;
+                }
+                const d3 ax{vrel.x / vrel_mag, vrel.y / vrel_mag, vrel.z / vrel_mag};
+                d3 t1, t2;
+                ortho_basis_f64(ax, t1, t2);
+                nb = t1 * nb.x + t2 * nb.y + ax * nb.z;
+                const double vdn = dot(vrel, nb);
+                const d3 vr = vrel - nb * (2.0 * vdn);
+                const double inv_mt = 1.0 / (m + P.m_gas);
+                const d3 Vcom = (vel * m + vn * P.m_gas) * inv_mt;
+                vel = Vcom + vr * (P.m_gas * inv_mt);
             }
         }
         if (live) {
@@ -1286,10 +1324,22 @@ KernelFn pick_surrogate(int field) {
     }
 }
 
+// Ions per wavefront of the geometry EHSS kernel: two wavefronts per SIMD fit
+// (registers and LDS), 2048 on the chip.  A wavefront works through its
+// colliding ions one after another, so the ions are spread evenly over the
+// least number of full rounds of 2048 wavefronts.
+uint32_t ehss_ions_per_wave(uint32_t n_ions) {
+    const uint32_t slots = 2048;
+    const uint32_t rounds = (n_ions + 64 * slots - 1) / (64 * slots);
+    const uint32_t g = (n_ions + rounds * slots - 1) / (rounds * slots);
+    return g < 1 ? 1 : g > 64 ? 64 : g;
+}
+
 // Returns hipSuccess, or hipErrorInvalidValue when the combination has no
 // kernel (the host maps that to ICARION_ERR_UNSUPPORTED).
 hipError_t launch_step(int integrator, int field, int coll, int precision, int surrogate,
-                       const StepParams& P, const IonPtrs& S, uint32_t block, hipStream_t stream) {
+                       const StepParams& params, const IonPtrs& S, uint32_t block, hipStream_t stream) {
+    StepParams P = params;
     KernelFn fn;
     if (surrogate) {
         fn = integrator == 1 ? pick_surrogate<1>(field) : pick_surrogate<0>(field);
@@ -1302,7 +1352,13 @@ hipError_t launch_step(int integrator, int field, int coll, int precision, int s
     // the surrogate kernel runs its own workgroup size (the handle's block size
     // does not change any result)
     if (surrogate) block = kSurrogateBlock;
-    const uint32_t grid = (P.n_ions + block - 1) / block;
+    uint32_t grid = (P.n_ions + block - 1) / block;
+    if (!surrogate && coll == COLL_EHSS) {
+        P.ions_per_wave = ehss_ions_per_wave(P.n_ions);
+        block = 256;
+        const uint32_t per_block = 4 * P.ions_per_wave;
+        grid = (P.n_ions + per_block - 1) / per_block;
+    }
     hipLaunchKernelGGL(fn, dim3(grid), dim3(block), 0, stream, P, S);
     return hipGetLastError();
 }

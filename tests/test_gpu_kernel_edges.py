@@ -1,0 +1,86 @@
+"""Kernel variants at the sizes where they can go wrong, against the CPU oracle:
+row and wavefront edges of the geometry EHSS kernel, and the field-array
+kernels' kept cell under ions that change cells in nearly every stage.
+
+FP64 runs draw the same random numbers on both sides and differ by rounding
+only: 1e-9 relative, as the parity tests; a contact or collision decided within
+rounding of its threshold (some 1e-15 of the tests) does not occur at these
+sizes, so every ion has to match.
+"""
+import numpy as np
+import pytest
+
+from icarion_amd import _abi
+from icarion_amd import workloads as W
+from test_gpu_parity import compare_ions, gpu_run, oracle_run
+
+pytestmark = pytest.mark.gpu
+
+
+def cluster_table(counts, spread, seed):
+    """Species of counts[s] atoms (1.7 A) spread over a cube of half edge spread[s]."""
+    rng = np.random.default_rng(seed)
+    atoms, species, off = [], [], 0
+    for c, h in zip(counts, spread):
+        a = np.zeros((c, 4), np.float32)
+        a[:, :3] = rng.uniform(-h, h, (c, 3))
+        a[:, 3] = 1.7e-10
+        atoms.append(a)
+        species.append(W.species(sigma_ehss=3e-18, atom_offset=off, atom_count=c))
+        off += c
+    return np.concatenate(atoms), species
+
+
+# atoms per cluster about the 64-atom rows and the 512 staged ones; the sparse
+# pair (atoms several nm apart) is missed by most impact parameters, so that the
+# draws go past the ones made ahead, past the expansion and past the last attempt
+COUNTS = (1, 2, 63, 64, 65, 128, 449, 511, 512, 513, 700)
+SPREAD = (0.0, 4e-9, 8e-10, 8e-10, 8e-10, 8e-10, 1.2e-9, 1.2e-9, 1.2e-9, 1.2e-9, 1.2e-9)
+
+
+@pytest.mark.parametrize("n", [1, 63, 2047, 2049, 5000])
+def test_geometry_ehss_rows_and_wavefronts(oracle, n):
+    atoms, species = cluster_table(COUNTS, SPREAD, seed=5)
+    w = W.ehss_surrogate_workload(n=1, seed=17, precision=_abi.PRECISION_FP64, ehss_mode=_abi.EHSS_GEOMETRY)
+    rng = np.random.default_rng(n)
+    which = rng.integers(0, len(species), n).astype(np.uint32)
+    which[:min(n, len(species))] = np.arange(min(n, len(species)))
+    ens = W.gaussian_cloud(n, 1200.0, 0.5e-3, seed=n)
+    ens.species[:] = which
+    w.update(species=species, atoms=atoms, ensemble=ens)
+    g, o = ens.copy(), ens.copy()
+    sg = gpu_run(w, g, 25)
+    so = oracle_run(oracle, w, o, 25)
+    assert so.collisions > 0 or n < 63
+    assert sg.collisions == so.collisions
+    assert compare_ions(g, o, rtol=1e-9).all()
+
+
+@pytest.mark.parametrize("integrator", [_abi.INTEGRATOR_RK4, _abi.INTEGRATOR_BORIS])
+@pytest.mark.parametrize("precision", [_abi.PRECISION_FP64, _abi.PRECISION_FP32_KAHAN])
+@pytest.mark.parametrize("n,grid", [(1, (2, 2, 2)), (257, (2, 3, 65)), (3001, (64, 63, 2)), (70001, (40, 41, 200))])
+def test_field_array_cell_changes(oracle, n, grid, precision, integrator):
+    """Ions at 10 km/s with steps of a good part of a cell: most stages find the
+    ion in another cell than the last one.  FP32 against the FP64 oracle: cell
+    coordinates of up to 200 in FP32 place an ion to 200 * 2^-24 of a cell, and
+    the field is continuous across cells, so 2e-5 as for the other collisionless
+    FP32 runs.  Potentials of a few volts: the field gradient of 5 V / mm^2 then
+    multiplies a deviation by less than exp(omega t) = 5 over the run (omega^2 =
+    q E' / m = 1.6e12 s^-2, t = 1.2 us); kilovolts would multiply it by exp(48)."""
+    E, origin, spacing = W.gaussian_potential_field(grid, n_gauss=4, seed=2)
+    E *= np.float32(1e-3)
+    w = W.field_array_workload(n=1, grid=(2, 2, 2), seed=2, precision=precision)
+    w["physics"] = W.physics(integrator, _abi.COLLISION_NONE, precision=precision, seed=2)
+    ens = W.gaussian_cloud(n, 300.0, (1e-3, 1e-3, 4e-3), center=(0.0, 0.0, 20e-3), seed=n)
+    ens.vx += 2e3
+    ens.vz += 1e4
+    w.update(ensemble=ens, field=(E, origin, spacing), dt=2e-8)
+    g, o = ens.copy(), ens.copy()
+    gpu_run(w, g, 60)
+    oracle_run(oracle, w, o, 60)
+    assert (g.active == o.active).mean() >= 0.999
+    both = (g.active != 0) & (o.active != 0)
+    tol = 1e-9 if precision == _abi.PRECISION_FP64 else 2e-5
+    for f, scale in (("x", 1e-3), ("y", 1e-3), ("z", 1e-2), ("vx", 1e3), ("vy", 1e3), ("vz", 1e4)):
+        d = np.abs(getattr(g, f) - getattr(o, f))[both]
+        assert d.size == 0 or d.max() <= tol * np.maximum(scale, np.abs(getattr(o, f))[both].max()), f
