@@ -25,6 +25,10 @@ constexpr double kBmaxExpansionFactor = 1.5;
 constexpr double kGeomEpsilon = 1e-12;
 constexpr double kMinVoltage = 1e-12;
 
+// Keeps a wave-uniform branch a branch: without it the compiler computes both
+// sides in every step and selects.
+__device__ __forceinline__ void keep_branch() { asm volatile(""); }
+
 template <typename T>
 struct vec3 {
     T x, y, z;
@@ -95,6 +99,66 @@ __device__ __forceinline__ float uniform24(uint32_t w) {
     return static_cast<float>(w >> 8) * 0x1.0p-24f + 0x1.0p-25f;
 }
 
+// ---- FP64 functions of the random draws ------------------------------------
+// The general sin, cos and log were a third of the FP64 HSS step's instructions:
+// they reduce any argument.  A draw is a uniform in (0, 1], so the angle is
+// reduced exactly in revolutions before it meets 2 pi, and the logarithm has no
+// special values.  The polynomials interpolate at Chebyshev nodes (evaluated in
+// extended precision; relative error of the fit below 5e-18).  Largest errors
+// over 4e5 draws against extended precision: sine and cosine 1.5e-16 absolute,
+// where the general functions of the rounded product 2 pi u had 6.9e-16;
+// logarithm 0.9 units in the last place.
+template <int N>
+__device__ __forceinline__ double horner(const double (&p)[N], double w) {
+    double r = p[N - 1];
+#pragma unroll
+    for (int i = N - 2; i >= 0; --i) r = fma(r, w, p[i]);
+    return r;
+}
+
+// sine and cosine of u revolutions, 0 <= u <= 1: u = k / 4 + r with |r| <= 1/8
+__device__ __forceinline__ void sincos_rev(double u, double& sn, double& cs) {
+    constexpr double ps[] = {6.283185307179586, -41.341702240399634, 81.60524927594857,
+                             -76.70585970444363, 42.058685043183644, -15.09380560388465,
+                             3.7808998789812995};
+    constexpr double pc[] = {-19.739208802178716, 64.93939402266825, -85.45681720664702,
+                             60.244641353320404, -26.426253328264924, 7.903208845913531,
+                             -1.699058459304078};
+    const double k = rint(4.0 * u);
+    const double r = fma(k, -0.25, u);
+    const double w = r * r;
+    const double s = r * horner(ps, w);
+    const double c = fma(w, horner(pc, w), 1.0);
+    const int q = static_cast<int>(k);
+    const double a = (q & 1) ? c : s, b = (q & 1) ? s : c;
+    sn = (q & 2) ? -a : a;
+    cs = ((q + 1) & 2) ? -b : b;
+}
+
+// natural logarithm of 0 < u <= 1 (a normal number): u = 2^e m, m in
+// [sqrt(1/2), sqrt(2)), log m = 2 atanh(s) with s = (m - 1) / (m + 1)
+__device__ __forceinline__ double log_unit(double u) {
+    constexpr double pa[] = {0.3333333333333335, 0.1999999999994975, 0.14285714312988573,
+                             0.11111105567284828, 0.09091444569747409, 0.07665860591894315,
+                             0.0730822712981302};
+    double m = __builtin_amdgcn_frexp_mant(u);
+    int e = __builtin_amdgcn_frexp_exp(u);
+    const bool low = m < 0.70710678118654752;
+    m = low ? m + m : m;
+    e = low ? e - 1 : e;
+    const double f = m - 1.0, d = m + 1.0;
+    double y = __builtin_amdgcn_rcp(d);
+    y = fma(y, fma(-d, y, 1.0), y);
+    y = fma(y, fma(-d, y, 1.0), y);
+    double s = f * y;
+    s = fma(fma(-d, s, f), y, s);
+    const double z = s * s;
+    const double ed = static_cast<double>(e);
+    // 2 s = f - s f; ln 2 in two parts, the first times e exact
+    const double t = s * (f - 2.0 * (z * horner(pa, z)));
+    return fma(ed, 0.6931471805598903, f - fma(ed, -5.497924164543644e-14, t));
+}
+
 // Per-(ion, step) stream, counter = (block, ion, step_lo, step_hi), key =
 // (seed_lo, seed_hi).  FP64 draws take two words (the oracle's PhiloxStream
 // hands out the identical sequence); FP32 draws take one word.
@@ -111,19 +175,13 @@ struct PhiloxStream {
           s_lo(static_cast<uint32_t>(step)), s_hi(static_cast<uint32_t>(step >> 32)), block(0),
           pos(4), n_have(false), n_cached(0.0) {}
 
-    // FRESH_KEYS: the round keys as scalar adds in this call (the key words,
-    // wave-uniform, are tied to the step's counter).  Hoisted out of the step
-    // loop the 18 keys overflow the scalar registers of the FP32 kernels and
-    // come back by v_readlane, on the vector pipe that bounds them; the FP64
-    // kernels wait on their own chain instead, where the adds would lengthen it.
-    template <bool FRESH_KEYS>
+    // The round keys as scalar adds in this call (the key words, wave-uniform,
+    // are tied to the step's counter).  Hoisted out of the step loop the 18 keys
+    // overflow the scalar registers and come back by v_readlane, on the vector
+    // pipe that bounds the step kernels.
     __device__ __forceinline__ void refill() {
-        uint32_t r0 = k0, r1 = k1;
-        if constexpr (FRESH_KEYS) {
-            r0 = __builtin_amdgcn_readfirstlane(k0);
-            r1 = __builtin_amdgcn_readfirstlane(k1);
-            asm("" : "+s"(r0), "+s"(r1) : "s"(__builtin_amdgcn_readfirstlane(s_lo)));
-        }
+        uint32_t r0 = __builtin_amdgcn_readfirstlane(k0), r1 = __builtin_amdgcn_readfirstlane(k1);
+        asm("" : "+s"(r0), "+s"(r1) : "s"(__builtin_amdgcn_readfirstlane(s_lo)));
         const u32x4 o = philox4x32_10(block, ion, s_lo, s_hi, r0, r1);
         buf[0] = o.v[0]; buf[1] = o.v[1]; buf[2] = o.v[2]; buf[3] = o.v[3];
         ++block;
@@ -134,7 +192,7 @@ struct PhiloxStream {
     // data-dependent loops); an indexed buffer goes to private memory there.
     // A stream takes FP64 draws only (pos 0 or 2) or FP32 draws only.
     __device__ __forceinline__ double uniform_f64() {
-        if (pos >= 4) refill<false>();
+        if (pos >= 4) refill();
         const bool second = pos >= 2;
         const double u = uniform53(second ? buf[2] : buf[0], second ? buf[3] : buf[1]);
         pos += 2;
@@ -151,15 +209,15 @@ struct PhiloxStream {
         }
         const double u1 = uniform_f64();
         const double u2 = uniform_f64();
-        const double r = sqrt(-2.0 * log(u1));
+        const double r = sqrt(-2.0 * log_unit(u1));
         double sn, cs;
-        sincos(2.0 * 3.14159265358979323846 * u2, &sn, &cs);
+        sincos_rev(u2, sn, cs);
         n_cached = r * sn;
         n_have = true;
         return r * cs;
     }
     __device__ __forceinline__ float uniform_f32() {
-        if (pos >= 4) refill<true>();
+        if (pos >= 4) refill();
         const uint32_t w = pos == 0 ? buf[0] : pos == 1 ? buf[1] : pos == 2 ? buf[2] : buf[3];
         const float u = uniform24(w);
         pos += 1;

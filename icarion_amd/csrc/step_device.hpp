@@ -15,7 +15,10 @@ using d3 = vec3<double>;
 
 __device__ __forceinline__ bool contains_f64(const StepParams& P, d3 p) {
     d3 l{p.x - P.origin[0], p.y - P.origin[1], p.z - P.origin[2]};
-    if (!P.rot_identity) l = mat_mul(P.g2l, l);
+    if (!P.rot_identity) {
+        keep_branch();
+        l = mat_mul(P.g2l, l);
+    }
     if (P.instrument == 3) {
         // OrbitrapGeometry::contains (OrbitrapGeometry.h:36-51).  The electrode
         // radius r_e(z) is the root of f(r) = z^2 - (r^2 - R^2)/2 - Rm^2 ln(R/r),
@@ -31,10 +34,9 @@ __device__ __forceinline__ bool contains_f64(const StepParams& P, d3 p) {
         const double f_out = z2 - 0.5 * (r2 - P.R_out * P.R_out) - P.R_char_sq * (P.ln_R_out - ln_r);
         return f_in >= 0.0 && f_out <= 0.0;
     }
-    if (l.z < -kGeomEpsilon || l.z >= P.L + kGeomEpsilon) return false;
     const double r2 = l.x * l.x + l.y * l.y;
     const double Re = P.R + kGeomEpsilon;
-    return r2 <= Re * Re;
+    return !(l.z < -kGeomEpsilon) & !(l.z >= P.L + kGeomEpsilon) & (r2 <= Re * Re);
 }
 
 // trilinear interpolation with clamping (fieldArrayLoader.cpp:103-162) on a
@@ -212,14 +214,20 @@ __device__ __forceinline__ d3 force_f64(const StepParams& P, d3 p, d3 v, double 
     return F;
 }
 
+// standard normal by Box-Muller, the cosine branch
+__device__ __forceinline__ double normal_of(double u1, double u2) {
+    double sn, cs;
+    sincos_rev(u2, sn, cs);
+    return sqrt(-2.0 * log_unit(u1)) * cs;
+}
+
 __device__ __forceinline__ d3 iso_dir_f64(PhiloxStream& rng) {
     const double u1 = rng.uniform_f64();
     const double u2 = rng.uniform_f64();
     const double cosT = 2.0 * u1 - 1.0;
     const double sinT = sqrt(fmax(0.0, 1.0 - cosT * cosT));
-    const double phi = 2.0 * kPi * u2;
     double s, c;
-    sincos(phi, &s, &c);
+    sincos_rev(u2, s, c);
     return d3{sinT * c, sinT * s, cosT};
 }
 
@@ -281,7 +289,7 @@ __device__ d3 ehss_core_f64(const StepParams& P, d3 v_ion, d3 v_n, double mi, do
         const double uB = rng.uniform_f64();
         const double b = b_max * sqrt(uA);
         double sphi, cphi;
-        sincos(2.0 * kPi * uB, &sphi, &cphi);
+        sincos_rev(uB, sphi, cphi);
         const d3 off = t1 * (b * cphi) + t2 * (b * sphi);
         bool hit = false;
         d3 nb{0, 0, 0};
@@ -335,10 +343,13 @@ __device__ d3 ehss_f64(const StepParams& P, d3 v_ion, d3 v_n, double mi, double 
     const double u2 = rng.uniform_f64();
     const double u3 = rng.uniform_f64();
     if (nat == 0) return v_ion;
-    const double q1 = sqrt(1.0 - u1) * sin(2.0 * kPi * u2);
-    const double q2 = sqrt(1.0 - u1) * cos(2.0 * kPi * u2);
-    const double q3 = sqrt(u1) * sin(2.0 * kPi * u3);
-    const double q4 = sqrt(u1) * cos(2.0 * kPi * u3);
+    double s2, c2, s3, c3;
+    sincos_rev(u2, s2, c2);
+    sincos_rev(u3, s3, c3);
+    const double q1 = sqrt(1.0 - u1) * s2;
+    const double q2 = sqrt(1.0 - u1) * c2;
+    const double q3 = sqrt(u1) * s3;
+    const double q4 = sqrt(u1) * c3;
     const double x = q1, y = q2, z = q3, w = q4;
     double O[9];
     O[0] = 1 - 2 * (y * y + z * z); O[1] = 2 * (x * y - z * w);     O[2] = 2 * (x * z + y * w);
@@ -374,11 +385,11 @@ __device__ __forceinline__ bool collide_f64(const StepParams& P, const SpeciesDe
             if (c < P.n_emix && P.emix_part[c]) {
                 const double sn = P.emix_sig[c];
                 double u1 = rng.uniform_f64(), u2 = rng.uniform_f64();
-                vn[c].x = sn * sqrt(-2.0 * log(u1)) * cos(2.0 * kPi * u2);
+                vn[c].x = sn * normal_of(u1, u2);
                 u1 = rng.uniform_f64(); u2 = rng.uniform_f64();
-                vn[c].y = sn * sqrt(-2.0 * log(u1)) * cos(2.0 * kPi * u2);
+                vn[c].y = sn * normal_of(u1, u2);
                 u1 = rng.uniform_f64(); u2 = rng.uniform_f64();
-                vn[c].z = sn * sqrt(-2.0 * log(u1)) * cos(2.0 * kPi * u2);
+                vn[c].z = sn * normal_of(u1, u2);
                 vn[c] = vn[c] + u_gas;
                 const d3 vr = v - vn[c];
                 const double vm = sqrt(dot(vr, vr));
@@ -437,11 +448,11 @@ __device__ __forceinline__ bool collide_f64(const StepParams& P, const SpeciesDe
                 if (c < P.n_mix) {
                     const double sn = P.mix_sig[c];
                     double u1 = rng.uniform_f64(), u2 = rng.uniform_f64();
-                    vn[c].x = sn * sqrt(-2.0 * log(u1)) * cos(2.0 * kPi * u2);
+                    vn[c].x = sn * normal_of(u1, u2);
                     u1 = rng.uniform_f64(); u2 = rng.uniform_f64();
-                    vn[c].y = sn * sqrt(-2.0 * log(u1)) * cos(2.0 * kPi * u2);
+                    vn[c].y = sn * normal_of(u1, u2);
                     u1 = rng.uniform_f64(); u2 = rng.uniform_f64();
-                    vn[c].z = sn * sqrt(-2.0 * log(u1)) * cos(2.0 * kPi * u2);
+                    vn[c].z = sn * normal_of(u1, u2);
                     vn[c] = vn[c] + u_gas;
                     const d3 vr = v - vn[c];
                     const double vm = sqrt(dot(vr, vr));
@@ -524,11 +535,11 @@ __device__ __forceinline__ bool collide_f64(const StepParams& P, const SpeciesDe
         d3 vn;
         {
             double u1 = rng.uniform_f64(), u2 = rng.uniform_f64();
-            vn.x = P.sigma_neutral * sqrt(-2.0 * log(u1)) * cos(2.0 * kPi * u2);
+            vn.x = P.sigma_neutral * normal_of(u1, u2);
             u1 = rng.uniform_f64(); u2 = rng.uniform_f64();
-            vn.y = P.sigma_neutral * sqrt(-2.0 * log(u1)) * cos(2.0 * kPi * u2);
+            vn.y = P.sigma_neutral * normal_of(u1, u2);
             u1 = rng.uniform_f64(); u2 = rng.uniform_f64();
-            vn.z = P.sigma_neutral * sqrt(-2.0 * log(u1)) * cos(2.0 * kPi * u2);
+            vn.z = P.sigma_neutral * normal_of(u1, u2);
             vn = vn + u_gas;
         }
         const d3 vrel = v - vn;

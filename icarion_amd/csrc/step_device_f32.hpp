@@ -18,10 +18,6 @@ __device__ __forceinline__ void kahan_add(float& hi, float& lo, float d) {
     hi = t;
 }
 
-// Keeps a wave-uniform branch a branch: without it the compiler computes both
-// sides in every step and selects.
-__device__ __forceinline__ void keep_branch() { asm volatile(""); }
-
 // hardware transcendentals: v_log_f32 (log2), v_exp_f32 (exp2), v_sin/cos_f32
 // (argument in revolutions), v_sqrt_f32, v_rcp_f32
 __device__ __forceinline__ float fast_ln(float u) { return __builtin_amdgcn_logf(u) * 0.69314718056f; }

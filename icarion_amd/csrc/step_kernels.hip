@@ -19,6 +19,24 @@
 
 namespace icarion {
 
+// The per-ion factor of the damping coefficient (DampingForce.cpp:150-177 / :269-271).
+__device__ __forceinline__ double damping_factor_f64(const StepParams& P, const SpeciesDev& sp, double m, double q) {
+    if (P.damping_model == 3) {
+        if (P.alpha_gas > 0.0 && P.n > 0.0 && P.v_th > 0.0 && P.m_gas > 0.0) {
+            const double mu = (m * P.m_gas) / (m + P.m_gas);
+            const double cs1 = kPi * q * sqrt(P.alpha_gas / (4.0 * kPi * kEpsilon0 * mu));
+            return P.n * cs1 * P.v_th * P.m_gas / (P.m_gas + m);
+        }
+    } else {
+        const double K0 = sp.K0_cm2_Vs;
+        if (K0 > 0.0 && m > 0.0 && P.n > 0.0) {
+            const double K0t = K0 * 1e-4 * sqrt(kStpTemp / fmax(P.T, 1.0));
+            return q / ((K0t * (kLoschmidt / P.n)) * m);
+        }
+    }
+    return 0.0;
+}
+
 // SUB: collision substeps; FLOW: the AxialParabolic gas flow (both read from P
 // at run time, instantiated apart because they cost the plain kernels
 // registers).
@@ -38,44 +56,31 @@ __device__ __forceinline__ void f64_ion(const StepParams& P, const IonPtrs& S, c
     double arrival = S.arrival[i];
     uint32_t nc = S.ncoll[i];
     const double inv_m = 1.0 / m;
-    // hoisted damping factor (DampingForce.cpp:150-177 / :269-271)
     double lpre = 0.0;
-    if constexpr (COLL == COLL_DAMPING) {
-        if (P.damping_model == 3) {
-            if (P.alpha_gas > 0.0 && P.n > 0.0 && P.v_th > 0.0 && P.m_gas > 0.0) {
-                const double mu = (m * P.m_gas) / (m + P.m_gas);
-                const double cs1 = kPi * q * sqrt(P.alpha_gas / (4.0 * kPi * kEpsilon0 * mu));
-                lpre = P.n * cs1 * P.v_th * P.m_gas / (P.m_gas + m);
-            }
-        } else {
-            const double K0 = sp.K0_cm2_Vs;
-            if (K0 > 0.0 && m > 0.0 && P.n > 0.0) {
-                const double K0t = K0 * 1e-4 * sqrt(kStpTemp / fmax(P.T, 1.0));
-                lpre = q / ((K0t * (kLoschmidt / P.n)) * m);
-            }
-        }
-    }
-    bool checked = false;   // position known to be inside the domain
+    if constexpr (COLL == COLL_DAMPING) lpre = damping_factor_f64(P, sp, m, q);
+    // 0: done, 1: stepping, 2: unborn, 3: stepping, position not yet known to
+    // be inside (see f32_ion: the loop is wave-uniform, its body masked)
+    uint32_t state = !born ? 2u : active ? 3u : 0u;
     const double dt = P.dt;
     const double half_dt = dt * 0.5;
     for (uint32_t k = 0; k < P.n_steps; ++k) {
-        const StepEntry te = P.table[k];
+        if (__ballot(state != 0u) == 0ull) break;
+        const StepEntry& te = P.table[k];
         const double t = te.t;
-        if (!born) {
-            if (t >= birth) {
+        if (__ballot(state > 1u) != 0ull) {   // before an ion's first step only
+            if (state == 2u && t >= birth) {
                 born = true;
-                active = true;
-                checked = false;
-            } else {
-                continue;
+                state = 3u;
+            }
+            if (state == 3u) {
+                state = 1u;
+                if (!contains_f64(P, pos)) {
+                    state = 0u;
+                    death = t;
+                }
             }
         }
-        if (!active) break;
-        if (!checked && !contains_f64(P, pos)) {
-            active = false;
-            death = t;
-            break;
-        }
+        if (state != 1u) continue;
         const double z_before = pos.z;
         // the step's gas density (update_dynamic_environments at the step
         // start, SimulationEngine.cpp:380): the damping coefficient and the
@@ -131,23 +136,18 @@ __device__ __forceinline__ void f64_ion(const StepParams& P, const IonPtrs& S, c
                 }
             }
         }
-        if (P.detect && isnan(arrival)) {
-            if (z_before < P.det_z && pos.z >= P.det_z)
+        if (P.detect) {
+            keep_branch();
+            if (isnan(arrival) && z_before < P.det_z && pos.z >= P.det_z)
                 arrival = t + dt * (P.det_z - z_before) / (pos.z - z_before);
         }
-        if (!contains_f64(P, pos)) {
-            active = false;
+        if (!(contains_f64(P, pos) & isfinite(pos.x) & isfinite(pos.y) & isfinite(pos.z) & isfinite(vel.x) &
+              isfinite(vel.y) & isfinite(vel.z))) {
+            state = 0u;
             death = t;
-            break;
-        }
-        checked = true;
-        if (!(isfinite(pos.x) && isfinite(pos.y) && isfinite(pos.z) && isfinite(vel.x) &&
-              isfinite(vel.y) && isfinite(vel.z))) {
-            active = false;
-            death = t;
-            break;
         }
     }
+    if (state != 2u) active = state != 0u;
     S.x[i] = pos.x; S.y[i] = pos.y; S.z[i] = pos.z;
     S.vx[i] = vel.x; S.vy[i] = vel.y; S.vz[i] = vel.z;
     S.flags[i] = static_cast<uint8_t>((active ? 1 : 0) | (born ? 2 : 0));
@@ -162,6 +162,181 @@ __global__ void __launch_bounds__(256) step_f64_kernel(const StepParams P, const
     uint32_t pushed = 0, ncoll_launch = 0;
     if (i < P.n_ions) f64_ion<INTEG, FIELD, COLL, SUB, SUB>(P, S, P.order ? P.order[i] : i, pushed, ncoll_launch);
     add_counters(P, pushed, ncoll_launch);
+}
+
+// ======================= FP64, four lanes per ion ============================
+//
+// The step of f64_ion for the analytic linear fields (no magnetic field) with
+// one ion on four lanes: lanes 0-2 hold the x, y and z components, lane 3
+// repeats z.  The draws of a step are four or five Philox blocks, three or four
+// Box-Muller transforms and a direction: lane c takes block c, so one block, one
+// logarithm, one sine and cosine per lane replace them (lane 3 draws the
+// collision test and the direction).  Scalars of an ion (speeds, tests) are
+// formed on all four lanes from broadcast components, in f64_ion's order of
+// operations: the results agree with it to rounding.
+// A wavefront's step is a third of f64_ion's instructions for a quarter of the
+// ions, and a cloud that does not fill the chip is bound by exactly that chain
+// (10,000 ions x 5000 HSS steps: 19.4 ms with f64_ion and the general sine,
+// cosine and logarithm, 7.6 ms here; 30,000 x 1000: 4.5 and 2.7 ms).  From three
+// wavefronts per SIMD on the lanes repeated by an ion cost what the chain gains:
+// 65,000 ions x 1000 steps took 4.6 ms here and 4.9 ms before both.
+constexpr uint32_t kQuadMaxIons = 49152;
+
+// Component K (0-3) of the ion's four lanes, on each of them.
+template <int K>
+__device__ __forceinline__ double quad_f64(double x) {
+    const int lo = __double2loint(x), hi = __double2hiint(x);
+    return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, K * 0x55, 0xf, 0xf, false),
+                            __builtin_amdgcn_update_dpp(lo, lo, K * 0x55, 0xf, 0xf, false));
+}
+__device__ __forceinline__ d3 quad_d3(double x) { return d3{quad_f64<0>(x), quad_f64<1>(x), quad_f64<2>(x)}; }
+
+template <int INTEG, int COLL>
+__global__ void __launch_bounds__(256) step_f64_quad_kernel(const StepParams P, const IonPtrs S) {
+    const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t c = tid & 3u;
+    const bool valid = (tid >> 2) < P.n_ions;
+    const uint32_t i = valid ? tid >> 2 : 0u;
+    const int comp = c < 2u ? static_cast<int>(c) : 2;
+    double* const px = comp == 0 ? S.x : comp == 1 ? S.y : S.z;
+    double* const pv = comp == 0 ? S.vx : comp == 1 ? S.vy : S.vz;
+    double p = px[i], v = pv[i];
+    const double m = S.mass[i], q = S.charge[i];
+    const uint32_t sidx = S.species[i];
+    const SpeciesDev sp = P.species[sidx];
+    const uint8_t flags = S.flags[i];
+    bool active = flags & 1, born = (flags >> 1) & 1;
+    const double birth = S.birth ? S.birth[i] : -INFINITY;
+    double death = S.death[i], arrival = S.arrival[i];
+    uint32_t nc = S.ncoll[i];
+    const double inv_m = 1.0 / m;
+    double lpre = 0.0;
+    if constexpr (COLL == COLL_DAMPING) lpre = damping_factor_f64(P, sp, m, q);
+    const double rf_sign = comp == 0 ? -2.0 : 2.0;
+    const double u_gas = comp == 0 ? P.u_gas[0] : comp == 1 ? P.u_gas[1] : P.u_gas[2];
+    const double inv_mt = 1.0 / (m + P.m_gas);
+    uint32_t pushed = 0, ncoll_launch = 0;
+    uint32_t state = !valid ? 0u : !born ? 2u : active ? 3u : 0u;   // as in f64_ion, alike on the ion's lanes
+    const double dt = P.dt;
+    const double half_dt = dt * 0.5;
+    for (uint32_t k = 0; k < P.n_steps; ++k) {
+        if (__ballot(state != 0u) == 0ull) break;
+        const StepEntry& te = P.table[k];
+        const double t = te.t;
+        if (__ballot(state > 1u) != 0ull) {   // before an ion's first step only
+            if (state == 2u && t >= birth) {
+                born = true;
+                state = 3u;
+            }
+            const bool in = contains_f64(P, quad_d3(p));
+            if (state == 3u) {
+                state = in ? 1u : 0u;
+                if (!in) death = t;
+            }
+        }
+        if (state != 1u) continue;
+        const double p_before = p;
+        const double lp = lpre * te.nrel;
+        // this lane's component of force / mass at (pc, vc)
+        auto accel = [&](double pc, double vc, double c_rf, double ez) {
+            double E = comp == 2 ? ez : 0.0;
+            if (P.has_rf && comp != 2) E = rf_sign * pc * c_rf;
+            double F = E * q;
+            if constexpr (COLL == COLL_DAMPING) {
+                const double g = gamma_f64(P, lp, quad_d3(vc));
+                if (g > 0.0) F = F + (vc - u_gas) * (-g * m);
+            }
+            return F * inv_m;
+        };
+        if constexpr (INTEG == 0) {
+            const double k1a = accel(p, v, te.c0, te.e0);
+            const double k2v = v + k1a * half_dt;
+            const double k2a = accel(p + v * half_dt, k2v, te.ch, te.eh);
+            const double k3v = v + k2a * half_dt;
+            const double k3a = accel(p + k2v * half_dt, k3v, te.ch, te.eh);
+            const double k4v = v + k3a * dt;
+            const double k4a = accel(p + k3v * dt, k4v, te.c1, te.e1);
+            const double h6 = dt / 6.0;
+            p = p + (v + k2v * 2.0 + k3v * 2.0 + k4v) * h6;
+            v = v + (k1a + k2a * 2.0 + k3a * 2.0 + k4a) * h6;
+        } else {
+            const double a = accel(p, v, te.c0, te.e0);
+            const double vm = v + a * half_dt;
+            p = p + vm * dt;
+            v = vm + a * half_dt;
+        }
+        ++pushed;
+        if constexpr (COLL == COLL_HSS) {
+            if (sp.sigma_hss > 0.0) {
+                const uint32_t s_lo = static_cast<uint32_t>(P.step0 + k), s_hi = static_cast<uint32_t>((P.step0 + k) >> 32);
+                const uint32_t k0 = static_cast<uint32_t>(P.seed), k1 = static_cast<uint32_t>(P.seed >> 32);
+                // draws 2 c and 2 c + 1 on lane c; draw 8 (the direction's angle) on all
+                const u32x4 o = philox4x32_10(c, i, s_lo, s_hi, k0, k1);
+                const u32x4 o4 = philox4x32_10(4u, i, s_lo, s_hi, k0, k1);
+                const double ua = uniform53(o.v[0], o.v[1]), ub = uniform53(o.v[2], o.v[3]);
+                double sn, cs;
+                sincos_rev(c == 3u ? uniform53(o4.v[0], o4.v[1]) : ub, sn, cs);
+                const double vn = P.sigma_neutral * (sqrt(-2.0 * log_unit(ua)) * cs) + u_gas;
+                const d3 rel = quad_d3(v - vn);
+                const double vm = sqrt(dot(rel, rel));
+                const double Pc = 1.0 - exp(-P.n * sp.sigma_hss * vm * (dt * te.nrel));
+                // lane 3's draws, on every lane (before any lane-dependent choice:
+                // a broadcast reads its source lane only while that is active)
+                const double u_test = quad_f64<3>(ua), u_dir = quad_f64<3>(ub);
+                const double sn3 = quad_f64<3>(sn), cs3 = quad_f64<3>(cs);
+                // vm below kMinRelativeVelocity: no collision (above it hss_collision's
+                // smaller bound never applies)
+                if (vm >= kMinRelativeVelocity && u_test < Pc) {
+                    const double cosT = 2.0 * u_dir - 1.0;
+                    const double sinT = sqrt(fmax(0.0, 1.0 - cosT * cosT));
+                    const double nd = comp == 2 ? cosT : sinT * (comp == 0 ? cs3 : sn3);
+                    v = (v * m + vn * P.m_gas) * inv_mt + (nd * vm) * (P.m_gas * inv_mt);
+                    ++nc;
+                    ++ncoll_launch;
+                }
+            }
+        } else if constexpr (COLL == COLL_DAMPING) {
+            if (P.ou_kicks) {
+                const double g = gamma_f64(P, lp, quad_d3(v));
+                if (g > 0.0 && dt > 0.0) {
+                    // draws 0, 1 for x (cosine) and y (sine), 2, 3 for z (cosine)
+                    const u32x4 o = philox4x32_10(c >> 1, i, static_cast<uint32_t>(P.step0 + k),
+                                                  static_cast<uint32_t>((P.step0 + k) >> 32),
+                                                  static_cast<uint32_t>(P.seed), static_cast<uint32_t>(P.seed >> 32));
+                    double sn, cs;
+                    sincos_rev(uniform53(o.v[2], o.v[3]), sn, cs);
+                    const double r = sqrt(-2.0 * log_unit(uniform53(o.v[0], o.v[1])));
+                    const double kBT_over_m = kBoltzmann * P.T / m;
+                    const double s = sqrt(2.0 * g * kBT_over_m * dt);
+                    v += s * (r * (comp == 1 ? sn : cs));
+                }
+            }
+        }
+        if (P.detect) {
+            keep_branch();
+            const double zb = quad_f64<2>(p_before), za = quad_f64<2>(p);
+            if (isnan(arrival) && zb < P.det_z && za >= P.det_z) arrival = t + dt * (P.det_z - zb) / (za - zb);
+        }
+        const d3 pos = quad_d3(p), vel = quad_d3(v);
+        if (!(contains_f64(P, pos) & isfinite(pos.x) & isfinite(pos.y) & isfinite(pos.z) & isfinite(vel.x) &
+              isfinite(vel.y) & isfinite(vel.z))) {
+            state = 0u;
+            death = t;
+        }
+    }
+    if (state != 2u) active = state != 0u;
+    if (valid) {
+        if (c < 3u) {
+            px[i] = p;
+            pv[i] = v;
+        } else {
+            S.flags[i] = static_cast<uint8_t>((active ? 1 : 0) | (born ? 2 : 0));
+            S.death[i] = death;
+            S.arrival[i] = arrival;
+            S.ncoll[i] = nc;
+        }
+    }
+    add_counters(P, c == 3u ? pushed : 0u, c == 3u ? ncoll_launch : 0u);
 }
 
 // ======================= FP64 geometry EHSS, wave-cooperative ===============
@@ -261,7 +436,7 @@ struct EhssDraws {
         double u1, u2, sn, cs;
         pair(5u + attempt, ion, u1, u2);
         const double b = sqrt(u1);
-        sincos(2.0 * kPi * u2, &sn, &cs);
+        sincos_rev(u2, sn, cs);
         ux = b * cs;
         uy = b * sn;
     }
@@ -370,11 +545,11 @@ __global__ void __launch_bounds__(256) step_f64_ehss_kernel(const StepParams P, 
         if (live && sp.sigma_ehss > 0.0) {
             double u1, u2;
             rng.pair(0u, i, u1, u2);
-            vn.x = P.sigma_neutral * sqrt(-2.0 * log(u1)) * cos(2.0 * kPi * u2);
+            vn.x = P.sigma_neutral * normal_of(u1, u2);
             rng.pair(1u, i, u1, u2);
-            vn.y = P.sigma_neutral * sqrt(-2.0 * log(u1)) * cos(2.0 * kPi * u2);
+            vn.y = P.sigma_neutral * normal_of(u1, u2);
             rng.pair(2u, i, u1, u2);
-            vn.z = P.sigma_neutral * sqrt(-2.0 * log(u1)) * cos(2.0 * kPi * u2);
+            vn.z = P.sigma_neutral * normal_of(u1, u2);
             vn = vn + d3{P.u_gas[0], P.u_gas[1], P.u_gas[2]};
             vrel = vel - vn;
             vrel_mag = sqrt(dot(vrel, vrel));
@@ -393,8 +568,8 @@ __global__ void __launch_bounds__(256) step_f64_ehss_kernel(const StepParams P, 
                 double u2, u3;
                 rng.pair(4u, i, u2, u3);
                 double s2, c2, s3, c3;
-                sincos(2.0 * kPi * u2, &s2, &c2);
-                sincos(2.0 * kPi * u3, &s3, &c3);
+                sincos_rev(u2, s2, c2);
+                sincos_rev(u3, s3, c3);
                 const double x = sqrt(1.0 - u1) * s2;
                 const double y = sqrt(1.0 - u1) * c2;
                 const double z = sqrt(u1) * s3;
@@ -1324,6 +1499,24 @@ KernelFn pick_surrogate(int field) {
     }
 }
 
+// The four-lanes-per-ion kernel of a combination, or null.
+KernelFn pick_quad(int integrator, int field, int coll) {
+    if (field != FIELD_LINEAR) return nullptr;
+    switch (coll) {
+        case COLL_NONE: return integrator == 1 ? step_f64_quad_kernel<1, COLL_NONE> : step_f64_quad_kernel<0, COLL_NONE>;
+        case COLL_HSS: return integrator == 1 ? step_f64_quad_kernel<1, COLL_HSS> : step_f64_quad_kernel<0, COLL_HSS>;
+        case COLL_DAMPING:
+            return integrator == 1 ? step_f64_quad_kernel<1, COLL_DAMPING> : step_f64_quad_kernel<0, COLL_DAMPING>;
+        default: return nullptr;
+    }
+}
+
+hipError_t launch_quad(KernelFn fn, const StepParams& P, const IonPtrs& S, hipStream_t stream) {
+    const uint32_t per_block = 256 / 4;
+    hipLaunchKernelGGL(fn, dim3((P.n_ions + per_block - 1) / per_block), dim3(256), 0, stream, P, S);
+    return hipGetLastError();
+}
+
 // Ions per wavefront of the geometry EHSS kernel: two wavefronts per SIMD fit
 // (registers and LDS), 2048 on the chip.  A wavefront works through its
 // colliding ions one after another, so the ions are spread evenly over the
@@ -1347,6 +1540,9 @@ hipError_t launch_step(int integrator, int field, int coll, int precision, int s
         // the extended instantiation: collision substeps or a parabolic flow
         const bool ext = P.n_sub > 1 || P.flow_parabolic;
         fn = integrator == 1 ? pick_field<1>(field, coll, precision, ext) : pick_field<0>(field, coll, precision, ext);
+        if (KernelFn quad = pick_quad(integrator, field, coll); quad && precision == 0 && !ext && !P.magnetic &&
+                                                                !P.order && P.n_ions <= kQuadMaxIons)
+            return launch_quad(quad, P, S, stream);
     }
     if (!fn) return hipErrorInvalidValue;
     // the surrogate kernel runs its own workgroup size (the handle's block size

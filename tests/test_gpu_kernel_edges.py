@@ -84,3 +84,39 @@ def test_field_array_cell_changes(oracle, n, grid, precision, integrator):
     for f, scale in (("x", 1e-3), ("y", 1e-3), ("z", 1e-2), ("vx", 1e3), ("vy", 1e3), ("vz", 1e4)):
         d = np.abs(getattr(g, f) - getattr(o, f))[both]
         assert d.size == 0 or d.max() <= tol * np.maximum(scale, np.abs(getattr(o, f))[both].max()), f
+
+
+@pytest.mark.parametrize("kind", ["drift", "trap_ou", "trap_quiet", "none", "friction"])
+@pytest.mark.parametrize("integrator", [_abi.INTEGRATOR_RK4, _abi.INTEGRATOR_BORIS])
+@pytest.mark.parametrize("n", [1, 15, 1025, 49152, 49153])
+def test_fp64_lanes_per_ion(oracle, n, integrator, kind):
+    """Both sides of the four-lanes-per-ion bound, partial quads and wavefronts,
+    births during the run, arrivals and losses, a rotated domain."""
+    if kind == "drift":
+        w = W.ims_hss_workload(n=n, seed=n)
+        w["domain"].detector_z_m = 2e-4
+        c, s = np.cos(0.3), np.sin(0.3)
+        w["domain"].rot_g2l = (1.0, 0.0, 0.0, 0.0, c, s, 0.0, -s, c)
+        w["domain"].rot_l2g = (1.0, 0.0, 0.0, 0.0, c, -s, 0.0, s, c)
+        w["domain"].radius_m = 2.5e-3
+        coll, ou, steps = _abi.COLLISION_HSS, 0, 40
+    else:
+        w = W.quadrupole_workload(n=n, seed=n, U=20.0)
+        coll = {"none": _abi.COLLISION_NONE, "friction": _abi.COLLISION_FRICTION}.get(kind, _abi.COLLISION_LANGEVIN)
+        ou, steps = int(kind == "trap_ou"), 40
+        w["domain"].radius_m = 0.5e-3   # ions lost during the run
+        w["species"] = [W.species(K0=2.1, ccs=100e-20)]
+    w["physics"] = W.physics(integrator, coll, ou=ou, seed=n)
+    ens = w["ensemble"]
+    rng = np.random.default_rng(n)
+    ens.birth_time_s = np.where(rng.random(n) < 0.3, rng.uniform(0.0, 50.0, n) * w["dt"], 0.0)
+    ens.born[:] = ens.birth_time_s == 0.0
+    ens.active[:] = ens.born
+    g, o = ens.copy(), ens.copy()
+    sg = gpu_run(w, g, steps)
+    so = oracle_run(oracle, w, o, steps)
+    assert (sg.ion_steps, sg.collisions, sg.alive, sg.arrived) == (so.ion_steps, so.collisions, so.alive, so.arrived)
+    assert compare_ions(g, o, rtol=1e-9).all()
+    assert np.array_equal(g.born, o.born) and np.array_equal(g.n_collisions, o.n_collisions)
+    np.testing.assert_allclose(g.death_time_s, o.death_time_s, rtol=1e-12)
+    np.testing.assert_allclose(g.arrival_time_s, o.arrival_time_s, rtol=1e-9)
