@@ -932,7 +932,7 @@ __global__ void __launch_bounds__(256) step_f32_kernel(const StepParams P, const
 // reflected about it (offline-table branch, EHSSCollisionHandler.cpp:253-277).
 // mlp_eval(step, coll, in, out) evaluates the MLP for the colliding lanes:
 // mlp_group_eval (the single-cloud kernel: the workgroup's colliding ions
-// gathered into 64-ion batches through LDS, so the matrix cores evaluate about
+// gathered into 32-ion blocks through LDS, so the matrix cores evaluate about
 // as many rows as there are collisions) or mlp_wave_eval_any (the batch
 // kernel: per wavefront, no barriers).  Every lane stays in the step loop
 // (dead lanes are masked, not exited) so that barriers and the wave-wide matrix
@@ -1097,7 +1097,10 @@ __global__ void __launch_bounds__(kSurrogateBlock, 3) step_surrogate_kernel(cons
     mlp_stage(P.mlp_blob, mlp_lds);
     const unsigned char* lds = reinterpret_cast<const unsigned char*>(mlp_lds);
     uint32_t pushed = 0, nc = 0;
-    surr_ion<INTEG, FIELD>(P, S, blockIdx.x * blockDim.x + threadIdx.x,
+    // lanes below ions_per_wave own an ion each; the others take part in the MLP
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t first = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * P.ions_per_wave;
+    surr_ion<INTEG, FIELD>(P, S, lane < P.ions_per_wave ? first + lane : 0xFFFFFFFFu,
                            [&](uint32_t k, bool coll, const float* in, float* out) {
                                return mlp_group_eval(lds, xch, k, coll, in, out, k + blockIdx.x);
                            },
@@ -1528,6 +1531,19 @@ uint32_t ehss_ions_per_wave(uint32_t n_ions) {
     return g < 1 ? 1 : g > 64 ? 64 : g;
 }
 
+// Ions per wavefront of the surrogate kernel: up to 131,072 ions one or two
+// wavefronts per SIMD, evenly filled (a step lasts as long as the workgroup's
+// chain, which is shorter with fewer colliding ions: 30,000 ions x 1000 steps
+// 5.7 ms with 64 per wavefront, 4.0 ms spread); above that full wavefronts, for
+// full MLP blocks.
+uint32_t surrogate_ions_per_wave(uint32_t n_ions) {
+    const uint32_t waves = 1024;
+    const uint32_t rounds = (n_ions + 64 * waves - 1) / (64 * waves);
+    if (rounds > 2) return 64;
+    const uint32_t g = (n_ions + rounds * waves - 1) / (rounds * waves);
+    return g < 1 ? 1 : g;
+}
+
 // Returns hipSuccess, or hipErrorInvalidValue when the combination has no
 // kernel (the host maps that to ICARION_ERR_UNSUPPORTED).
 hipError_t launch_step(int integrator, int field, int coll, int precision, int surrogate,
@@ -1545,12 +1561,12 @@ hipError_t launch_step(int integrator, int field, int coll, int precision, int s
             return launch_quad(quad, P, S, stream);
     }
     if (!fn) return hipErrorInvalidValue;
-    // the surrogate kernel runs its own workgroup size (the handle's block size
+    // the EHSS kernels run their own workgroup size (the handle's block size
     // does not change any result)
-    if (surrogate) block = kSurrogateBlock;
+    static_assert(kSurrogateBlock == 256, "four wavefronts per workgroup");
     uint32_t grid = (P.n_ions + block - 1) / block;
-    if (!surrogate && coll == COLL_EHSS) {
-        P.ions_per_wave = ehss_ions_per_wave(P.n_ions);
+    if (surrogate || coll == COLL_EHSS) {
+        P.ions_per_wave = surrogate ? surrogate_ions_per_wave(P.n_ions) : ehss_ions_per_wave(P.n_ions);
         block = 256;
         const uint32_t per_block = 4 * P.ions_per_wave;
         grid = (P.n_ions + per_block - 1) / per_block;

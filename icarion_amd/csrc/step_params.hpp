@@ -238,7 +238,7 @@ struct StepParams {
     uint64_t seed;
     uint32_t n_steps;
     uint32_t n_ions;
-    uint32_t ions_per_wave;   // geometry EHSS kernel: ions each wavefront owns
+    uint32_t ions_per_wave;   // EHSS kernels: ions each wavefront owns
     // lane t of the launch takes ion order[t] (a permutation of the ions that
     // puts neighbours in the field-array grid on neighbouring lanes); null:
     // lane t takes ion t.  The ion keeps its index (state, random streams).

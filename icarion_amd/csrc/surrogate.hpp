@@ -316,7 +316,7 @@ __device__ __forceinline__ bool mlp_wave_eval_any(const unsigned char* lds, bool
 }
 
 // LDS exchange of a workgroup (up to 4 wavefronts) whose colliding ions are
-// gathered into full 64-ion batches for the MLP.  Wavefront w writes the inputs
+// gathered into full 32-ion blocks for the MLP.  Wavefront w writes the inputs
 // of its colliding lanes, in lane order, to slots 64 w .. 64 w + count - 1, as
 // the eight bf16 operand slots of layer 1 (x0..x5, 1, 0); the counts are
 // double-buffered by step parity, since a workgroup without any colliding ion
@@ -339,14 +339,16 @@ __device__ __forceinline__ void mlp_exchange_init(MlpExchange<WAVES>& X) {
 // MLP outputs for the colliding lanes of the whole workgroup.  Every lane of
 // every wavefront calls this once per step (it holds barriers); `coll` lanes
 // pass their inputs in in[] and receive their outputs in out[].  The colliding
-// ions are numbered wavefront by wavefront, lane by lane; batch b holds ions
-// 64 b .. 64 b + 63 of that numbering and is evaluated by wavefront
-// (b + rot) mod (waves), so that successive steps spread the matrix work over
-// the SIMDs.  Batches are padded with zero operands whose outputs are dropped.
-// An ion's outputs do not depend on its batch or column: each output column of
-// a matrix instruction is its own dot product, and the operands are the bf16
-// values mlp_wave_eval forms.  Returns false when no ion of the workgroup
-// collides (out[] is then untouched).
+// ions are numbered wavefront by wavefront, lane by lane; block b holds ions
+// 32 b .. 32 b + 31 of that numbering and is evaluated by wavefront
+// (b + rot) mod (waves), so that a step's blocks run side by side on the SIMDs
+// (a step waits for the wavefront with the most blocks: with two blocks after
+// one another per wavefront 3001 ions x 2000 steps took 10.5 ms, now 6.9 ms,
+// 1M x 4000 158.9 and 151.8 ms) and successive steps spread the odd one.  The last block is padded with zero operands whose
+// outputs are dropped.  An ion's outputs do not depend on its block or column:
+// each output column of a matrix instruction is its own dot product, and the
+// operands are the bf16 values mlp_wave_eval forms.  Returns false when no ion
+// of the workgroup collides (out[] is then untouched).
 template <int WAVES>
 __device__ __forceinline__ bool mlp_group_eval(const unsigned char* lds, MlpExchange<WAVES>& X, uint32_t step,
                                                bool coll, const float in[kMlpIn], float out[kMlpOut],
@@ -376,12 +378,16 @@ __device__ __forceinline__ bool mlp_group_eval(const unsigned char* lds, MlpExch
     for (int v = 0; v < WAVES; ++v) start[v + 1] = start[v] + __builtin_amdgcn_readfirstlane(cnt[v]);
     const uint32_t total = start[WAVES];
     if (total == 0) return false;
-    const uint32_t nb = (total + 63) >> 6;
-    const uint32_t b = (w + nw - rot % nw) % nw;
-    if (b < nb) {
-        // slot of colliding ion g (g < total) in the exchange: its wavefront
-        // is the number of wavefront starts past 0 at or below g
-        auto slot_of = [&](uint32_t g) {
+    const uint32_t half = lane >> 5;
+    const uint32_t* xin = reinterpret_cast<const uint32_t*>(X.in);
+    for (uint32_t b = (w + nw - rot % nw) % nw; 32 * b < total; b += nw) {
+        // lanes l and l + 32 carry ion 32 b + l: operand slots 0-3 and 4-7.  Its
+        // slot in the exchange: its wavefront is the number of wavefront starts
+        // past 0 at or below its number
+        const uint32_t g = 32 * b + (lane & 31);
+        const bool have = g < total;
+        uint32_t s = 0u, o0 = 0u, o1 = 0u;
+        if (have) {
             uint32_t ww = 0, base = 0;
 #pragma unroll
             for (int v = 1; v < WAVES; ++v) {
@@ -389,55 +395,25 @@ __device__ __forceinline__ bool mlp_group_eval(const unsigned char* lds, MlpExch
                 ww += past ? 1u : 0u;
                 base = past ? start[v] : base;
             }
-            return 64 * ww + (g - base);
-        };
-        const uint32_t half = lane >> 5;
-        const uint32_t g_own = 64 * b + lane, g_par = g_own ^ 32u;
-        const bool have_own = g_own < total, have_par = g_par < total;
-        const uint32_t s_own = have_own ? slot_of(g_own) : 0u;
-        const uint32_t s_par = have_par ? slot_of(g_par) : 0u;
-        // lane l carries operand slots 4*half .. 4*half+3: dwords 2*half, 2*half+1
-        const uint32_t* xin = reinterpret_cast<const uint32_t*>(X.in);
-        uint32_t o0 = 0u, o1 = 0u, q0 = 0u, q1 = 0u;
-        if (have_own) {
-            o0 = xin[4 * s_own + 2 * half];
-            o1 = xin[4 * s_own + 2 * half + 1];
+            s = 64 * ww + (g - base);
+            o0 = xin[4 * s + 2 * half];
+            o1 = xin[4 * s + 2 * half + 1];
         }
-        if (have_par) {
-            q0 = xin[4 * s_par + 2 * half];
-            q1 = xin[4 * s_par + 2 * half + 1];
-        }
-        const bf16x4 own = __builtin_bit_cast(bf16x4, static_cast<uint64_t>(o0) | (static_cast<uint64_t>(o1) << 32));
-        const bf16x4 par = __builtin_bit_cast(bf16x4, static_cast<uint64_t>(q0) | (static_cast<uint64_t>(q1) << 32));
-        // block 0 = ions 64 b + 0..31, block 1 = ions 64 b + 32..63; the
-        // blocks go through the network one at a time (fewer live registers),
-        // and a block past the last colliding ion is skipped
-        const bf16x4 X0 = half == 0 ? own : par;
-        const bf16x4 X1 = half == 0 ? par : own;
-        const uint32_t n_blocks = total > 64 * b + 32 ? 2u : 1u;
+        const bf16x4 xb = __builtin_bit_cast(bf16x4, static_cast<uint64_t>(o0) | (static_cast<uint64_t>(o1) << 32));
         // a wave in its matrix-core section runs at raised priority so that
-        // its MFMA chain keeps issuing while the other wave of the SIMD fills
+        // its MFMA chain keeps issuing while the other waves of the SIMD fill
         // the gaps with vector work
         __builtin_amdgcn_s_setprio(1);
-        // lanes < 32: block 0 is ion g_own, block 1 is ion g_par = g_own + 32
         float r[3];
-        mlp_block_core(lds, X0, r);
-        if (half == 0 && have_own) {
+        mlp_block_core(lds, xb, r);
+        if (half == 0 && have) {
 #pragma unroll
-            for (int c = 0; c < kMlpOut; ++c) X.out[c][s_own] = r[c];
-        }
-        if (n_blocks > 1) {
-            // a compiler memory fence: the second block reloads the weight
-            // fragments from LDS instead of keeping the first block's 128
-            // registers of them live
-            asm volatile("" ::: "memory");
-            mlp_block_core(lds, X1, r);
-            if (half == 0 && have_par) {
-#pragma unroll
-                for (int c = 0; c < kMlpOut; ++c) X.out[c][s_par] = r[c];
-            }
+            for (int c = 0; c < kMlpOut; ++c) X.out[c][s] = r[c];
         }
         __builtin_amdgcn_s_setprio(0);
+        // a compiler memory fence: a second block reloads the weight fragments
+        // from LDS instead of keeping the first block's 128 registers of them
+        asm volatile("" ::: "memory");
     }
     __syncthreads();
     if (coll) {
