@@ -939,7 +939,14 @@ __global__ void __launch_bounds__(256) step_f32_kernel(const StepParams P, const
 // instructions see every lane they need.  One ion per lane over P.n_steps
 // steps; with mlp_group_eval every lane of the workgroup calls it with the same
 // P.n_steps (lanes with i >= P.n_ions are carried along masked).
-template <int INTEG, int FIELD, class MlpEval>
+// An index whose addresses are formed where it is used: hoisted out of the step
+// loop, the addresses of rare events take registers all along.
+__device__ __forceinline__ uint32_t here(uint32_t i) {
+    asm volatile("" : "+v"(i));
+    return i;
+}
+
+template <int INTEG, int FIELD, bool AHEAD, class MlpEval>
 __device__ __forceinline__ void surr_ion(const StepParams& P, const IonPtrs& S, uint32_t i,
                                          MlpEval&& mlp_eval, uint32_t& pushed, uint32_t& ncoll_launch) {
     const bool valid = i < P.n_ions;
@@ -959,34 +966,40 @@ __device__ __forceinline__ void surr_ion(const StepParams& P, const IonPtrs& S, 
     const float qm = (float)(qd / md);
     const float m = (float)md;
     const float inv_m_plus = (float)(1.0 / (md + P.m_gas));
-    uint8_t flags = S.flags[ii];
-    bool active = valid && (flags & 1), born = valid && ((flags >> 1) & 1);
-    const double birth = S.birth ? S.birth[ii] : -INFINITY;
-    double death = S.death[ii];
-    double arrival = S.arrival[ii];
-    uint32_t nc = S.ncoll[ii];
-    bool checked = false;
+    const uint8_t flags = S.flags[ii];
+    const bool active = flags & 1, born = (flags >> 1) & 1;
+    // 0: done, 1: stepping, 2: unborn, 3: stepping, position not yet known to
+    // be inside.  Birth, death and arrival times stay in memory until their
+    // event: registers decide this kernel's occupancy.
+    uint32_t state = !valid ? 0u : !born ? 2u : active ? 3u : 0u;
+    uint32_t nc = 0;
     const float dt = (float)P.dt;
     const float half_dt = 0.5f * dt;
     const float h6 = dt * (1.0f / 6.0f);
     CellF32 cell;
-    // the next step's table entry is loaded one step ahead
-    StepEntry te_next = P.n_steps ? P.table[0] : StepEntry{};
+    // AHEAD: the next step's table entry is loaded one step ahead
+    StepEntry te_next{};
+    if (AHEAD && P.n_steps) te_next = P.table[0];
     for (uint32_t k = 0; k < P.n_steps; ++k) {
-        const StepEntry te = te_next;
-        if (k + 1 < P.n_steps) te_next = P.table[k + 1];
+        StepEntry te;
+        if constexpr (AHEAD) {
+            te = te_next;
+            if (k + 1 < P.n_steps) te_next = P.table[k + 1];
+        } else {
+            te = P.table[k];
+        }
         const double t = te.t;
-        if (valid && !born && t >= birth) {
-            born = true;
-            active = true;
-            checked = false;
+        if (__ballot(state > 1u) != 0ull) {   // before an ion's first step only
+            if (state == 2u && (!S.birth || t >= S.birth[here(ii)])) state = 3u;
+            if (state == 3u) {
+                state = 1u;
+                if (!contains_f32(P, C, hi[0], hi[1], hi[2])) {
+                    state = 0u;
+                    S.death[here(ii)] = t;
+                }
+            }
         }
-        bool live = active && born;
-        if (live && !checked && !contains_f32(P, C, hi[0], hi[1], hi[2])) {
-            active = false;
-            death = t;
-            live = false;
-        }
+        const bool live = state == 1u;
         bool coll = false;
         float in[8] = {0, 0, 0, 0, 0, 0, 0, 0};
         f3 vn{0.f, 0.f, 0.f}, vrel{0.f, 0.f, 0.f};
@@ -1060,18 +1073,19 @@ __device__ __forceinline__ void surr_ion(const StepParams& P, const IonPtrs& S, 
             }
         }
         if (live) {
-            if (P.detect && isnan(arrival)) {
+            if (P.detect) {
+                keep_branch();
                 const double zb = (double)z_before + (double)z_before_lo;
                 const double za = (double)hi[2] + (double)lo[2];
-                if (zb < P.det_z && za >= P.det_z) arrival = t + P.dt * (P.det_z - zb) / (za - zb);
+                if (zb < P.det_z && za >= P.det_z) {
+                    double& arrival = S.arrival[here(ii)];
+                    if (isnan(arrival)) arrival = t + P.dt * (P.det_z - zb) / (za - zb);
+                }
             }
-            if (!contains_f32(P, C, hi[0], hi[1], hi[2]) ||
-                !(isfinite(hi[0]) && isfinite(hi[1]) && isfinite(hi[2]) && isfinite(hi[3]) &&
-                  isfinite(hi[4]) && isfinite(hi[5]))) {
-                active = false;
-                death = t;
-            } else {
-                checked = true;
+            if (!(contains_f32(P, C, hi[0], hi[1], hi[2]) & isfinite(hi[0]) & isfinite(hi[1]) & isfinite(hi[2]) &
+                  isfinite(hi[3]) & isfinite(hi[4]) & isfinite(hi[5]))) {
+                state = 0u;
+                S.death[here(ii)] = t;
             }
         }
     }
@@ -1082,15 +1096,17 @@ __device__ __forceinline__ void surr_ion(const StepParams& P, const IonPtrs& S, 
         S.vx[i] = (double)hi[3] + (double)lo[3];
         S.vy[i] = (double)hi[4] + (double)lo[4];
         S.vz[i] = (double)hi[5] + (double)lo[5];
-        S.flags[i] = static_cast<uint8_t>((active ? 1 : 0) | (born ? 2 : 0));
-        S.death[i] = death;
-        S.arrival[i] = arrival;
-        S.ncoll[i] = nc;
+        if (state != 2u) S.flags[i] = static_cast<uint8_t>((state != 0u ? 1 : 0) | 2);
+        S.ncoll[i] += nc;
     }
 }
 
-template <int INTEG, int FIELD>
-__global__ void __launch_bounds__(kSurrogateBlock, 3) step_surrogate_kernel(const StepParams P, const IonPtrs S) {
+// OCC: wavefronts per SIMD.  Four (128 registers, 40 KB of LDS per workgroup)
+// run a large cloud faster, three a small one, whose one or two wavefronts per
+// SIMD gain from the registers instead: 1M ions x 4000 steps 151.8 and 141 ms,
+// 3001 x 2000 6.9 and 7.8 ms (three and four).
+template <int INTEG, int FIELD, int OCC>
+__global__ void __launch_bounds__(kSurrogateBlock, OCC) step_surrogate_kernel(const StepParams P, const IonPtrs S) {
     __shared__ uint4 mlp_lds[kPackBytes / 16];
     __shared__ MlpExchange<kSurrogateBlock / 64> xch;
     mlp_exchange_init(xch);
@@ -1100,7 +1116,7 @@ __global__ void __launch_bounds__(kSurrogateBlock, 3) step_surrogate_kernel(cons
     // lanes below ions_per_wave own an ion each; the others take part in the MLP
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t first = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * P.ions_per_wave;
-    surr_ion<INTEG, FIELD>(P, S, lane < P.ions_per_wave ? first + lane : 0xFFFFFFFFu,
+    surr_ion<INTEG, FIELD, OCC == 3>(P, S, lane < P.ions_per_wave ? first + lane : 0xFFFFFFFFu,
                            [&](uint32_t k, bool coll, const float* in, float* out) {
                                return mlp_group_eval(lds, xch, k, coll, in, out, k + blockIdx.x);
                            },
@@ -1264,10 +1280,10 @@ __global__ void __launch_bounds__(256, 2) batch_surrogate_kernel(const StepParam
         if (wave_first < P.n_ions) {
             const uint32_t i = first + threadIdx.x;
             switch (kind) {
-                case 0: surr_ion<0, FIELD_LINEAR>(P, S, i, eval, pushed, nc); break;
-                case 1: surr_ion<1, FIELD_LINEAR>(P, S, i, eval, pushed, nc); break;
-                case 2: surr_ion<0, FIELD_ORBITRAP>(P, S, i, eval, pushed, nc); break;
-                case 3: surr_ion<1, FIELD_ORBITRAP>(P, S, i, eval, pushed, nc); break;
+                case 0: surr_ion<0, FIELD_LINEAR, true>(P, S, i, eval, pushed, nc); break;
+                case 1: surr_ion<1, FIELD_LINEAR, true>(P, S, i, eval, pushed, nc); break;
+                case 2: surr_ion<0, FIELD_ORBITRAP, true>(P, S, i, eval, pushed, nc); break;
+                case 3: surr_ion<1, FIELD_ORBITRAP, true>(P, S, i, eval, pushed, nc); break;
                 default: break;
             }
         }
@@ -1492,14 +1508,20 @@ KernelFn pick_field(int field, int coll, int precision, bool sub) {
     }
 }
 
-template <int I>
-KernelFn pick_surrogate(int field) {
+template <int I, int OCC>
+KernelFn pick_surrogate_occ(int field) {
     switch (field) {
-        case FIELD_ORBITRAP: return step_surrogate_kernel<I, FIELD_ORBITRAP>;
-        case FIELD_ARRAY: return step_surrogate_kernel<I, FIELD_ARRAY>;
-        case FIELD_ARRAY_X: return step_surrogate_kernel<I, FIELD_ARRAY_X>;
-        default: return step_surrogate_kernel<I, FIELD_LINEAR>;
+        case FIELD_ORBITRAP: return step_surrogate_kernel<I, FIELD_ORBITRAP, OCC>;
+        case FIELD_ARRAY: return step_surrogate_kernel<I, FIELD_ARRAY, OCC>;
+        case FIELD_ARRAY_X: return step_surrogate_kernel<I, FIELD_ARRAY_X, OCC>;
+        default: return step_surrogate_kernel<I, FIELD_LINEAR, OCC>;
     }
+}
+template <int I>
+KernelFn pick_surrogate(int field, bool large) {
+    // (the field-array kernels keep a cell's corners in registers: three)
+    const bool four = large && field != FIELD_ARRAY && field != FIELD_ARRAY_X;
+    return four ? pick_surrogate_occ<I, 4>(field) : pick_surrogate_occ<I, 3>(field);
 }
 
 // The four-lanes-per-ion kernel of a combination, or null.
@@ -1551,7 +1573,8 @@ hipError_t launch_step(int integrator, int field, int coll, int precision, int s
     StepParams P = params;
     KernelFn fn;
     if (surrogate) {
-        fn = integrator == 1 ? pick_surrogate<1>(field) : pick_surrogate<0>(field);
+        const bool large = surrogate_ions_per_wave(P.n_ions) == 64;
+        fn = integrator == 1 ? pick_surrogate<1>(field, large) : pick_surrogate<0>(field, large);
     } else {
         // the extended instantiation: collision substeps or a parabolic flow
         const bool ext = P.n_sub > 1 || P.flow_parabolic;

@@ -58,15 +58,16 @@ constexpr int kGemmWorkspaceFloats = kGemmSplitMax * (kMlpH * kMlpH + kMlpH);
 // Packed inference blob (bytes): bf16 A fragments in lane order, then biases.
 //   A1: [4 mb][64 lanes] x 4 bf16         ( 2048 B)  column 6 = b1
 //   A2: [4 mb][8 kc][64 lanes] x 8 bf16   (32768 B)
-//   A3: [8 kc][64 lanes] x 8 bf16         ( 8192 B)  rows 3..31 zero
+//   A3: [8 kc][2 halves][4 rows] x 8 bf16 ( 1024 B)  row 3 zero, read by the lanes
+//                                                    of rows 3..31
 //   b2[128] float                         (  512 B)  layer 2's accumulators start at b2
-//   b3[32] float                          (  128 B)
+//   b3[4] float                           (   16 B)
 constexpr int kPackA1 = 0;
 constexpr int kPackA2 = kPackA1 + 4 * 64 * 8;
 constexpr int kPackA3 = kPackA2 + 4 * 8 * 64 * 16;
-constexpr int kPackB2 = kPackA3 + 8 * 64 * 16;
+constexpr int kPackB2 = kPackA3 + 8 * 2 * 4 * 16;
 constexpr int kPackB3 = kPackB2 + kMlpH * 4;
-constexpr int kPackBytes = kPackB3 + 32 * 4;
+constexpr int kPackBytes = kPackB3 + 4 * 4;
 static_assert(kPackBytes % 16 == 0, "the blob is staged as uint4");
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
@@ -120,11 +121,10 @@ inline void mlp_pack_blob(const float* p, unsigned char* blob) {
                 }
     memcpy(blob + kPackB2, p + kOffB2, kMlpH * 4);
     for (int kc = 0; kc < 8; ++kc)
-        for (int lane = 0; lane < 64; ++lane)
-            for (int j = 0; j < 8; ++j) {
-                const int row = lane % 32, k = mlp_chunk_unit(kc, lane / 32, j);
-                put(kPackA3 + (kc * 64 + lane) * 16, j, row < kMlpOut ? W3[row * kMlpH + k] : 0.f);
-            }
+        for (int h = 0; h < 2; ++h)
+            for (int row = 0; row < kMlpOut; ++row)
+                for (int j = 0; j < 8; ++j)
+                    put(kPackA3 + ((kc * 2 + h) * 4 + row) * 16, j, W3[row * kMlpH + mlp_chunk_unit(kc, h, j)]);
     memcpy(blob + kPackB3, p + kOffB3, kMlpOut * 4);
 }
 
@@ -170,7 +170,8 @@ __device__ __forceinline__ void mlp_wave_core(const unsigned char* lds, bf16x4 X
     const int half = lane >> 5;  // 0: lanes 0-31, 1: lanes 32-63
     const bf16x4* A1 = reinterpret_cast<const bf16x4*>(lds + kPackA1);
     const bf16x8* A2 = reinterpret_cast<const bf16x8*>(lds + kPackA2);
-    const bf16x8* A3 = reinterpret_cast<const bf16x8*>(lds + kPackA3);
+    // this lane's row of layer 3; the rows past the outputs share the zero row
+    const bf16x8* A3 = reinterpret_cast<const bf16x8*>(lds + kPackA3) + half * 4 + min(lane & 31, kMlpOut);
     const float* b2 = reinterpret_cast<const float*>(lds + kPackB2);
     const float* b3 = reinterpret_cast<const float*>(lds + kPackB3);
     // Both 32-ion blocks go through each weight fragment together, so every
@@ -214,7 +215,7 @@ __device__ __forceinline__ void mlp_wave_core(const unsigned char* lds, bf16x4 X
         }
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
-            const bf16x8 a3 = A3[(2 * mb + q) * 64 + lane];
+            const bf16x8 a3 = A3[(2 * mb + q) * 8];
             y0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a3, relu_pack8(c0, 8 * q), y0, 0, 0, 0);
             y1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a3, relu_pack8(c1, 8 * q), y1, 0, 0, 0);
         }
@@ -237,7 +238,8 @@ __device__ __forceinline__ void mlp_block_core(const unsigned char* lds, bf16x4 
     const int half = lane >> 5;
     const bf16x4* A1 = reinterpret_cast<const bf16x4*>(lds + kPackA1);
     const bf16x8* A2 = reinterpret_cast<const bf16x8*>(lds + kPackA2);
-    const bf16x8* A3 = reinterpret_cast<const bf16x8*>(lds + kPackA3);
+    // this lane's row of layer 3; the rows past the outputs share the zero row
+    const bf16x8* A3 = reinterpret_cast<const bf16x8*>(lds + kPackA3) + half * 4 + min(lane & 31, kMlpOut);
     const float* b2 = reinterpret_cast<const float*>(lds + kPackB2);
     const float* b3 = reinterpret_cast<const float*>(lds + kPackB3);
     bf16x8 H[8];
@@ -265,7 +267,7 @@ __device__ __forceinline__ void mlp_block_core(const unsigned char* lds, bf16x4 
         for (int kc = 0; kc < 8; ++kc) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A2m[kc * 64], H[kc], c, 0, 0, 0);
 #pragma unroll
         for (int q = 0; q < 2; ++q)
-            y = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A3[(2 * mb + q) * 64 + lane], relu_pack8(c, 8 * q), y, 0, 0, 0);
+            y = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A3[(2 * mb + q) * 8], relu_pack8(c, 8 * q), y, 0, 0, 0);
     }
 #pragma unroll
     for (int c = 0; c < 3; ++c) r[c] = y[c] + b3[c];
@@ -321,11 +323,12 @@ __device__ __forceinline__ bool mlp_wave_eval_any(const unsigned char* lds, bool
 // the eight bf16 operand slots of layer 1 (x0..x5, 1, 0); the counts are
 // double-buffered by step parity, since a workgroup without any colliding ion
 // passes only one barrier per step.
+// The evaluating wavefront puts an ion's outputs in the slot it read the inputs
+// from, which no other wavefront touches in between.
 template <int WAVES>
 struct MlpExchange {
     static constexpr int kWaves = WAVES;
-    u32v4 in[64 * WAVES];
-    float out[kMlpOut][64 * WAVES];
+    u32v4 slot[64 * WAVES];
     uint32_t count[2][WAVES];
 };
 
@@ -365,7 +368,7 @@ __device__ __forceinline__ bool mlp_group_eval(const unsigned char* lds, MlpExch
         // copied with packed-float moves, which are disabled in this build)
         const uint64_t lo4 = __builtin_bit_cast(uint64_t, mlp_pack4(in[0], in[1], in[2], in[3]));
         const uint64_t hi4 = __builtin_bit_cast(uint64_t, mlp_pack4(in[4], in[5], 1.0f, 0.0f));
-        X.in[slot] = u32v4{static_cast<uint32_t>(lo4), static_cast<uint32_t>(lo4 >> 32),
+        X.slot[slot] = u32v4{static_cast<uint32_t>(lo4), static_cast<uint32_t>(lo4 >> 32),
                            static_cast<uint32_t>(hi4), static_cast<uint32_t>(hi4 >> 32)};
     }
     uint32_t* cnt = X.count[step & 1];
@@ -379,7 +382,7 @@ __device__ __forceinline__ bool mlp_group_eval(const unsigned char* lds, MlpExch
     const uint32_t total = start[WAVES];
     if (total == 0) return false;
     const uint32_t half = lane >> 5;
-    const uint32_t* xin = reinterpret_cast<const uint32_t*>(X.in);
+    const uint32_t* xin = reinterpret_cast<const uint32_t*>(X.slot);
     for (uint32_t b = (w + nw - rot % nw) % nw; 32 * b < total; b += nw) {
         // lanes l and l + 32 carry ion 32 b + l: operand slots 0-3 and 4-7.  Its
         // slot in the exchange: its wavefront is the number of wavefront starts
@@ -406,10 +409,8 @@ __device__ __forceinline__ bool mlp_group_eval(const unsigned char* lds, MlpExch
         __builtin_amdgcn_s_setprio(1);
         float r[3];
         mlp_block_core(lds, xb, r);
-        if (half == 0 && have) {
-#pragma unroll
-            for (int c = 0; c < kMlpOut; ++c) X.out[c][s] = r[c];
-        }
+        if (half == 0 && have)
+            X.slot[s] = u32v4{__float_as_uint(r[0]), __float_as_uint(r[1]), __float_as_uint(r[2]), 0u};
         __builtin_amdgcn_s_setprio(0);
         // a compiler memory fence: a second block reloads the weight fragments
         // from LDS instead of keeping the first block's 128 registers of them
@@ -417,8 +418,9 @@ __device__ __forceinline__ bool mlp_group_eval(const unsigned char* lds, MlpExch
     }
     __syncthreads();
     if (coll) {
+        const u32v4 r = X.slot[slot];
 #pragma unroll
-        for (int c = 0; c < kMlpOut; ++c) out[c] = X.out[c][slot];
+        for (int c = 0; c < kMlpOut; ++c) out[c] = __uint_as_float(r[c]);
     }
     return true;
 }

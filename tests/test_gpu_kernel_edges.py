@@ -120,3 +120,43 @@ def test_fp64_lanes_per_ion(oracle, n, integrator, kind):
     assert np.array_equal(g.born, o.born) and np.array_equal(g.n_collisions, o.n_collisions)
     np.testing.assert_allclose(g.death_time_s, o.death_time_s, rtol=1e-12)
     np.testing.assert_allclose(g.arrival_time_s, o.arrival_time_s, rtol=1e-9)
+
+
+@pytest.mark.parametrize("n", [1, 5, 4097, 131072, 131073])
+def test_surrogate_launch_shapes(n):
+    """An ion's run depends on its index and the seed alone: the first ions of a
+    cloud, stepped in clouds of other sizes (other ions per wavefront, the other
+    instantiation), take the same course.  FP32: the instantiations round alike
+    to some ulps, and one collision test in some 1e7 may turn out otherwise."""
+    from icarion_amd import gpu
+    import icarion_amd
+    m = min(n, 1000)
+    w = W.ehss_surrogate_workload(n=1, seed=3)
+    w["domain"].detector_z_m = 1e-5
+    params = np.load(icarion_amd.__path__[0] + "/data/surrogate_he_20td_clusters.npy")
+    counts = W.ehss_cluster_counts(40, 3)
+    rng = np.random.default_rng(9)
+    full = W.gaussian_cloud(131073, 1500.0, 0.5e-3, seed=3)
+    full.species[:] = rng.integers(0, 40, full.n)
+    full.birth_time_s = np.where(rng.random(full.n) < 0.3, rng.uniform(0.0, 60.0, full.n) * w["dt"], 0.0)
+    full.born[:] = full.active[:] = full.birth_time_s == 0.0
+    out = []
+    for size in (n, 2001):
+        e = full.subset(np.arange(size))
+        with gpu.Handle(device=0) as h:
+            h.set_domain(w["domain"], w["physics"])
+            h.synth_clusters(counts, seed=3)
+            h.surrogate_set_params(params)
+            h.upload_state(e)
+            st = h.step(0.0, w["dt"], 50)
+            h.download_state(e)
+        born = e.born != 0
+        assert st.ion_steps == np.where(e.birth_time_s == 0.0, 50, 50 - np.ceil(e.birth_time_s / w["dt"]))[born].sum()
+        assert st.collisions == e.n_collisions.sum()
+        out.append(e.subset(np.arange(m)))
+    a, b = out
+    assert np.array_equal(a.active, b.active) and np.array_equal(a.born, b.born)
+    same = a.n_collisions == b.n_collisions
+    for f, scale in (("x", 1e-6), ("z", 1e-6), ("vx", 1.0), ("vz", 1.0)):
+        same &= np.abs(getattr(a, f) - getattr(b, f)) <= 1e-5 * np.maximum(np.abs(getattr(b, f)), scale)
+    assert same.mean() >= 0.998
