@@ -135,21 +135,35 @@ int guarded(F&& f) {
     }
 }
 
+// Device memory of its own (freed with it), or a view into another buffer.
 template <class T>
 struct DevBuf {
     T* p = nullptr;
     size_t n = 0;
+    bool owned = true;
+    DevBuf() = default;
+    DevBuf(const DevBuf&) = delete;
+    DevBuf& operator=(const DevBuf&) = delete;
+    DevBuf(DevBuf&& o) noexcept : p(o.p), n(o.n), owned(o.owned) { o.p = nullptr; o.n = 0; }
+    ~DevBuf() { release(); }
     void resize(size_t count) {
-        if (count == n && p) return;
+        if (count == n && p && owned) return;
         release();
         if (count == 0) return;
         hip_check(hipMalloc(reinterpret_cast<void**>(&p), count * sizeof(T)), "hipMalloc");
         n = count;
     }
+    void view(void* at, size_t count) {
+        release();
+        p = static_cast<T*>(at);
+        n = count;
+        owned = false;
+    }
     void release() {
-        if (p) (void)hipFree(p);
+        if (p && owned) (void)hipFree(p);
         p = nullptr;
         n = 0;
+        owned = true;
     }
 };
 
@@ -163,6 +177,46 @@ template <class T>
 void copy_out(T* dst, const DevBuf<T>& b, size_t n, hipStream_t s, const char* what) {
     if (dst && n) hip_check(hipMemcpyAsync(dst, b.p, n * sizeof(T), hipMemcpyDeviceToHost, s), what);
 }
+
+// The per-ion arrays of a cloud (or of all clouds of a batch) in one device
+// allocation, and host memory of the same layout, so that a small state crosses
+// in one copy each way: the arrays a run changes first, then the read-only ones.
+enum SlabArray { kX, kY, kZ, kVx, kVy, kVz, kDeath, kArrival, kTime, kDt, kNcoll, kFlags, kMass, kCharge, kSpec, kBirth,
+                 kSlabArrays };
+struct StateSlab {
+    DevBuf<unsigned char> dev;
+    std::unique_ptr<unsigned char[]> host;
+    size_t host_cap = 0;
+    size_t off[kSlabArrays + 1] = {};
+
+    // rk45: with ion times and steps
+    void layout(size_t n, bool rk45, bool birth) {
+        size_t at = 0;
+        for (int k = 0; k < kSlabArrays; ++k) {
+            off[k] = at;
+            size_t width = 8;
+            if (k == kNcoll || k == kSpec) width = 4;
+            if (k == kFlags) width = 1;
+            if (((k == kTime || k == kDt) && !rk45) || (k == kBirth && !birth)) width = 0;
+            at += (width * n + 255) / 256 * 256;
+        }
+        off[kSlabArrays] = at;
+        if (dev.n < at) dev.resize(at);
+        if (host_cap < at) {
+            host.reset(new unsigned char[at]);   // pages are touched only where they are used
+            host_cap = at;
+        }
+    }
+    size_t changed_bytes() const { return off[kMass]; }
+    size_t bytes() const { return off[kSlabArrays]; }
+    template <class T>
+    T* at(SlabArray k) const { return reinterpret_cast<T*>(host.get() + off[k]); }
+    unsigned char* dev_at(SlabArray k) const { return dev.p + off[k]; }
+};
+// Up to this many ions a state is gathered in the slab's host memory and crosses
+// in one copy (a copy's own cost is 5-10 us); larger arrays cross one by one,
+// straight from and to the caller's memory.
+constexpr size_t kSlabOneCopyIons = 32768;
 
 constexpr double kPiHost = 3.14159265358979323846;
 constexpr double kBoltzmannHost = 1.380649e-23;
@@ -289,6 +343,8 @@ struct icarion_gpu {
 
     size_t n = 0;
     bool have_state = false;
+    StateSlab slab;              // the arrays below are views into it
+    bool rk45_fresh = true;      // RK45 step-control memory not yet set for this state
     DevBuf<double> x, y, z, vx, vy, vz, mass, charge, birth, death, arrival;
     DevBuf<uint32_t> spec, ncoll;
     DevBuf<uint8_t> flags;
@@ -322,6 +378,7 @@ struct icarion_gpu {
     };
     uint32_t b_n = 0;
     size_t b_total = 0;
+    StateSlab b_slab;            // the batch's per-ion arrays
     std::vector<BatchCloud> b_clouds;
     std::vector<StepParams> b_params;
     DevBuf<StepParams> b_params_d;
@@ -876,14 +933,16 @@ __global__ void __launch_bounds__(256) count_state_kernel(const uint8_t* __restr
 }
 
 // Sum of the stripes: word w of every stripe into out[w] (w = 0..3), written
-// straight to mapped pinned host memory.
-__global__ void fold_counters_kernel(const unsigned long long* counters, int stripes, unsigned long long* out) {
-    const int w = threadIdx.x;
-    if (w < 4) {
-        unsigned long long a = 0;
-        for (int k = 0; k < stripes; ++k) a += counters[k * kCounterStride + w];
-        out[w] = a;
-    }
+// straight to mapped pinned host memory.  One wavefront per word, a stripe per
+// lane.
+static_assert(kCounterStripes == 64, "a stripe per lane");
+__global__ void __launch_bounds__(256) fold_counters_kernel(const unsigned long long* counters,
+                                                            unsigned long long* out) {
+    const int w = threadIdx.x >> 6;
+    unsigned long long a = counters[(threadIdx.x & 63) * kCounterStride + w];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off, 64);
+    if ((threadIdx.x & 63) == 0) out[w] = a;
 }
 
 // Counters of the call: ion-steps and collisions of its launches, and the
@@ -901,8 +960,7 @@ CallCounts read_counters(icarion_gpu* h, hipStream_t s, bool with_state, unsigne
                            counters, kCounterStripes);
         hip_check(hipGetLastError(), "count state launch");
     }
-    hipLaunchKernelGGL(fold_counters_kernel, dim3(1), dim3(64), 0, s, counters, kCounterStripes,
-                       h->host_ctr_dev);
+    hipLaunchKernelGGL(fold_counters_kernel, dim3(1), dim3(256), 0, s, counters, h->host_ctr_dev);
     hip_check(hipGetLastError(), "fold counters launch");
     hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
     CallCounts c;
@@ -990,6 +1048,14 @@ void upload_rk45_waves(icarion_gpu* h, StepParams& P, bool voltages) {
 
 // The RK45 engine loop: one launch pair (step kernel + engine-time advance) per
 // engine step, replayed from a captured HIP graph of up to 32 steps.
+__global__ void rk45_fresh_kernel(double* err, double* k1x, double* k1y, double* k1z, uint8_t* fsal, uint32_t n) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    err[i] = 1.0;
+    k1x[i] = k1y[i] = k1z[i] = 0.0;
+    fsal[i] = 0;
+}
+
 void do_step_rk45(icarion_gpu* h, double t0, double dt, uint64_t n_steps, uint64_t step_offset,
                   icarion_step_stats* stats) {
     const int field = launch_field_kind(h);
@@ -1026,6 +1092,18 @@ void do_step_rk45(icarion_gpu* h, double t0, double dt, uint64_t n_steps, uint64
     fill_fast_const(P);
     const IonPtrs S = ion_ptrs(h);
     h->r_eng.resize(1);
+    if (h->rk45_fresh) {
+        // fresh step-control memory (RK45Strategy.h:192-198)
+        h->r_err.resize(h->n); h->r_k1x.resize(h->n); h->r_k1y.resize(h->n); h->r_k1z.resize(h->n);
+        h->r_fsal.resize(h->n);
+        if (h->n) {
+            hipLaunchKernelGGL(rk45_fresh_kernel, dim3(static_cast<uint32_t>((h->n + 255) / 256)), dim3(256), 0,
+                               h->stream, h->r_err.p, h->r_k1x.p, h->r_k1y.p, h->r_k1z.p, h->r_fsal.p,
+                               static_cast<uint32_t>(h->n));
+            hip_check(hipGetLastError(), "RK45 state");
+        }
+        h->rk45_fresh = false;
+    }
     Rk45Ptrs R{h->r_t.p, h->r_dt.p, h->r_err.p, h->r_k1x.p, h->r_k1y.p, h->r_k1z.p, h->r_fsal.p, h->r_eng.p};
     Rk45Engine e0{t0, dt, step_offset, 0ull, ~0ull, 0ull, 0ull, 0ull};
     hip_check(hipMemcpyAsync(h->r_eng.p, &e0, sizeof(e0), hipMemcpyHostToDevice, s), "upload engine record");
@@ -1705,7 +1783,14 @@ void do_step_multi(icarion_gpu* h, double t0, double dt, uint64_t n_steps, uint6
     finish_stats(h, t_end, ms, stats, h->counters.p);
 }
 
-void do_upload(icarion_gpu* h, const icarion_ion_soa* ions) {
+__global__ void zero_u32_array(uint32_t* p, size_t n) {
+    for (size_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += static_cast<size_t>(gridDim.x) * blockDim.x)
+        p[i] = 0u;
+}
+
+// sync = false: the caller waits for the stream before it returns to its own
+// caller (whose arrays may be in flight until then).
+void do_upload(icarion_gpu* h, const icarion_ion_soa* ions, bool sync = true) {
     if (!ions) fail(ICARION_ERR_INVALID, "ions is NULL");
     if (!h->have_species) fail(ICARION_ERR_STATE, "icarion_gpu_set_species must precede upload_state");
     const size_t n = ions->n;
@@ -1713,57 +1798,73 @@ void do_upload(icarion_gpu* h, const icarion_ion_soa* ions) {
     if (n && (!ions->x || !ions->y || !ions->z || !ions->vx || !ions->vy || !ions->vz ||
               !ions->mass_kg || !ions->charge_C || !ions->species || !ions->active))
         fail(ICARION_ERR_INVALID, "x, y, z, vx, vy, vz, mass_kg, charge_C, species, active are required");
-    uint32_t used = 0;
+    uint32_t top = 0;
+    bool massive = true;
     for (size_t i = 0; i < n; ++i) {
-        if (ions->species[i] >= h->n_species)
-            fail(ICARION_ERR_INVALID, "species index " + std::to_string(ions->species[i]) +
-                                          " of ion " + std::to_string(i) + " out of range");
-        if (!(ions->mass_kg[i] > 0.0))
-            fail(ICARION_ERR_INVALID, "mass_kg of ion " + std::to_string(i) + " must be > 0");
-        used = std::max(used, ions->species[i] + 1);
+        top = std::max(top, ions->species[i]);
+        massive &= ions->mass_kg[i] > 0.0;
     }
-    h->species_used = used;
+    if (n && (top >= h->n_species || !massive))
+        for (size_t i = 0; i < n; ++i) {
+            if (ions->species[i] >= h->n_species)
+                fail(ICARION_ERR_INVALID, "species index " + std::to_string(ions->species[i]) +
+                                              " of ion " + std::to_string(i) + " out of range");
+            if (!(ions->mass_kg[i] > 0.0))
+                fail(ICARION_ERR_INVALID, "mass_kg of ion " + std::to_string(i) + " must be > 0");
+        }
+    h->species_used = n ? top + 1 : 0;
     set_device(h);
     hipStream_t s = h->stream;
-    copy_in(h->x, ions->x, n, s, "upload x");
-    copy_in(h->y, ions->y, n, s, "upload y");
-    copy_in(h->z, ions->z, n, s, "upload z");
-    copy_in(h->vx, ions->vx, n, s, "upload vx");
-    copy_in(h->vy, ions->vy, n, s, "upload vy");
-    copy_in(h->vz, ions->vz, n, s, "upload vz");
-    copy_in(h->mass, ions->mass_kg, n, s, "upload mass");
-    copy_in(h->charge, ions->charge_C, n, s, "upload charge");
-    copy_in(h->spec, ions->species, n, s, "upload species");
-    std::vector<uint8_t> fl(n);
+    h->has_birth = ions->birth_time_s != nullptr;
+    StateSlab& L = h->slab;
+    h->have_state = false;   // until the new state is in place
+    L.layout(n, true, h->has_birth);
+    h->x.view(L.dev_at(kX), n); h->y.view(L.dev_at(kY), n); h->z.view(L.dev_at(kZ), n);
+    h->vx.view(L.dev_at(kVx), n); h->vy.view(L.dev_at(kVy), n); h->vz.view(L.dev_at(kVz), n);
+    h->death.view(L.dev_at(kDeath), n); h->arrival.view(L.dev_at(kArrival), n);
+    h->r_t.view(L.dev_at(kTime), n); h->r_dt.view(L.dev_at(kDt), n);
+    h->ncoll.view(L.dev_at(kNcoll), n); h->flags.view(L.dev_at(kFlags), n);
+    h->mass.view(L.dev_at(kMass), n); h->charge.view(L.dev_at(kCharge), n); h->spec.view(L.dev_at(kSpec), n);
+    h->birth.view(L.dev_at(kBirth), h->has_birth ? n : 0);
+    const bool one_copy = n <= kSlabOneCopyIons;
+    // an array of the caller's, or its default value
+    auto put = [&](SlabArray k, const auto* src, auto fallback) {
+        using T = decltype(fallback);
+        if (k == kBirth && !src) return;
+        if (!src) std::fill_n(L.at<T>(k), n, fallback);
+        else if (one_copy) std::memcpy(L.at<T>(k), src, n * sizeof(T));
+        if (!one_copy && n)
+            hip_check(hipMemcpyAsync(L.dev_at(k), src ? src : L.at<T>(k), n * sizeof(T), hipMemcpyHostToDevice, s),
+                      "upload state");
+    };
+    put(kX, ions->x, 0.0); put(kY, ions->y, 0.0); put(kZ, ions->z, 0.0);
+    put(kVx, ions->vx, 0.0); put(kVy, ions->vy, 0.0); put(kVz, ions->vz, 0.0);
+    put(kDeath, ions->death_time_s, -1.0);
+    put(kArrival, ions->arrival_time_s, static_cast<double>(NAN));
+    // RK45 state: ion time / dt from the caller (NaN / <= 0 = set by the first
+    // step); its step-control memory is set by the first RK45 step
+    put(kTime, ions->time_s, static_cast<double>(NAN));
+    put(kDt, ions->dt_s, 0.0);
+    put(kNcoll, ions->n_collisions, 0u);
+    put(kMass, ions->mass_kg, 0.0); put(kCharge, ions->charge_C, 0.0); put(kSpec, ions->species, 0u);
+    put(kBirth, ions->birth_time_s, 0.0);
+    uint8_t* const fl = L.at<uint8_t>(kFlags);
     for (size_t i = 0; i < n; ++i)
         fl[i] = static_cast<uint8_t>((ions->active[i] ? 1 : 0) | ((ions->born ? ions->born[i] : 1) ? 2 : 0));
-    copy_in(h->flags, fl.data(), n, s, "upload flags");
-    h->has_birth = ions->birth_time_s != nullptr;
-    if (h->has_birth) copy_in(h->birth, ions->birth_time_s, n, s, "upload birth");
-    // host staging buffers stay alive until the stream synchronisation below
-    std::vector<double> dead(ions->death_time_s ? 0 : n, -1.0);
-    std::vector<double> arr(ions->arrival_time_s ? 0 : n, NAN);
-    copy_in(h->death, ions->death_time_s ? ions->death_time_s : dead.data(), n, s, "upload death");
-    copy_in(h->arrival, ions->arrival_time_s ? ions->arrival_time_s : arr.data(), n, s, "upload arrival");
-    std::vector<uint32_t> nc(n, 0);
-    copy_in(h->ncoll, ions->n_collisions ? ions->n_collisions : nc.data(), n, s, "upload ncoll");
-    // RK45 state: ion time / dt from the caller (NaN / <= 0 = set by the first
-    // step), fresh step-control memory (RK45Strategy.h:192-198)
-    std::vector<double> tt(ions->time_s ? 0 : n, NAN), dd(ions->dt_s ? 0 : n, 0.0);
-    std::vector<double> ones(n, 1.0), zeros(n, 0.0);
-    std::vector<uint8_t> nofsal(n, 0);
-    copy_in(h->r_t, ions->time_s ? ions->time_s : tt.data(), n, s, "upload time");
-    copy_in(h->r_dt, ions->dt_s ? ions->dt_s : dd.data(), n, s, "upload dt");
-    copy_in(h->r_err, ones.data(), n, s, "upload rk45 error");
-    copy_in(h->r_k1x, zeros.data(), n, s, "upload rk45 k1");
-    copy_in(h->r_k1y, zeros.data(), n, s, "upload rk45 k1");
-    copy_in(h->r_k1z, zeros.data(), n, s, "upload rk45 k1");
-    copy_in(h->r_fsal, nofsal.data(), n, s, "upload rk45 fsal");
+    if (n)
+        hip_check(one_copy ? hipMemcpyAsync(L.dev.p, L.host.get(), L.bytes(), hipMemcpyHostToDevice, s)
+                           : hipMemcpyAsync(L.dev_at(kFlags), fl, n, hipMemcpyHostToDevice, s),
+                  "upload state");
+    h->rk45_fresh = true;
     // domain index before the first step: 0, IonState's default (IonState.h:48);
     // several domains set it at each step start
-    std::vector<int32_t> dom0(n, 0);
-    copy_in(h->ion_dom, dom0.data(), n, s, "upload domain index");
-    hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
+    h->ion_dom.resize(n);
+    if (n) {
+        hipLaunchKernelGGL(zero_u32_array, dim3(std::min<uint32_t>(1024, static_cast<uint32_t>((n + 255) / 256))),
+                           dim3(256), 0, s, reinterpret_cast<uint32_t*>(h->ion_dom.p), n);
+        hip_check(hipGetLastError(), "reset domain index");
+    }
+    if (sync) hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
     h->n = n;
     h->have_state = true;
 }
@@ -1774,21 +1875,30 @@ void do_download(icarion_gpu* h, icarion_ion_soa* ions) {
     if (ions->n != h->n) fail(ICARION_ERR_INVALID, "ions->n differs from the resident ensemble size");
     set_device(h);
     const size_t n = h->n;
+    if (n == 0) return;
     hipStream_t s = h->stream;
-    copy_out(ions->x, h->x, n, s, "download x");
-    copy_out(ions->y, h->y, n, s, "download y");
-    copy_out(ions->z, h->z, n, s, "download z");
-    copy_out(ions->vx, h->vx, n, s, "download vx");
-    copy_out(ions->vy, h->vy, n, s, "download vy");
-    copy_out(ions->vz, h->vz, n, s, "download vz");
-    copy_out(ions->death_time_s, h->death, n, s, "download death");
-    copy_out(ions->arrival_time_s, h->arrival, n, s, "download arrival");
-    copy_out(ions->n_collisions, h->ncoll, n, s, "download ncoll");
-    copy_out(ions->time_s, h->r_t, n, s, "download time");
-    copy_out(ions->dt_s, h->r_dt, n, s, "download dt");
-    std::vector<uint8_t> fl(n);
-    copy_out(fl.data(), h->flags, n, s, "download flags");
-    hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
+    StateSlab& L = h->slab;
+    const bool one_copy = n <= kSlabOneCopyIons;
+    if (one_copy) {
+        hip_check(hipMemcpyAsync(L.host.get(), L.dev.p, L.changed_bytes(), hipMemcpyDeviceToHost, s), "download state");
+        hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
+    }
+    auto get = [&](SlabArray k, auto* dst) {
+        using T = std::remove_pointer_t<decltype(dst)>;
+        if (!dst) return;
+        if (one_copy) std::memcpy(dst, L.at<T>(k), n * sizeof(T));
+        else hip_check(hipMemcpyAsync(dst, L.dev_at(k), n * sizeof(T), hipMemcpyDeviceToHost, s), "download state");
+    };
+    get(kX, ions->x); get(kY, ions->y); get(kZ, ions->z);
+    get(kVx, ions->vx); get(kVy, ions->vy); get(kVz, ions->vz);
+    get(kDeath, ions->death_time_s); get(kArrival, ions->arrival_time_s);
+    get(kNcoll, ions->n_collisions);
+    get(kTime, ions->time_s); get(kDt, ions->dt_s);
+    uint8_t* const fl = L.at<uint8_t>(kFlags);
+    if (!one_copy) {
+        get(kFlags, fl);
+        hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
+    }
     for (size_t i = 0; i < n; ++i) {
         if (ions->active) ions->active[i] = fl[i] & 1;
         if (ions->born) ions->born[i] = (fl[i] >> 1) & 1;
@@ -2011,35 +2121,40 @@ void do_batch_upload(icarion_gpu* h, const icarion_cloud_desc* clouds, uint32_t 
     if (total > 0xFFFFFFFFull) fail(ICARION_ERR_INVALID, "at most 2^32-1 ions per batch");
     set_device(h);
     hipStream_t s = h->stream;
-    // concatenated SoA; host staging lives until the synchronisation below
-    std::vector<double> hx(total), hy(total), hz(total), hvx(total), hvy(total), hvz(total), hm(total),
-        hq(total), hb(total, -INFINITY), hd(total, -1.0), ha(total, NAN);
-    std::vector<uint32_t> hs(total), hn(total, 0);
-    std::vector<uint8_t> hf(total);
+    // the clouds' arrays one after another in the slab, across in one copy
+    const size_t nt = std::max<size_t>(total, 1);
+    StateSlab& L = h->b_slab;
+    h->b_n = 0;   // until the new batch is in place
+    L.layout(nt, false, true);
     for (uint32_t c = 0; c < n_clouds; ++c) {
         const icarion_ion_soa* io = clouds[c].ions;
-        const size_t o = bc[c].off;
-        for (size_t i = 0; i < bc[c].n; ++i) {
-            hx[o + i] = io->x[i]; hy[o + i] = io->y[i]; hz[o + i] = io->z[i];
-            hvx[o + i] = io->vx[i]; hvy[o + i] = io->vy[i]; hvz[o + i] = io->vz[i];
-            hm[o + i] = io->mass_kg[i]; hq[o + i] = io->charge_C[i];
-            hs[o + i] = io->species[i];
-            hf[o + i] = static_cast<uint8_t>((io->active[i] ? 1 : 0) | ((io->born ? io->born[i] : 1) ? 2 : 0));
-            if (io->birth_time_s) hb[o + i] = io->birth_time_s[i];
-            if (io->death_time_s) hd[o + i] = io->death_time_s[i];
-            if (io->arrival_time_s) ha[o + i] = io->arrival_time_s[i];
-            if (io->n_collisions) hn[o + i] = io->n_collisions[i];
-        }
+        const size_t o = bc[c].off, n = bc[c].n;
+        auto put = [&](SlabArray k, const auto* src, auto fallback) {
+            using T = decltype(fallback);
+            if (src) std::memcpy(L.at<T>(k) + o, src, n * sizeof(T));
+            else std::fill_n(L.at<T>(k) + o, n, fallback);
+        };
+        put(kX, io->x, 0.0); put(kY, io->y, 0.0); put(kZ, io->z, 0.0);
+        put(kVx, io->vx, 0.0); put(kVy, io->vy, 0.0); put(kVz, io->vz, 0.0);
+        put(kMass, io->mass_kg, 0.0); put(kCharge, io->charge_C, 0.0); put(kSpec, io->species, 0u);
+        if (io->birth_time_s) put(kBirth, io->birth_time_s, 0.0);   // else never read
+        put(kDeath, io->death_time_s, -1.0);
+        put(kArrival, io->arrival_time_s, static_cast<double>(NAN));
+        put(kNcoll, io->n_collisions, 0u);
+        uint8_t* const fl = L.at<uint8_t>(kFlags) + o;
+        for (size_t i = 0; i < n; ++i)
+            fl[i] = static_cast<uint8_t>((io->active[i] ? 1 : 0) | ((io->born ? io->born[i] : 1) ? 2 : 0));
     }
-    const size_t nt = std::max<size_t>(total, 1);
-    h->b_x.resize(nt); h->b_y.resize(nt); h->b_z.resize(nt);
-    copy_in(h->b_x, hx.data(), total, s, "batch x"); copy_in(h->b_y, hy.data(), total, s, "batch y");
-    copy_in(h->b_z, hz.data(), total, s, "batch z"); copy_in(h->b_vx, hvx.data(), total, s, "batch vx");
-    copy_in(h->b_vy, hvy.data(), total, s, "batch vy"); copy_in(h->b_vz, hvz.data(), total, s, "batch vz");
-    copy_in(h->b_mass, hm.data(), total, s, "batch mass"); copy_in(h->b_charge, hq.data(), total, s, "batch charge");
-    copy_in(h->b_birth, hb.data(), total, s, "batch birth"); copy_in(h->b_death, hd.data(), total, s, "batch death");
-    copy_in(h->b_arrival, ha.data(), total, s, "batch arrival"); copy_in(h->b_spec, hs.data(), total, s, "batch species");
-    copy_in(h->b_ncoll, hn.data(), total, s, "batch ncoll"); copy_in(h->b_flags, hf.data(), total, s, "batch flags");
+    bool births = false;
+    for (const auto& x : bc) births |= x.has_birth;
+    hip_check(hipMemcpyAsync(L.dev.p, L.host.get(), births ? L.bytes() : L.off[kBirth], hipMemcpyHostToDevice, s),
+              "batch state");
+    h->b_x.view(L.dev_at(kX), nt); h->b_y.view(L.dev_at(kY), nt); h->b_z.view(L.dev_at(kZ), nt);
+    h->b_vx.view(L.dev_at(kVx), nt); h->b_vy.view(L.dev_at(kVy), nt); h->b_vz.view(L.dev_at(kVz), nt);
+    h->b_mass.view(L.dev_at(kMass), nt); h->b_charge.view(L.dev_at(kCharge), nt);
+    h->b_birth.view(L.dev_at(kBirth), nt); h->b_death.view(L.dev_at(kDeath), nt);
+    h->b_arrival.view(L.dev_at(kArrival), nt); h->b_spec.view(L.dev_at(kSpec), nt);
+    h->b_ncoll.view(L.dev_at(kNcoll), nt); h->b_flags.view(L.dev_at(kFlags), nt);
     copy_in(h->b_species, species.data(), species.size(), s, "batch species table");
     copy_in(h->b_tables, tables.data(), std::max<size_t>(tables.size(), 1), s, "batch step tables");
     h->b_atoms.resize(std::max<size_t>(atoms_all.size(), 1));
@@ -2175,6 +2290,33 @@ float batch_launch(icarion_gpu* h, icarion_batch_tuning t64, icarion_batch_tunin
     return ms;
 }
 
+// Alive and arrived ions of each cloud into words 2 and 3 of its counters (one
+// workgroup per cloud).
+__global__ void __launch_bounds__(256) count_clouds_kernel(const StepParams* params, const IonPtrs* ions,
+                                                           unsigned long long* counters) {
+    __shared__ uint32_t sum[2][4];
+    const uint32_t n = params[blockIdx.x].n_ions;
+    const IonPtrs S = ions[blockIdx.x];
+    uint32_t alive = 0, arrived = 0;
+    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
+        alive += (S.flags[i] & 3u) == 3u;
+        arrived += S.arrival[i] == S.arrival[i];
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        alive += __shfl_xor(alive, off, 64);
+        arrived += __shfl_xor(arrived, off, 64);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        sum[0][threadIdx.x >> 6] = alive;
+        sum[1][threadIdx.x >> 6] = arrived;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2)
+        counters[4ull * blockIdx.x + 2 + threadIdx.x] = static_cast<unsigned long long>(sum[threadIdx.x][0]) +
+            sum[threadIdx.x][1] + sum[threadIdx.x][2] + sum[threadIdx.x][3];
+}
+
 void do_batch_run(icarion_gpu* h, const icarion_batch_tuning* r64, const icarion_batch_tuning* r32,
                   icarion_cloud_stats* per_cloud, double* device_ms) {
     if (h->b_n == 0) fail(ICARION_ERR_STATE, "icarion_gpu_batch_upload not called");
@@ -2185,14 +2327,12 @@ void do_batch_run(icarion_gpu* h, const icarion_batch_tuning* r64, const icarion
     if (!per_cloud) return;
     const uint32_t n = h->b_n;
     std::vector<unsigned long long> cnt(4ull * n), done(n), start(1);
-    std::vector<uint8_t> fl(h->b_total);
-    std::vector<double> ar(h->b_total);
     hipStream_t s = h->stream;
+    hipLaunchKernelGGL(count_clouds_kernel, dim3(n), dim3(256), 0, s, h->b_params_d.p, h->b_ions_d.p, h->b_counters.p);
+    hip_check(hipGetLastError(), "batch counts");
     copy_out(cnt.data(), h->b_counters, cnt.size(), s, "batch counters");
     copy_out(done.data(), h->b_done, n, s, "batch completion clocks");
     copy_out(start.data(), h->b_start, 1, s, "batch start clock");
-    copy_out(fl.data(), h->b_flags, h->b_total, s, "batch flags");
-    copy_out(ar.data(), h->b_arrival, h->b_total, s, "batch arrival");
     hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
     const double tick_ms = h->clock_khz > 0 ? 1.0 / static_cast<double>(h->clock_khz) : 0.0;
     for (uint32_t c = 0; c < n; ++c) {
@@ -2200,13 +2340,8 @@ void do_batch_run(icarion_gpu* h, const icarion_batch_tuning* r64, const icarion
         icarion_cloud_stats& st = per_cloud[c];
         st.ion_steps = cnt[4ull * c];
         st.collisions = cnt[4ull * c + 1];
-        uint64_t alive = 0, arrived = 0;
-        for (size_t i = bc.off; i < bc.off + bc.n; ++i) {
-            if ((fl[i] & 3) == 3) ++alive;
-            if (!std::isnan(ar[i])) ++arrived;
-        }
-        st.alive = alive;
-        st.arrived = arrived;
+        st.alive = cnt[4ull * c + 2];
+        st.arrived = cnt[4ull * c + 3];
         st.t_end_s = bc.t_end;
         st.done_ms = (done[c] && start[0] != ~0ull && done[c] >= start[0])
                          ? static_cast<double>(done[c] - start[0]) * tick_ms : 0.0;
@@ -2283,32 +2418,24 @@ void do_batch_download(icarion_gpu* h, const icarion_cloud_desc* clouds, uint32_
     set_device(h);
     hipStream_t s = h->stream;
     const size_t n = h->b_total;
-    std::vector<double> hx(n), hy(n), hz(n), hvx(n), hvy(n), hvz(n), hd(n), ha(n);
-    std::vector<uint32_t> hn(n);
-    std::vector<uint8_t> hf(n);
-    copy_out(hx.data(), h->b_x, n, s, "batch x"); copy_out(hy.data(), h->b_y, n, s, "batch y");
-    copy_out(hz.data(), h->b_z, n, s, "batch z"); copy_out(hvx.data(), h->b_vx, n, s, "batch vx");
-    copy_out(hvy.data(), h->b_vy, n, s, "batch vy"); copy_out(hvz.data(), h->b_vz, n, s, "batch vz");
-    copy_out(hd.data(), h->b_death, n, s, "batch death"); copy_out(ha.data(), h->b_arrival, n, s, "batch arrival");
-    copy_out(hn.data(), h->b_ncoll, n, s, "batch ncoll"); copy_out(hf.data(), h->b_flags, n, s, "batch flags");
+    StateSlab& L = h->b_slab;
+    if (n) hip_check(hipMemcpyAsync(L.host.get(), L.dev.p, L.changed_bytes(), hipMemcpyDeviceToHost, s), "batch state");
     hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
     for (uint32_t c = 0; c < n_clouds; ++c) {
         icarion_ion_soa* io = clouds[c].ions;
         const auto& bc = h->b_clouds[c];
         if (!io || io->n != bc.n) fail(ICARION_ERR_INVALID, "cloud " + std::to_string(c) + ": ions->n differs");
-        const size_t o = bc.off;
+        auto get = [&](SlabArray k, auto* dst) {
+            using T = std::remove_pointer_t<decltype(dst)>;
+            if (dst) std::memcpy(dst, L.at<T>(k) + bc.off, bc.n * sizeof(T));
+        };
+        get(kX, io->x); get(kY, io->y); get(kZ, io->z);
+        get(kVx, io->vx); get(kVy, io->vy); get(kVz, io->vz);
+        get(kDeath, io->death_time_s); get(kArrival, io->arrival_time_s); get(kNcoll, io->n_collisions);
+        const uint8_t* const fl = L.at<uint8_t>(kFlags) + bc.off;
         for (size_t i = 0; i < bc.n; ++i) {
-            if (io->x) io->x[i] = hx[o + i];
-            if (io->y) io->y[i] = hy[o + i];
-            if (io->z) io->z[i] = hz[o + i];
-            if (io->vx) io->vx[i] = hvx[o + i];
-            if (io->vy) io->vy[i] = hvy[o + i];
-            if (io->vz) io->vz[i] = hvz[o + i];
-            if (io->death_time_s) io->death_time_s[i] = hd[o + i];
-            if (io->arrival_time_s) io->arrival_time_s[i] = ha[o + i];
-            if (io->n_collisions) io->n_collisions[i] = hn[o + i];
-            if (io->active) io->active[i] = hf[o + i] & 1;
-            if (io->born) io->born[i] = (hf[o + i] >> 1) & 1;
+            if (io->active) io->active[i] = fl[i] & 1;
+            if (io->born) io->born[i] = (fl[i] >> 1) & 1;
         }
     }
 }
@@ -3537,9 +3664,14 @@ int icarion_gpu_step_batch(icarion_gpu* h, icarion_ion_soa* ions, double t, doub
                            uint64_t step_index, icarion_step_stats* stats) {
     return guarded([&] {
         if (!h) fail(ICARION_ERR_INVALID, "NULL handle");
-        do_upload(h, ions);
-        do_step(h, t, dt, 1, step_index, stats);
-        do_download(h, ions);
+        try {
+            do_upload(h, ions, false);
+            do_step(h, t, dt, 1, step_index, stats);
+            do_download(h, ions);
+        } catch (...) {
+            (void)hipStreamSynchronize(h->stream);   // the caller's arrays may still be in flight
+            throw;
+        }
     });
 }
 
