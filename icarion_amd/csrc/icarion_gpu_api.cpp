@@ -902,6 +902,10 @@ constexpr int kCounterWords = kCounterStripes * kCounterStride;
 // Field-array clouds of at least this many ions run in grid-brick order.
 constexpr size_t kOrderMinIons = 65536;
 
+// Single-cloud runs of at least this many ions drop lost ions' lanes between
+// launches (a launch of 2000 steps is then 2 ms and more, the count 0.03 ms).
+constexpr size_t kCompactMinIons = 262144;
+
 // Clear the striped launch counters of a single cloud.
 void zero_counters(unsigned long long* counters, hipStream_t s) {
     hipLaunchKernelGGL(zero_u64, dim3(1), dim3(256), 0, s, counters, kCounterWords);
@@ -969,6 +973,28 @@ CallCounts read_counters(icarion_gpu* h, hipStream_t s, bool with_state, unsigne
     c.alive = h->host_ctr[2];
     c.arrived = h->host_ctr[3];
     return c;
+}
+
+// The number of live ions, added to a running total of this call (words 6 and 7
+// of the launch counter stripes, cleared at its start); returns the total.
+uint64_t count_alive(icarion_gpu* h, unsigned long long* counters) {
+    const uint32_t n = static_cast<uint32_t>(h->n);
+    hipLaunchKernelGGL(count_state_kernel, dim3(std::min<uint32_t>((n + 255) / 256, 1024)), dim3(256), 0, h->stream,
+                       h->flags.p, h->arrival.p, n, counters + 4, kCounterStripes);
+    hipLaunchKernelGGL(fold_counters_kernel, dim3(1), dim3(256), 0, h->stream, counters + 4, h->host_ctr_dev);
+    hip_check(hipGetLastError(), "count live ions");
+    hip_check(hipStreamSynchronize(h->stream), "hipStreamSynchronize");
+    return h->host_ctr[2];
+}
+
+// The buffers of a lane order of n ions.
+void resize_order(icarion_gpu* h, uint32_t n) {
+    h->ord.resize(n);
+    h->ord_keys_a.resize(n);
+    h->ord_keys_b.resize(n);
+    h->ord_idx.resize(n);
+    const size_t tb = brick_sort_temp_bytes(n);
+    if (h->ord_temp.n < tb) h->ord_temp.resize(tb);
 }
 
 IonPtrs ion_ptrs(icarion_gpu* h) {
@@ -1509,13 +1535,7 @@ void do_step(icarion_gpu* h, double t0, double dt, uint64_t n_steps, uint64_t st
         double o_origin[3] = {0, 0, 0}, o_inv[3] = {0, 0, 0};
         uint32_t o_nb[3] = {1, 1, 1};
         if (order) {
-            const uint32_t n = static_cast<uint32_t>(h->n);
-            h->ord.resize(n);
-            h->ord_keys_a.resize(n);
-            h->ord_keys_b.resize(n);
-            h->ord_idx.resize(n);
-            const size_t tb = brick_sort_temp_bytes(n);
-            if (h->ord_temp.n < tb) h->ord_temp.resize(tb);
+            resize_order(h, static_cast<uint32_t>(h->n));
             const auto& f = h->fsrc;
             const double first[3] = {f.x0, f.y0, f.z0}, last[3] = {f.x_last, f.y_last, f.z_last};
             const uint32_t nn[3] = {static_cast<uint32_t>(f.nx), static_cast<uint32_t>(f.ny), static_cast<uint32_t>(f.nz)};
@@ -1526,11 +1546,49 @@ void do_step(icarion_gpu* h, double t0, double dt, uint64_t n_steps, uint64_t st
                 o_inv[a] = spacing > 0.0 ? 1.0 / (4.0 * spacing) : 0.0;
             }
         }
+        // Ions that are lost leave their lanes idle for the rest of a launch, and
+        // without this for all launches after it.  Between launches of a large
+        // cloud the live ions are counted; once an eighth of the running lanes
+        // is idle, the next launches run the live ions alone (sorted to the
+        // front, lane t takes ion order[t]).  The count makes the host wait for
+        // the launch, so it is left out for longer each time it finds nothing.
+        // 1M ions x 20,000 steps in a quadrupole that loses two fifths of them in
+        // the first launch: 97.9 ms, now 71.3 ms.
+        const bool compact = !ws && !surrogate && !h->has_birth && field != FIELD_ARRAY &&
+                             launch_coll_kind(h) != COLL_EHSS && h->n >= kCompactMinIons;
+        uint32_t lanes = static_cast<uint32_t>(h->n);
+        uint64_t counted = 0;          // the running total behind the counts
+        uint32_t quiet = 0, wait = 0;  // counts without a find, launches until the next
+        const uint32_t* live_order = nullptr;
         ms = run_launches(h, S, n_steps, step_offset, spl, plan, snap, [&](uint64_t k0, uint64_t nk) {
             P.table = table + k0;
             P.step0 = step_offset + k0;
             P.n_steps = static_cast<uint32_t>(nk);
-            P.order = nullptr;
+            if (compact && k0 > 0) {
+                if (wait > 0) {
+                    --wait;
+                } else {
+                    const uint64_t total = count_alive(h, counters);
+                    const uint32_t alive = static_cast<uint32_t>(total - counted);
+                    counted = total;
+                    if (alive < lanes - lanes / 8) {
+                        const uint32_t n = static_cast<uint32_t>(h->n);
+                        resize_order(h, n);
+                        hip_check(sort_ions_by_brick(h->x.p, h->y.p, h->z.p, h->flags.p, n, o_origin, o_inv, o_nb,
+                                                     h->ord_keys_a.p, h->ord_keys_b.p, h->ord_idx.p, h->ord.p,
+                                                     h->ord_temp.p, h->ord_temp.n, h->stream),
+                                  "live ions first");
+                        live_order = h->ord.p;
+                        lanes = alive;
+                        quiet = 0;
+                    } else {
+                        wait = quiet < 4 ? 1u << quiet++ : 16u;
+                    }
+                }
+                if (lanes == 0) return;
+            }
+            P.n_ions = lanes;
+            P.order = live_order;
             if (order) {
                 hip_check(sort_ions_by_brick(h->x.p, h->y.p, h->z.p, h->flags.p, static_cast<uint32_t>(h->n),
                                              o_origin, o_inv, o_nb, h->ord_keys_a.p, h->ord_keys_b.p, h->ord_idx.p,

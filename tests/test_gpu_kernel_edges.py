@@ -160,3 +160,30 @@ def test_surrogate_launch_shapes(n):
     for f, scale in (("x", 1e-6), ("z", 1e-6), ("vx", 1.0), ("vz", 1.0)):
         same &= np.abs(getattr(a, f) - getattr(b, f)) <= 1e-5 * np.maximum(np.abs(getattr(b, f)), scale)
     assert same.mean() >= 0.998
+
+
+@pytest.mark.parametrize("precision", [_abi.PRECISION_FP64, _abi.PRECISION_FP32_KAHAN])
+def test_lost_ions_leave_the_launches(precision):
+    """A large trap that loses ions in every launch, among them all but a few at
+    last: the ions run alone after the first launches are the same, bit for bit,
+    as with one launch for the whole run, where no lane is dropped."""
+    w = W.quadrupole_workload(n=262144 + 77, seed=8, precision=precision)
+    w["domain"].radius_m = 0.6e-3
+    a, b = w["ensemble"].copy(), w["ensemble"].copy()
+    for e in (a, b):
+        e.active[::1001] = 0     # dead on arrival
+    sa = gpu_run(w, a, 3000, steps_per_launch=150)
+    sb = gpu_run(w, b, 3000, steps_per_launch=3000)
+    assert 0 < sa.alive < 0.7 * a.n
+    assert (sa.ion_steps, sa.collisions, sa.alive) == (sb.ion_steps, sb.collisions, sb.alive)
+    for f in ("x", "y", "z", "vx", "vy", "vz", "death_time_s", "active", "born"):
+        assert np.array_equal(getattr(a, f), getattr(b, f)), f
+
+
+def test_all_ions_lost(precision=_abi.PRECISION_FP32_KAHAN):
+    """Launches after the last ion is gone have nothing to run."""
+    w = W.quadrupole_workload(n=262144, seed=8, precision=precision)
+    w["domain"].length_m = 1e-9
+    g = w["ensemble"].copy()
+    st = gpu_run(w, g, 400, steps_per_launch=100)
+    assert st.alive == 0 and not g.active.any()
