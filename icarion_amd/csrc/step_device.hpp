@@ -358,6 +358,18 @@ __device__ d3 ehss_f64(const StepParams& P, d3 v_ion, d3 v_n, double mi, double 
     return ehss_core_f64(P, v_ion, v_n, mi, mn, r_gas, a0, nat, O, 0.0, kEhssMaxAttempts, rng);
 }
 
+// The HSS collision's sums with the rounding written out: which product of a sum
+// of two goes into the fma is else the compiler's choice in each kernel, and a
+// batch's ions, one to a lane, have to equal a single cloud's, four lanes each.
+__device__ __forceinline__ double speed_f64(d3 v) { return sqrt(fma(v.z, v.z, fma(v.y, v.y, v.x * v.x))); }
+
+// A component of the velocity after hss_collision: the centre of mass's plus the
+// relative speed vm along nd times the neutral's share of the mass.
+__device__ __forceinline__ double hss_velocity_f64(double v, double m, double vn, double m_gas, double inv_mt,
+                                                   double nd, double vm, double share) {
+    return fma(nd * vm, share, fma(v, m, vn * m_gas) * inv_mt);
+}
+
 // One collision stage; returns true on a collision event.  FLOW: the neutrals
 // move with ug (the gas velocity at the ion's position), else with the
 // constant gas velocity.
@@ -543,7 +555,7 @@ __device__ __forceinline__ bool collide_f64(const StepParams& P, const SpeciesDe
             vn = vn + u_gas;
         }
         const d3 vrel = v - vn;
-        const double vrel_mag = sqrt(dot(vrel, vrel));
+        const double vrel_mag = COLL == COLL_HSS ? speed_f64(vrel) : sqrt(dot(vrel, vrel));
         if (vrel_mag < kMinRelativeVelocity) return false;
         const double Pc = 1.0 - exp(-P.n * sigma * vrel_mag * dt);
         if (rng.uniform_f64() >= Pc) return false;
@@ -557,8 +569,10 @@ __device__ __forceinline__ bool collide_f64(const StepParams& P, const SpeciesDe
             }
             const d3 nd = iso_dir_f64(rng);
             const double inv_mt = 1.0 / (m + P.m_gas);
-            const d3 Vcom = (v * m + vn * P.m_gas) * inv_mt;
-            v = Vcom + (nd * vm) * (P.m_gas * inv_mt);
+            const double share = P.m_gas * inv_mt;
+            v = d3{hss_velocity_f64(v.x, m, vn.x, P.m_gas, inv_mt, nd.x, vm, share),
+                   hss_velocity_f64(v.y, m, vn.y, P.m_gas, inv_mt, nd.y, vm, share),
+                   hss_velocity_f64(v.z, m, vn.z, P.m_gas, inv_mt, nd.z, vm, share)};
         } else if (COLL == COLL_EHSS_TAB && off.y > 0u) {
             // offline branch of apply_collision (EHSSCollisionHandler.cpp:253-277)
             uint32_t mi = static_cast<uint32_t>(rng.uniform_f64() * static_cast<double>(off.z));

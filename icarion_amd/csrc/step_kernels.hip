@@ -277,8 +277,7 @@ __global__ void __launch_bounds__(256) step_f64_quad_kernel(const StepParams P, 
                 double sn, cs;
                 sincos_rev(c == 3u ? uniform53(o4.v[0], o4.v[1]) : ub, sn, cs);
                 const double vn = P.sigma_neutral * (sqrt(-2.0 * log_unit(ua)) * cs) + u_gas;
-                const d3 rel = quad_d3(v - vn);
-                const double vm = sqrt(dot(rel, rel));
+                const double vm = speed_f64(quad_d3(v - vn));
                 const double Pc = 1.0 - exp(-P.n * sp.sigma_hss * vm * (dt * te.nrel));
                 // lane 3's draws, on every lane (before any lane-dependent choice:
                 // a broadcast reads its source lane only while that is active)
@@ -290,7 +289,7 @@ __global__ void __launch_bounds__(256) step_f64_quad_kernel(const StepParams P, 
                     const double cosT = 2.0 * u_dir - 1.0;
                     const double sinT = sqrt(fmax(0.0, 1.0 - cosT * cosT));
                     const double nd = comp == 2 ? cosT : sinT * (comp == 0 ? cs3 : sn3);
-                    v = (v * m + vn * P.m_gas) * inv_mt + (nd * vm) * (P.m_gas * inv_mt);
+                    v = hss_velocity_f64(v, m, vn, P.m_gas, inv_mt, nd, vm, P.m_gas * inv_mt);
                     ++nc;
                     ++ncoll_launch;
                 }
