@@ -26,8 +26,15 @@ constexpr double kGeomEpsilon = 1e-12;
 constexpr double kMinVoltage = 1e-12;
 
 // Keeps a wave-uniform branch a branch: without it the compiler computes both
-// sides in every step and selects.
+// sides in every step and selects.  A unit whose uniform records lie in memory
+// defines KEEP_BRANCH_READS_ONLY: its branches are held by a scheduling barrier that
+// nothing is bound by, since an asm statement counts as a write to memory and takes
+// the scalar loads away from every record read after it.
+#ifdef KEEP_BRANCH_READS_ONLY
+__device__ __forceinline__ void keep_branch() { __builtin_amdgcn_sched_barrier(0x7ff); }
+#else
 __device__ __forceinline__ void keep_branch() { asm volatile(""); }
+#endif
 
 template <typename T>
 struct vec3 {

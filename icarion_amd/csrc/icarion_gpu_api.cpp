@@ -1792,6 +1792,21 @@ void do_step_multi(icarion_gpu* h, double t0, double dt, uint64_t n_steps, uint6
         h->dom_tables.resize(tabs.size());
         copy_in(h->dom_tables, tabs.data(), tabs.size(), h->stream, "domain tables");
         for (uint32_t d = 0; d < nd; ++d) Ps[d].table = h->dom_tables.p + size_t(d) * n_steps;
+        // each domain's own span, where the list's search would start at it: the
+        // spans' upper ends in order (they are sorted by the lower ones)
+        bool ordered = !h->dom_has_orbitrap;
+        for (size_t k = 1; k < h->dom_spans.size(); ++k) ordered &= h->dom_spans[k - 1].z_max <= h->dom_spans[k].z_max;
+        for (uint32_t d = 0; d < nd; ++d) Ps[d].span_alone = 0;
+        for (size_t k = 0; ordered && k < h->dom_spans.size(); ++k) {
+            const DomainSpan& sp = h->dom_spans[k];
+            if (sp.idx < 0 || sp.idx >= static_cast<int>(nd)) continue;
+            StepParams& P = Ps[sp.idx];
+            P.span_z_min = sp.z_min;
+            P.span_z_max = sp.z_max;
+            P.span_r2 = sp.radius * sp.radius;
+            P.span_before = k ? h->dom_spans[k - 1].z_max : -INFINITY;
+            P.span_alone = 1;
+        }
         h->dom_params_d.resize(nd);
         copy_in(h->dom_params_d, Ps.data(), nd, h->stream, "domain parameters");
         h->dom_ap_d.resize(nd);

@@ -2,10 +2,15 @@
 // + Kahan with the domain logic kept in FP64).
 //
 // A multi-domain instrument: every domain keeps its own geometry, analytic
-// field and gas, read per lane from a parameter record in global memory (a
-// wave may hold ions in several domains).  Per step and ion, the engine's
-// domain logic (SimulationEngineLifecycle.cpp:72-195) around the same push and
-// collision bodies as the single-domain kernels:
+// field and gas in a parameter record in global memory.  A wavefront runs a step
+// once for each domain that its ions are in, most often one: the record and its
+// step table entry are then wave-uniform and come by scalar loads, and the
+// domain lookup after the push starts with the domain's own span.  What bounds it
+// is the latency of the step's chain (100,000 ions are 1.5 wavefronts a SIMD).
+// With a record per lane every parameter was a vector load, the lookup a chain of
+// five dependent ones: 100,000 ions x 4000 steps in FP32 took 13.9 ms, now 12.8.
+// Per step and ion, the engine's domain logic (SimulationEngineLifecycle.cpp:
+// 72-195) around the same push and collision bodies as the single-domain kernels:
 //   prepare:  birth; the domain = DomainManager::find_domain_index of the
 //             position (DomainManager.cpp:66-109); none -> death at t;
 //   push:     RK4 (RK4Strategy.cpp:181-361) or Boris (BorisStrategy.cpp:18-98)
@@ -18,6 +23,7 @@
 //             death at t; found -> shared_boundary_handoff_domain
 //             (DomainManager.cpp:176-198) may move the index on; NaN kill.
 // An ion kept alive by the bridge is looked up again at the next step start.
+#define KEEP_BRANCH_READS_ONLY
 #include "step_device.hpp"
 #include "step_device_f32.hpp"
 
@@ -69,6 +75,33 @@ __device__ __forceinline__ int handoff_domain(const MultiParams& M, int cur, int
     const double dx = p.x - D.origin[0];
     const double dy = p.y - D.origin[1];
     return (dx * dx + dy * dy <= M.ap_sq[cur]) ? cur + 1 : -1;
+}
+
+// Whether find_domain(M, p) is domain d by its own span alone: no span before it
+// in the z order reaches p.z, so the search starts at d's.
+__device__ __forceinline__ bool in_own_span(const StepParams& D, d3 p) {
+    return D.span_alone & (p.z > D.span_before) & (p.z <= D.span_z_max) & (p.z >= D.span_z_min) &
+           !(p.x * p.x + p.y * p.y > D.span_r2) & contains_f64(D, p);
+}
+
+// The end of a step at position p for an ion that made it in domain `dom`: its
+// domain index and whether it stays alive; found / checked as at the step start.
+__device__ __forceinline__ bool settle_domain(const MultiParams& M, const StepParams& D, int dom, d3 p, int& cur,
+                                              int& found, bool& checked) {
+    cur = dom;
+    found = dom;
+    if (!in_own_span(D, p)) found = find_domain(M, p);
+    if (found < 0) {
+        const int b = bridge_domain(M, dom, p);
+        if (b < 0) return false;
+        cur = b;
+        checked = false;
+        return true;
+    }
+    const int h = handoff_domain(M, dom, found, p);
+    cur = h >= 0 ? h : found;
+    checked = true;
+    return true;
 }
 
 // The hoisted damping factor of the single-domain kernels for one domain's gas
@@ -130,120 +163,116 @@ __device__ __forceinline__ void multi_ion(const MultiParams& M, const IonPtrs& S
     bool checked = false;   // found = the domain of the current position
     const double dt = M.dt;
     const double half_dt = dt * 0.5;
+    // 0: done, 1: stepping, 2: unborn
+    uint32_t state = !born ? 2u : active ? 1u : 0u;
+    const uint32_t lane = threadIdx.x & 63u;
     for (uint32_t k = 0; k < M.n_steps; ++k) {
+        if (__ballot(state != 0u) == 0ull) break;
         const double t = M.t_table[M.k0 + k].t;
-        if (!born) {
-            if (t >= birth) {
-                born = true;
-                active = true;
-                checked = false;
-            } else {
-                continue;
+        if (state == 2u && t >= birth) {
+            born = true;
+            checked = false;
+            state = 1u;
+        }
+        if (state == 1u && !checked) {
+            found = find_domain(M, pos);
+            if (found < 0) {
+                state = 0u;
+                death = t;
             }
         }
-        if (!active) break;
-        const int dom = checked ? found : find_domain(M, pos);
-        if (dom < 0) {
-            active = false;
-            death = t;
-            break;
-        }
-        cur = dom;
-        const StepParams& D = M.dom[dom];
-        if (dom != sp_dom) {
-            sp = D.species[sidx];
-            sp_dom = dom;
-        }
-        if constexpr (COLL == COLL_DAMPING) {
-            if (dom != lpre_dom) {
-                lpre = damping_pre_f64(D, sp, m, q);
-                lpre_dom = dom;
+        // one pass for each domain the wavefront's live ions are in
+        const int dom = found;
+        for (uint64_t todo = __ballot(state == 1u); todo;) {
+            const int next = __builtin_amdgcn_readlane(dom, __builtin_ctzll(todo));
+            const bool here = state == 1u && dom == next && ((todo >> lane) & 1ull);
+            todo &= ~__ballot(here);
+            if (!here) continue;
+            // next again, read where only its own lanes are: uniform to the compiler
+            const int d = __builtin_amdgcn_readfirstlane(dom);
+            const StepParams& D = M.dom[d];
+            if (d != sp_dom) {
+                sp = D.species[sidx];
+                sp_dom = d;
             }
-        }
-        const StepEntry te = D.table[M.k0 + k];
-        const double z_before = pos.z;
-        // the domain's gas density at the step start over its constant one
-        const double lp = lpre * te.nrel;
-        if constexpr (INTEG == 0) {
-            const d3 p0 = pos, v0 = vel;
-            const d3 k1v = v0;
-            const d3 k1a = domain_force<COLL, EXT>(D, p0, v0, te.c0, te.e0, q, m, lp) * inv_m;
-            const d3 k2v = v0 + k1a * half_dt;
-            const d3 k2a = domain_force<COLL, EXT>(D, p0 + k1v * half_dt, k2v, te.ch, te.eh, q, m, lp) * inv_m;
-            const d3 k3v = v0 + k2a * half_dt;
-            const d3 k3a = domain_force<COLL, EXT>(D, p0 + k2v * half_dt, k3v, te.ch, te.eh, q, m, lp) * inv_m;
-            const d3 k4v = v0 + k3a * dt;
-            const d3 k4a = domain_force<COLL, EXT>(D, p0 + k3v * dt, k4v, te.c1, te.e1, q, m, lp) * inv_m;
-            const double h6 = dt / 6.0;
-            pos = p0 + (k1v + k2v * 2.0 + k3v * 2.0 + k4v) * h6;
-            vel = v0 + (k1a + k2a * 2.0 + k3a * 2.0 + k4a) * h6;
-        } else {
-            const d3 a = domain_force<COLL, EXT>(D, pos, vel, te.c0, te.e0, q, m, lp) * inv_m;
-            const d3 vm = vel + a * half_dt;
-            d3 vp = vm;
-            if (D.magnetic) {
-                const double qm = q * inv_m;
-                const d3 tv = d3{D.B[0], D.B[1], D.B[2]} * (qm * dt * 0.5);
-                const double s_f = 2.0 / (1.0 + dot(tv, tv));
-                const d3 sv = tv * s_f;
-                const d3 vprime = vm + cross(vm, tv);
-                vp = vm + cross(vprime, sv);
-            }
-            pos = pos + vp * dt;
-            vel = vp + a * half_dt;
-        }
-        ++pushed;
-        if constexpr (COLL != COLL_NONE) {
-            PhiloxStream rng(M.seed, i, M.step0 + k);
-            // collision substeps in the EXT instantiation (one stage otherwise)
-            const int ns = EXT ? D.n_sub : 1;
-            const double dtc = EXT ? dt / static_cast<double>(D.n_sub) : dt;
-            // rates take the density ratio through dt, the OU kick through gamma
-            const double dtn = COLL == COLL_DAMPING ? dtc : dtc * te.nrel;
-            // the step domain's gas velocity at the pushed position
-            const d3 ug = EXT ? gas_velocity_f64(D, pos) : d3{0.0, 0.0, 0.0};
-            for (int s = 0; s < ns; ++s) {
-                bool hit;
-                if constexpr (COLL == COLL_HSS_MIX)   // per domain: its mixture, else its single gas
-                    hit = D.n_mix > 0 ? collide_f64<COLL_HSS_MIX, EXT>(D, sp, sidx, m, lp, vel, rng, dtn, ug)
-                                      : collide_f64<COLL_HSS, EXT>(D, sp, sidx, m, lp, vel, rng, dtn, ug);
-                else if constexpr (COLL == COLL_EHSS_MIX)
-                    hit = D.n_emix > 0 ? collide_f64<COLL_EHSS_MIX, EXT>(D, sp, sidx, m, lp, vel, rng, dtn, ug)
-                                       : collide_f64<COLL_EHSS, EXT>(D, sp, sidx, m, lp, vel, rng, dtn, ug);
-                else
-                    hit = collide_f64<COLL, EXT>(D, sp, sidx, m, lp, vel, rng, dtn, ug);
-                if (hit) {
-                    ++nc;
-                    ++ncoll_launch;
+            if constexpr (COLL == COLL_DAMPING) {
+                if (d != lpre_dom) {
+                    lpre = damping_pre_f64(D, sp, m, q);
+                    lpre_dom = d;
                 }
             }
-        }
-        if (D.detect && isnan(arrival)) {
-            if (z_before < D.det_z && pos.z >= D.det_z)
-                arrival = t + dt * (D.det_z - z_before) / (pos.z - z_before);
-        }
-        found = find_domain(M, pos);
-        if (found < 0) {
-            const int b = bridge_domain(M, cur, pos);
-            if (b < 0) {
-                active = false;
-                death = t;
-                break;
+            const StepEntry& te = D.table[M.k0 + k];
+            const double z_before = pos.z;
+            // the domain's gas density at the step start over its constant one
+            const double lp = lpre * te.nrel;
+            if constexpr (INTEG == 0) {
+                const d3 p0 = pos, v0 = vel;
+                const d3 k1v = v0;
+                const d3 k1a = domain_force<COLL, EXT>(D, p0, v0, te.c0, te.e0, q, m, lp) * inv_m;
+                const d3 k2v = v0 + k1a * half_dt;
+                const d3 k2a = domain_force<COLL, EXT>(D, p0 + k1v * half_dt, k2v, te.ch, te.eh, q, m, lp) * inv_m;
+                const d3 k3v = v0 + k2a * half_dt;
+                const d3 k3a = domain_force<COLL, EXT>(D, p0 + k2v * half_dt, k3v, te.ch, te.eh, q, m, lp) * inv_m;
+                const d3 k4v = v0 + k3a * dt;
+                const d3 k4a = domain_force<COLL, EXT>(D, p0 + k3v * dt, k4v, te.c1, te.e1, q, m, lp) * inv_m;
+                const double h6 = dt / 6.0;
+                pos = p0 + (k1v + k2v * 2.0 + k3v * 2.0 + k4v) * h6;
+                vel = v0 + (k1a + k2a * 2.0 + k3a * 2.0 + k4a) * h6;
+            } else {
+                const d3 a = domain_force<COLL, EXT>(D, pos, vel, te.c0, te.e0, q, m, lp) * inv_m;
+                const d3 vm = vel + a * half_dt;
+                d3 vp = vm;
+                if (D.magnetic) {
+                    const double qm = q * inv_m;
+                    const d3 tv = d3{D.B[0], D.B[1], D.B[2]} * (qm * dt * 0.5);
+                    const double s_f = 2.0 / (1.0 + dot(tv, tv));
+                    const d3 sv = tv * s_f;
+                    const d3 vprime = vm + cross(vm, tv);
+                    vp = vm + cross(vprime, sv);
+                }
+                pos = pos + vp * dt;
+                vel = vp + a * half_dt;
             }
-            cur = b;
-            checked = false;
-        } else {
-            const int h = handoff_domain(M, cur, found, pos);
-            cur = h >= 0 ? h : found;
-            checked = true;
-        }
-        if (!(isfinite(pos.x) && isfinite(pos.y) && isfinite(pos.z) && isfinite(vel.x) &&
-              isfinite(vel.y) && isfinite(vel.z))) {
-            active = false;
-            death = t;
-            break;
+            ++pushed;
+            if constexpr (COLL != COLL_NONE) {
+                PhiloxStream rng(M.seed, i, M.step0 + k);
+                // collision substeps in the EXT instantiation (one stage otherwise)
+                const int ns = EXT ? D.n_sub : 1;
+                const double dtc = EXT ? dt / static_cast<double>(D.n_sub) : dt;
+                // rates take the density ratio through dt, the OU kick through gamma
+                const double dtn = COLL == COLL_DAMPING ? dtc : dtc * te.nrel;
+                // the step domain's gas velocity at the pushed position
+                const d3 ug = EXT ? gas_velocity_f64(D, pos) : d3{0.0, 0.0, 0.0};
+                for (int s = 0; s < ns; ++s) {
+                    bool hit;
+                    if constexpr (COLL == COLL_HSS_MIX)   // per domain: its mixture, else its single gas
+                        hit = D.n_mix > 0 ? collide_f64<COLL_HSS_MIX, EXT>(D, sp, sidx, m, lp, vel, rng, dtn, ug)
+                                          : collide_f64<COLL_HSS, EXT>(D, sp, sidx, m, lp, vel, rng, dtn, ug);
+                    else if constexpr (COLL == COLL_EHSS_MIX)
+                        hit = D.n_emix > 0 ? collide_f64<COLL_EHSS_MIX, EXT>(D, sp, sidx, m, lp, vel, rng, dtn, ug)
+                                           : collide_f64<COLL_EHSS, EXT>(D, sp, sidx, m, lp, vel, rng, dtn, ug);
+                    else
+                        hit = collide_f64<COLL, EXT>(D, sp, sidx, m, lp, vel, rng, dtn, ug);
+                    if (hit) {
+                        ++nc;
+                        ++ncoll_launch;
+                    }
+                }
+            }
+            if (D.detect && isnan(arrival)) {
+                if (z_before < D.det_z && pos.z >= D.det_z)
+                    arrival = t + dt * (D.det_z - z_before) / (pos.z - z_before);
+            }
+            bool alive = settle_domain(M, D, d, pos, cur, found, checked);
+            alive = alive && (isfinite(pos.x) && isfinite(pos.y) && isfinite(pos.z) && isfinite(vel.x) &&
+                    isfinite(vel.y) && isfinite(vel.z));
+            if (!alive) {
+                state = 0u;
+                death = t;
+            }
         }
     }
+    if (state != 2u) active = state != 0u;
     S.x[i] = pos.x; S.y[i] = pos.y; S.z[i] = pos.z;
     S.vx[i] = vel.x; S.vy[i] = vel.y; S.vz[i] = vel.z;
     S.flags[i] = static_cast<uint8_t>((active ? 1 : 0) | (born ? 2 : 0));
@@ -253,14 +282,20 @@ __device__ __forceinline__ void multi_ion(const MultiParams& M, const IonPtrs& S
     S.domain[i] = cur;
 }
 
-template <int COLL, bool EXT>
-__device__ __forceinline__ f3 domain_accel_f32(const StepParams& D, f3 p, f3 v, double c, double ez, float qm,
-                                               float lpre) {
+template <int INTEG, int COLL, bool EXT>
+__device__ __forceinline__ void domain_push_f32(const StepParams& D, const StepEntry& te, f3 p0, f3 v0, float qm,
+                                                float lp, float dt, float half_dt, float h6, f3& dpos, f3& dvel) {
+    CellF32 cell;
     if constexpr (EXT) {
-        if (D.field_array) return accel_f32<FIELD_ARRAY, COLL, EXT>(D, D.fc, p, v, c, ez, qm, lpre);
+        if (D.field_array) {
+            push_f32<INTEG, FIELD_ARRAY, COLL, EXT>(D, D.fc, te, p0, v0, qm, lp, dt, half_dt, h6, cell, dpos, dvel);
+            return;
+        }
     }
-    if (D.instrument == 3) return accel_f32<FIELD_ORBITRAP, COLL, EXT>(D, D.fc, p, v, c, ez, qm, lpre);
-    return accel_f32<FIELD_LINEAR, COLL, EXT>(D, D.fc, p, v, c, ez, qm, lpre);
+    if (D.instrument == 3)
+        push_f32<INTEG, FIELD_ORBITRAP, COLL, EXT>(D, D.fc, te, p0, v0, qm, lp, dt, half_dt, h6, cell, dpos, dvel);
+    else
+        push_f32<INTEG, FIELD_LINEAR, COLL, EXT>(D, D.fc, te, p0, v0, qm, lp, dt, half_dt, h6, cell, dpos, dvel);
 }
 
 // The FP32 + Kahan body of the single-domain fast path over several domains:
@@ -301,136 +336,109 @@ __device__ __forceinline__ void multi_ion_f32(const MultiParams& M, const IonPtr
     const float dt = (float)M.dt;
     const float half_dt = 0.5f * dt;
     const float h6 = dt * (1.0f / 6.0f);
+    // 0: done, 1: stepping, 2: unborn
+    uint32_t state = !born ? 2u : active ? 1u : 0u;
+    const uint32_t lane = threadIdx.x & 63u;
     for (uint32_t k = 0; k < M.n_steps; ++k) {
+        if (__ballot(state != 0u) == 0ull) break;
         const double t = M.t_table[M.k0 + k].t;
-        if (!born) {
-            if (t >= birth) {
-                born = true;
-                active = true;
-                checked = false;
-            } else {
-                continue;
-            }
-        }
-        if (!active) break;
-        const int dom = checked ? found : find_domain(M, pos64());
-        if (dom < 0) {
-            active = false;
-            death = t;
-            break;
-        }
-        cur = dom;
-        const StepParams& D = M.dom[dom];
-        if (dom != const_dom) {
-            sp = D.species[sidx];
-            if constexpr (COLL == COLL_DAMPING) lpre = (float)damping_pre_f64(D, sp, md, qd);
-            inv_m_plus = (float)(1.0 / (md + D.m_gas));
-            kbt2_dt_over_m = (float)(2.0 * kBoltzmann * D.T / md * D.dt);
-            const_dom = dom;
-        }
-        const StepEntry te = D.table[M.k0 + k];
-        const float z_before = hi[2];
-        const float z_before_lo = lo[2];
-        const float nrel = (float)te.nrel;
-        const float lp = lpre * nrel;
-        const f3 p0{hi[0], hi[1], hi[2]};
-        const f3 v0{hi[3], hi[4], hi[5]};
-        f3 dpos, dvel;
-        if constexpr (INTEG == 0) {
-            const f3 k1a = domain_accel_f32<COLL, EXT>(D, p0, v0, te.c0, te.e0, qm, lp);
-            const f3 k2v = v0 + k1a * half_dt;
-            const f3 k2a = domain_accel_f32<COLL, EXT>(D, p0 + v0 * half_dt, k2v, te.ch, te.eh, qm, lp);
-            const f3 k3v = v0 + k2a * half_dt;
-            const f3 k3a = domain_accel_f32<COLL, EXT>(D, p0 + k2v * half_dt, k3v, te.ch, te.eh, qm, lp);
-            const f3 k4v = v0 + k3a * dt;
-            const f3 k4a = domain_accel_f32<COLL, EXT>(D, p0 + k3v * dt, k4v, te.c1, te.e1, qm, lp);
-            dpos = (v0 + k2v * 2.0f + k3v * 2.0f + k4v) * h6;
-            dvel = (k1a + k2a * 2.0f + k3a * 2.0f + k4a) * h6;
-        } else {
-            const f3 a = domain_accel_f32<COLL, EXT>(D, p0, v0, te.c0, te.e0, qm, lp);
-            const f3 vm = v0 + a * half_dt;
-            f3 rot{0.0f, 0.0f, 0.0f};
-            if (D.magnetic) {
-                const f3 tv = f3{(float)D.B[0], (float)D.B[1], (float)D.B[2]} * (qm * half_dt);
-                const float s_f = 2.0f / (1.0f + dot(tv, tv));
-                const f3 vprime = vm + cross(vm, tv);
-                rot = cross(vprime, tv * s_f);
-            }
-            dpos = (vm + rot) * dt;
-            dvel = a * dt + rot;
-        }
-        kahan_add(hi[0], lo[0], dpos.x);
-        kahan_add(hi[1], lo[1], dpos.y);
-        kahan_add(hi[2], lo[2], dpos.z);
-        kahan_add(hi[3], lo[3], dvel.x);
-        kahan_add(hi[4], lo[4], dvel.y);
-        kahan_add(hi[5], lo[5], dvel.z);
-        ++pushed;
-        if constexpr (COLL != COLL_NONE) {
-            PhiloxStream rng(M.seed, i, M.step0 + k);
-            f3 v{hi[3], hi[4], hi[5]};
-            const f3 vin = v;
-            // collision substeps in the EXT instantiation (one stage otherwise)
-            const int ns = EXT ? D.n_sub : 1;
-            const float sub = EXT ? 1.0f / static_cast<float>(D.n_sub) : 1.0f;
-            const float dtc = EXT ? static_cast<float>(M.dt / static_cast<double>(D.n_sub)) : dt;
-            uint32_t hits = 0;
-            const f3 ug = EXT ? gas_velocity_f32(D, D.fc, f3{hi[0], hi[1], hi[2]}) : f3{0.0f, 0.0f, 0.0f};
-            for (int s = 0; s < ns; ++s) {
-                bool hit;
-                if constexpr (COLL == COLL_HSS_MIX)
-                    hit = D.n_mix > 0 ? collide_f32<COLL_HSS_MIX, EXT>(D, D.fc, sp, sidx, m, inv_m_plus, lp,
-                                                                       kbt2_dt_over_m * sub, v, rng, dtc * nrel,
-                                                                       D.fc.n_dt * sub * nrel, ug)
-                                      : collide_f32<COLL_HSS, EXT>(D, D.fc, sp, sidx, m, inv_m_plus, lp,
-                                                                   kbt2_dt_over_m * sub, v, rng, dtc * nrel,
-                                                                   D.fc.n_dt * sub * nrel, ug);
-                else
-                    hit = collide_f32<COLL, EXT>(D, D.fc, sp, sidx, m, inv_m_plus, lp, kbt2_dt_over_m * sub, v,
-                                                 rng, dtc * nrel, D.fc.n_dt * sub * nrel, ug);
-                hits += hit ? 1u : 0u;
-            }
-            if (COLL == COLL_HSS || COLL == COLL_HSS_MIX) {
-                if (hits) {
-                    hi[3] = v.x; hi[4] = v.y; hi[5] = v.z;
-                    lo[3] = 0.0f; lo[4] = 0.0f; lo[5] = 0.0f;
-                    nc += hits;
-                    ncoll_launch += hits;
-                }
-            } else {
-                kahan_add(hi[3], lo[3], v.x - vin.x);
-                kahan_add(hi[4], lo[4], v.y - vin.y);
-                kahan_add(hi[5], lo[5], v.z - vin.z);
-            }
-        }
-        if (D.detect && isnan(arrival)) {
-            const double zb = (double)z_before + (double)z_before_lo;
-            const double za = (double)hi[2] + (double)lo[2];
-            if (zb < D.det_z && za >= D.det_z) arrival = t + M.dt * (D.det_z - zb) / (za - zb);
-        }
-        const d3 p_after = pos64();
-        found = find_domain(M, p_after);
-        if (found < 0) {
-            const int b = bridge_domain(M, cur, p_after);
-            if (b < 0) {
-                active = false;
-                death = t;
-                break;
-            }
-            cur = b;
+        if (state == 2u && t >= birth) {
+            born = true;
             checked = false;
-        } else {
-            const int hnd = handoff_domain(M, cur, found, p_after);
-            cur = hnd >= 0 ? hnd : found;
-            checked = true;
+            state = 1u;
         }
-        if (!(isfinite(hi[0]) && isfinite(hi[1]) && isfinite(hi[2]) && isfinite(hi[3]) && isfinite(hi[4]) &&
-              isfinite(hi[5]))) {
-            active = false;
-            death = t;
-            break;
+        if (state == 1u && !checked) {
+            found = find_domain(M, pos64());
+            if (found < 0) {
+                state = 0u;
+                death = t;
+            }
+        }
+        // one pass for each domain the wavefront's live ions are in
+        const int dom = found;
+        for (uint64_t todo = __ballot(state == 1u); todo;) {
+            const int next = __builtin_amdgcn_readlane(dom, __builtin_ctzll(todo));
+            const bool here = state == 1u && dom == next && ((todo >> lane) & 1ull);
+            todo &= ~__ballot(here);
+            if (!here) continue;
+            // next again, read where only its own lanes are: uniform to the compiler
+            const int d = __builtin_amdgcn_readfirstlane(dom);
+            const StepParams& D = M.dom[d];
+            if (d != const_dom) {
+                sp = D.species[sidx];
+                if constexpr (COLL == COLL_DAMPING) lpre = (float)damping_pre_f64(D, sp, md, qd);
+                inv_m_plus = (float)(1.0 / (md + D.m_gas));
+                kbt2_dt_over_m = (float)(2.0 * kBoltzmann * D.T / md * D.dt);
+                const_dom = d;
+            }
+            const StepEntry& te = D.table[M.k0 + k];
+            const float z_before = hi[2];
+            const float z_before_lo = lo[2];
+            const float nrel = te.nrelf;
+            const float lp = lpre * nrel;
+            const f3 p0{hi[0], hi[1], hi[2]};
+            const f3 v0{hi[3], hi[4], hi[5]};
+            f3 dpos, dvel;
+            domain_push_f32<INTEG, COLL, EXT>(D, te, p0, v0, qm, lp, dt, half_dt, h6, dpos, dvel);
+            kahan_add(hi[0], lo[0], dpos.x);
+            kahan_add(hi[1], lo[1], dpos.y);
+            kahan_add(hi[2], lo[2], dpos.z);
+            kahan_add(hi[3], lo[3], dvel.x);
+            kahan_add(hi[4], lo[4], dvel.y);
+            kahan_add(hi[5], lo[5], dvel.z);
+            ++pushed;
+            if constexpr (COLL != COLL_NONE) {
+                PhiloxStream rng(M.seed, i, M.step0 + k);
+                f3 v{hi[3], hi[4], hi[5]};
+                const f3 vin = v;
+                // collision substeps in the EXT instantiation (one stage otherwise)
+                const int ns = EXT ? D.n_sub : 1;
+                const float sub = EXT ? 1.0f / static_cast<float>(D.n_sub) : 1.0f;
+                const float dtc = EXT ? static_cast<float>(M.dt / static_cast<double>(D.n_sub)) : dt;
+                uint32_t hits = 0;
+                const f3 ug = EXT ? gas_velocity_f32(D, D.fc, f3{hi[0], hi[1], hi[2]}) : f3{0.0f, 0.0f, 0.0f};
+                for (int s = 0; s < ns; ++s) {
+                    bool hit;
+                    if constexpr (COLL == COLL_HSS_MIX)
+                        hit = D.n_mix > 0 ? collide_f32<COLL_HSS_MIX, EXT>(D, D.fc, sp, sidx, m, inv_m_plus, lp,
+                                                                           kbt2_dt_over_m * sub, v, rng, dtc * nrel,
+                                                                           D.fc.n_dt * sub * nrel, ug)
+                                          : collide_f32<COLL_HSS, EXT>(D, D.fc, sp, sidx, m, inv_m_plus, lp,
+                                                                       kbt2_dt_over_m * sub, v, rng, dtc * nrel,
+                                                                       D.fc.n_dt * sub * nrel, ug);
+                    else
+                        hit = collide_f32<COLL, EXT>(D, D.fc, sp, sidx, m, inv_m_plus, lp, kbt2_dt_over_m * sub, v,
+                                                     rng, dtc * nrel, D.fc.n_dt * sub * nrel, ug);
+                    hits += hit ? 1u : 0u;
+                }
+                if (COLL == COLL_HSS || COLL == COLL_HSS_MIX) {
+                    if (hits) {
+                        hi[3] = v.x; hi[4] = v.y; hi[5] = v.z;
+                        lo[3] = 0.0f; lo[4] = 0.0f; lo[5] = 0.0f;
+                        nc += hits;
+                        ncoll_launch += hits;
+                    }
+                } else {
+                    kahan_add(hi[3], lo[3], v.x - vin.x);
+                    kahan_add(hi[4], lo[4], v.y - vin.y);
+                    kahan_add(hi[5], lo[5], v.z - vin.z);
+                }
+            }
+            if (D.detect && isnan(arrival)) {
+                const double zb = (double)z_before + (double)z_before_lo;
+                const double za = (double)hi[2] + (double)lo[2];
+                if (zb < D.det_z && za >= D.det_z) arrival = t + M.dt * (D.det_z - zb) / (za - zb);
+            }
+            bool alive = settle_domain(M, D, d, pos64(), cur, found, checked);
+            alive = alive && (isfinite(hi[0]) && isfinite(hi[1]) && isfinite(hi[2]) && isfinite(hi[3]) &&
+                              isfinite(hi[4]) && isfinite(hi[5]));
+            if (!alive) {
+                state = 0u;
+                death = t;
+            }
         }
     }
+    if (state != 2u) active = state != 0u;
     S.x[i] = (double)hi[0] + (double)lo[0];
     S.y[i] = (double)hi[1] + (double)lo[1];
     S.z[i] = (double)hi[2] + (double)lo[2];

@@ -256,6 +256,10 @@ struct StepParams {
     uint32_t pressure_wave;
     double pressure_scale;
     double wave_const[ICARION_N_VOLTAGE_SLOTS];
+    // several domains: this domain's entry of the span list, and the largest
+    // z_max of the spans before it; span_alone = 0: look it up in the list
+    double span_z_min, span_z_max, span_r2, span_before;
+    int span_alone;
 };
 
 // Fill P.fc from the FP64 fields (after P.dt is set).

@@ -546,3 +546,31 @@ def test_snapshots_over_several_domains():
     for s in snaps:
         seen |= set(s["domain"].tolist())
     assert seen == {0, 1, 2}
+
+
+@pytest.mark.parametrize("spans", [
+    ((0.0, 5e-3, 3e-3), (5e-3, 15e-3, 2e-3), (15e-3, 20e-3, 3e-3)),     # end to end
+    ((0.0, 8e-3, 3e-3), (5e-3, 15e-3, 2e-3), (12e-3, 20e-3, 3e-3)),     # overlapping
+    ((0.0, 20e-3, 1.5e-3), (5e-3, 8e-3, 3e-3), (8e-3, 12e-3, 2.5e-3)),  # the first holds the others' axis
+    ((12e-3, 20e-3, 2e-3), (0.0, 12e-3, 2e-3), (4e-3, 6e-3, 3e-3)),     # not in z order, one inside another
+])
+def test_wavefronts_over_several_domains(oracle, spans):
+    """Every wavefront's ions in all the domains at once, which follow one another,
+    overlap or lie within each other: no gas, ion by ion as the oracle."""
+    w = W.multi_domain_workload(n=391, seed=9, n_steps=600, dt=5e-9)
+    doms = [W.ims_domain(origin_z=a, length=b - a, radius=r, axial_V=20.0 * (k + 1), gas="N2", pressure_Pa=10.0)
+            for k, (a, b, r) in enumerate(spans)]
+    rng = np.random.default_rng(11)
+    ens = w["ensemble"]
+    ens.z[:] = rng.uniform(-1e-3, 21e-3, ens.n)
+    g, o = ens.copy(), ens.copy()
+    ap = [1.5e-3, 1e-3, 0.0]
+    sg, dg = gpu_multi(w, g, 600, domains=doms, apertures=ap)
+    so, do = oracle_multi(oracle, w, o, 600, domains=doms, apertures=ap)
+    assert 0 < so.alive < ens.n and len(set(do)) == 3
+    assert (sg.ion_steps, sg.alive) == (so.ion_steps, so.alive)
+    np.testing.assert_array_equal(dg, do)
+    np.testing.assert_array_equal(g.active, o.active)
+    np.testing.assert_array_equal(g.death_time_s, o.death_time_s)
+    for f in ("x", "y", "z", "vx", "vy", "vz"):
+        np.testing.assert_allclose(getattr(g, f), getattr(o, f), rtol=1e-9, atol=1e-15, err_msg=f)
