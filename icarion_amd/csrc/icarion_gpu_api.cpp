@@ -2309,7 +2309,7 @@ icarion_batch_tuning batch_shape(const icarion_gpu* h, int cls, const icarion_ba
 // classes in `mask`); returns device milliseconds.
 float batch_launch(icarion_gpu* h, icarion_batch_tuning t64, icarion_batch_tuning t32, int mask) {
     // the surrogate class has one shape: 256 ions per tile and two workgroups
-    // per CU, the occupancy its registers (2 waves per SIMD) and 47 KB of LDS
+    // per CU, the occupancy its registers (2 waves per SIMD) and 36 KB of LDS
     // weights allow
     const icarion_batch_tuning shape[kBatchClasses] = {t64, t32, {256, 2}};
     for (int cls = 0; cls < kBatchClasses; ++cls) batch_build_tiles(h, cls, shape[cls].block_size);

@@ -1,6 +1,7 @@
 // step_kernels.hip - fused multi-step ion kernels for gfx950.
 //
-// One ion per lane.  A lane loads its ion once (coalesced SoA), runs
+// One ion per lane (four lanes in FP64 for small clouds, a wavefront's lanes
+// together through geometry EHSS).  A lane loads its ion once (coalesced SoA), runs
 // params.n_steps engine steps with the state in registers, and stores it
 // once; per step it does what the reference engine does to one ion:
 //   prepare  (SimulationEngineLifecycle.cpp:86-107): birth, domain lookup;

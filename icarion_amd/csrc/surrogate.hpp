@@ -37,9 +37,8 @@ namespace icarion {
 constexpr int kMlpIn = 6;
 constexpr int kMlpH = 128;
 constexpr int kMlpOut = 3;
-// Workgroup size of the single-cloud surrogate step kernel, which runs three
-// wavefronts per SIMD (3 workgroups of 50 KB LDS per CU).  Eight-wavefront
-// workgroups at four wavefronts per SIMD spill registers and run no faster.
+// Workgroup size of the single-cloud surrogate step kernel: 40 KB of LDS each,
+// so that four (large clouds) or three workgroups fit a CU.
 constexpr int kSurrogateBlock = 256;
 constexpr int kMlpParams = kMlpH * kMlpIn + kMlpH + kMlpH * kMlpH + kMlpH + kMlpOut * kMlpH + kMlpOut;
 // natural parameter layout (row-major, out x in)
