@@ -85,7 +85,8 @@ hipError_t launch_precompute(const float4* atoms, const uint32_t* offsets, const
 struct TrainBuffers {
     float *X, *T;
     float *Z1, *H1, *Z2, *H2, *Y, *dY, *dH2, *dH1;
-    float *params, *grad, *m, *v, *loss;
+    float *params, *grad, *m, *v;
+    double* loss;
     float* ws;
     int B;
 };
@@ -2598,13 +2599,19 @@ __global__ void zero_f32_kernel(float* p, int n) {
     if (i < n) p[i] = 0.f;
 }
 
+__global__ void zero_f64_kernel(double* p, int n) {
+    const int i = threadIdx.x;
+    if (i < n) p[i] = 0.0;
+}
+
 __global__ void zero_u32_kernel(uint32_t* p, int n) {
     const int i = threadIdx.x;
     if (i < n) p[i] = 0u;
 }
 
 struct TrainDev {
-    DevBuf<float> Z1, H1, Z2, H2, Y, dY, dH2, dH1, params, grad, m, v, loss, Xb, Tb, ws;
+    DevBuf<float> Z1, H1, Z2, H2, Y, dY, dH2, dH1, params, grad, m, v, Xb, Tb, ws;
+    DevBuf<double> loss;
     void alloc(int B) {
         Z1.resize(static_cast<size_t>(B) * kMlpH); H1.resize(static_cast<size_t>(B) * kMlpH);
         Z2.resize(static_cast<size_t>(B) * kMlpH); H2.resize(static_cast<size_t>(B) * kMlpH);
@@ -2623,8 +2630,9 @@ struct TrainDev {
         return t;
     }
     void release() {
-        for (DevBuf<float>* b : {&Z1, &H1, &Z2, &H2, &Y, &dY, &dH2, &dH1, &params, &grad, &m, &v, &loss, &Xb, &Tb, &ws})
+        for (DevBuf<float>* b : {&Z1, &H1, &Z2, &H2, &Y, &dY, &dH2, &dH1, &params, &grad, &m, &v, &Xb, &Tb, &ws})
             b->release();
+        loss.release();
     }
 };
 
@@ -3628,13 +3636,13 @@ int icarion_gpu_surrogate_train(icarion_gpu* h, const float* X, const float* T, 
                 hip_check(random_permutation(static_cast<uint32_t>(n), desc->seed, ep, keys_a.p, keys_b.p, idx.p,
                                              perm_d.p, sort_temp.p, temp_bytes, s),
                           "epoch permutation");
-                hipLaunchKernelGGL(zero_f32_kernel, dim3(1), dim3(64), 0, s, td.loss.p, 1);
+                hipLaunchKernelGGL(zero_f64_kernel, dim3(1), dim3(64), 0, s, td.loss.p, 1);
                 hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, s, ctr.p, 1);  // batch index only
                 for (size_t b = 0; b < n_batches; ++b) hip_check(hipGraphLaunch(exec, s), "hipGraphLaunch");
-                float l = 0.f;
-                hip_check(hipMemcpyAsync(&l, td.loss.p, sizeof(float), hipMemcpyDeviceToHost, s), "read loss");
+                double l = 0.0;
+                hip_check(hipMemcpyAsync(&l, td.loss.p, sizeof(l), hipMemcpyDeviceToHost, s), "read loss");
                 hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
-                if (loss_per_epoch) loss_per_epoch[ep] = l / static_cast<float>(n_batches);
+                if (loss_per_epoch) loss_per_epoch[ep] = static_cast<float>(l / static_cast<double>(n_batches));
             }
         } catch (...) {
             (void)hipGraphExecDestroy(exec);
@@ -3665,13 +3673,13 @@ int icarion_gpu_surrogate_grad(icarion_gpu* h, const float* X, const float* T, s
         copy_in(td.params, h->params.data(), kMlpParams, s, "upload params");
         copy_in(td.Xb, X, n * kMlpIn, s, "upload X");
         copy_in(td.Tb, T, n * kMlpOut, s, "upload T");
-        hipLaunchKernelGGL(zero_f32_kernel, dim3(1), dim3(64), 0, s, td.loss.p, 1);
+        hipLaunchKernelGGL(zero_f64_kernel, dim3(1), dim3(64), 0, s, td.loss.p, 1);
         hip_check(mlp_fwd_bwd(td.view(td.Xb.p, td.Tb.p, B), s), "fwd/bwd");
         copy_out(grad_out, td.grad, kMlpParams, s, "download grad");
-        float l = 0.f;
-        hip_check(hipMemcpyAsync(&l, td.loss.p, sizeof(float), hipMemcpyDeviceToHost, s), "read loss");
+        double l = 0.0;
+        hip_check(hipMemcpyAsync(&l, td.loss.p, sizeof(l), hipMemcpyDeviceToHost, s), "read loss");
         hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
-        if (loss_out) *loss_out = l;
+        if (loss_out) *loss_out = static_cast<float>(l);
         td.release();
     });
 }

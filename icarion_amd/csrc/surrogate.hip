@@ -156,8 +156,10 @@ __global__ void gemm_reduce_kernel(const float* __restrict__ W, int splits, int 
     gemm_epilogue(mode, v, idx, static_cast<int>(idx % N), C, bias, H, mask, accumulate);
 }
 
-// dY = (Y - T) / B; loss accumulated (sum of 0.5 d^2 / B)
-__global__ void out_grad_kernel(const float* Y, const float* T, float* dY, int n, float inv_b, float* loss) {
+// dY = (Y - T) / B; loss accumulated (sum of 0.5 d^2 / B).  The sum is in 64 bits: the
+// wavefronts add in any order, which an epoch's FP32 sum showed at 1e-6 from run to
+// run.  The add is the hardware's (ordinary device memory), without a retry loop.
+__global__ void out_grad_kernel(const float* Y, const float* T, float* dY, int n, float inv_b, double* loss) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     float l = 0.f;
     if (i < n) {
@@ -167,7 +169,7 @@ __global__ void out_grad_kernel(const float* Y, const float* T, float* dY, int n
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off, 64);
-    if ((threadIdx.x & 63) == 0) atomicAdd(loss, l);
+    if ((threadIdx.x & 63) == 0) unsafeAtomicAdd(loss, static_cast<double>(l));
 }
 
 __global__ void adam_kernel(float* p, const float* g, float* m, float* v, int n, float lr, float b1,
@@ -250,7 +252,8 @@ hipError_t gemm_f32(bool ta, bool tb, const float* A, const float* B, float* C, 
 struct TrainBuffers {
     float *X, *T;            // batch views
     float *Z1, *H1, *Z2, *H2, *Y, *dY, *dH2, *dH1;
-    float *params, *grad, *m, *v, *loss;
+    float *params, *grad, *m, *v;
+    double* loss;
     float* ws;               // kGemmWorkspaceFloats
     int B;
 };
