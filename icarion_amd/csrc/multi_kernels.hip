@@ -284,18 +284,18 @@ __device__ __forceinline__ void multi_ion(const MultiParams& M, const IonPtrs& S
 
 template <int INTEG, int COLL, bool EXT>
 __device__ __forceinline__ void domain_push_f32(const StepParams& D, const StepEntry& te, f3 p0, f3 v0, float qm,
-                                                float lp, float dt, float half_dt, float h6, f3& dpos, f3& dvel) {
+                                                float lp, float dt, float half_dt, f3& dpos, f3& dvel) {
     CellF32 cell;
     if constexpr (EXT) {
         if (D.field_array) {
-            push_f32<INTEG, FIELD_ARRAY, COLL, EXT>(D, D.fc, te, p0, v0, qm, lp, dt, half_dt, h6, cell, dpos, dvel);
+            push_f32<INTEG, FIELD_ARRAY, COLL, EXT>(D, D.fc, te, p0, v0, qm, lp, dt, half_dt, cell, dpos, dvel);
             return;
         }
     }
     if (D.instrument == 3)
-        push_f32<INTEG, FIELD_ORBITRAP, COLL, EXT>(D, D.fc, te, p0, v0, qm, lp, dt, half_dt, h6, cell, dpos, dvel);
+        push_f32<INTEG, FIELD_ORBITRAP, COLL, EXT>(D, D.fc, te, p0, v0, qm, lp, dt, half_dt, cell, dpos, dvel);
     else
-        push_f32<INTEG, FIELD_LINEAR, COLL, EXT>(D, D.fc, te, p0, v0, qm, lp, dt, half_dt, h6, cell, dpos, dvel);
+        push_f32<INTEG, FIELD_LINEAR, COLL, EXT>(D, D.fc, te, p0, v0, qm, lp, dt, half_dt, cell, dpos, dvel);
 }
 
 // The FP32 + Kahan body of the single-domain fast path over several domains:
@@ -379,13 +379,8 @@ __device__ __forceinline__ void multi_ion_f32(const MultiParams& M, const IonPtr
             const f3 p0{hi[0], hi[1], hi[2]};
             const f3 v0{hi[3], hi[4], hi[5]};
             f3 dpos, dvel;
-            domain_push_f32<INTEG, COLL, EXT>(D, te, p0, v0, qm, lp, dt, half_dt, h6, dpos, dvel);
-            kahan_add(hi[0], lo[0], dpos.x);
-            kahan_add(hi[1], lo[1], dpos.y);
-            kahan_add(hi[2], lo[2], dpos.z);
-            kahan_add(hi[3], lo[3], dvel.x);
-            kahan_add(hi[4], lo[4], dvel.y);
-            kahan_add(hi[5], lo[5], dvel.z);
+            domain_push_f32<INTEG, COLL, EXT>(D, te, p0, v0, qm, lp, dt, half_dt, dpos, dvel);
+            apply_push_f32<INTEG>(hi, lo, dpos, dvel, dt, h6);
             ++pushed;
             if constexpr (COLL != COLL_NONE) {
                 PhiloxStream rng(M.seed, i, M.step0 + k);

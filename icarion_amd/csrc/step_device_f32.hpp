@@ -10,13 +10,37 @@ namespace icarion {
 
 using f3 = vec3<float>;
 
+// The products and sums of the push are written with their rounding (fmaf): left
+// to the compiler, a product is fused with its sum only where both end up in one
+// basic block, so that another branch or another kernel around the same lines
+// would give other last bits, and an ion another course from its next collision
+// test on.
+__device__ __forceinline__ f3 fma3(f3 a, float s, f3 b) {
+    return f3{fmaf(a.x, s, b.x), fmaf(a.y, s, b.y), fmaf(a.z, s, b.z)};
+}
+__device__ __forceinline__ float dot(f3 a, f3 b) { return fmaf(a.z, b.z, fmaf(a.x, b.x, a.y * b.y)); }
+// |v|^2 of a relative velocity after a push by INTEG (0 RK4, 1 Boris): their
+// kernels have always begun the sum with another component.
+template <int INTEG>
+__device__ __forceinline__ float speed2_f32(f3 v) {
+    return fmaf(v.z, v.z, INTEG == 0 ? fmaf(v.x, v.x, v.y * v.y) : fmaf(v.y, v.y, v.x * v.x));
+}
+__device__ __forceinline__ f3 cross(f3 a, f3 b) {
+    return f3{fmaf(a.y, b.z, -(a.z * b.y)), fmaf(a.z, b.x, -(a.x * b.z)), fmaf(a.x, b.y, -(a.y * b.x))};
+}
+__device__ __forceinline__ f3 mat_mul(const float m[9], f3 v) {
+    return f3{dot(f3{m[0], m[1], m[2]}, v), dot(f3{m[3], m[4], m[5]}, v), dot(f3{m[6], m[7], m[8]}, v)};
+}
+
 // compensated accumulation: (hi, lo) <- hi + lo + d  (Kahan / Fast2Sum)
-__device__ __forceinline__ void kahan_add(float& hi, float& lo, float d) {
-    const float y = d + lo;
+__device__ __forceinline__ void kahan_sum(float& hi, float& lo, float y) {
     const float t = hi + y;
     lo = y - (t - hi);
     hi = t;
 }
+__device__ __forceinline__ void kahan_add(float& hi, float& lo, float d) { kahan_sum(hi, lo, d + lo); }
+// the same with d = a s, the product unrounded
+__device__ __forceinline__ void kahan_fma(float& hi, float& lo, float a, float s) { kahan_sum(hi, lo, fmaf(a, s, lo)); }
 
 // hardware transcendentals: v_log_f32 (log2), v_exp_f32 (exp2), v_sin/cos_f32
 // (argument in revolutions), v_sqrt_f32, v_rcp_f32
@@ -59,18 +83,14 @@ __device__ __forceinline__ f3 field_f32(const StepParams& P, const FastConst& C,
         f3 l = s;
         if (!P.rot_identity) {
             keep_branch();
-            l = f3{C.g2l[0] * s.x + C.g2l[1] * s.y + C.g2l[2] * s.z,
-                   C.g2l[3] * s.x + C.g2l[4] * s.y + C.g2l[5] * s.z,
-                   C.g2l[6] * s.x + C.g2l[7] * s.y + C.g2l[8] * s.z};
+            l = mat_mul(C.g2l, s);
         }
         const float r_sq = fmaxf(1e-18f, l.x * l.x + l.y * l.y);
         const float Cf = 1.0f - C.R_char_sq * __builtin_amdgcn_rcpf(r_sq);
         f3 E{C.orbi_hk * l.x * Cf, C.orbi_hk * l.y * Cf, -C.orbi_k * l.z};
         if (!P.rot_identity) {
             keep_branch();
-            E = f3{C.l2g[0] * E.x + C.l2g[1] * E.y + C.l2g[2] * E.z,
-                   C.l2g[3] * E.x + C.l2g[4] * E.y + C.l2g[5] * E.z,
-                   C.l2g[6] * E.x + C.l2g[7] * E.y + C.l2g[8] * E.z};
+            E = mat_mul(C.l2g, E);
         }
         return E;
     } else {
@@ -189,11 +209,9 @@ __device__ __forceinline__ bool contains_f32(const StepParams& P, const FastCons
     f3 l = s;
     if (!P.rot_identity) {
         keep_branch();
-        l = f3{C.g2l[0] * s.x + C.g2l[1] * s.y + C.g2l[2] * s.z,
-               C.g2l[3] * s.x + C.g2l[4] * s.y + C.g2l[5] * s.z,
-               C.g2l[6] * s.x + C.g2l[7] * s.y + C.g2l[8] * s.z};
+        l = mat_mul(C.g2l, s);
     }
-    const float r2 = l.x * l.x + l.y * l.y;
+    const float r2 = fmaf(l.x, l.x, l.y * l.y);
     if (P.instrument == 3) {
         const float z_abs = fabsf(l.z);
         if (z_abs > C.half_L) return false;
@@ -205,6 +223,12 @@ __device__ __forceinline__ bool contains_f32(const StepParams& P, const FastCons
         return f_in >= 0.0f && f_out <= 0.0f;
     }
     return !(l.z < 0.0f) & !(l.z >= C.L) & (r2 <= C.R_eps_sq);
+}
+
+// 1 - exp(-x), small x by its series
+__device__ __forceinline__ float collision_probability_f32(float x) {
+    return x < 1e-3f ? x * fmaf(-0.5f * x, fmaf(x, -1.0f / 3.0f, 1.0f), 1.0f)
+                     : 1.0f - __builtin_amdgcn_exp2f(-x * 1.44269504089f);
 }
 
 __device__ __forceinline__ f3 iso_dir_f32(PhiloxStream& rng) {
@@ -245,7 +269,7 @@ __device__ __forceinline__ bool collide_f32(const StepParams& P, const FastConst
                     vn[c] = f3{r1 * fast_cos_rev(u2) + u_gas.x, r1 * fast_sin_rev(u2) + u_gas.y,
                                r2 * fast_cos_rev(u4) + u_gas.z};
                     const f3 vr = v - vn[c];
-                    const float vm = fast_sqrt(dot(vr, vr));
+                    const float vm = fast_sqrt(dot<float>(vr, vr));
                     if (vm >= (float)kMinRelativeVelocity) {
                         k[c] = (float)(P.mix_n[c] * sg[c]) * vm;
                         k_total += k[c];
@@ -279,7 +303,7 @@ __device__ __forceinline__ bool collide_f32(const StepParams& P, const FastConst
                 }
             }
             const f3 vr = v - vs;
-            const float vm = fast_sqrt(dot(vr, vr));
+            const float vm = fast_sqrt(dot<float>(vr, vr));
             const f3 nd = iso_dir_f32(rng);
             const float inv_mt = 1.0f / (m + ms);
             const f3 Vcom = (v * m + vs * ms) * inv_mt;
@@ -297,7 +321,7 @@ __device__ __forceinline__ bool collide_f32(const StepParams& P, const FastConst
         const f3 vn{r1 * fast_cos_rev(u2) + u_gas.x, r1 * fast_sin_rev(u2) + u_gas.y,
                     r2 * fast_cos_rev(u4) + u_gas.z};
         const f3 vrel = v - vn;
-        const float vm2 = dot(vrel, vrel);
+        const float vm2 = dot<float>(vrel, vrel);
         const float vm = fast_sqrt(vm2);
         if (vm < (float)kMinRelativeVelocity) return false;
         // P = 1 - exp(-x), evaluated as -expm1(-x) to keep small x accurate
@@ -311,7 +335,7 @@ __device__ __forceinline__ bool collide_f32(const StepParams& P, const FastConst
         return true;
     } else if constexpr (COLL == COLL_DAMPING) {
         if (P.ou_kicks) {
-            const float g = (P.damping_model == 3) ? lpre / fmaxf(1e-6f, fast_sqrt(dot(v, v))) : lpre;
+            const float g = (P.damping_model == 3) ? lpre / fmaxf(1e-6f, fast_sqrt(dot<float>(v, v))) : lpre;
             if (!(g > 0.0f)) return false;
             const float s = fast_sqrt(g * kbt2_dt_over_m);
             const float u1 = rng.uniform_f32(), u2 = rng.uniform_f32();
@@ -348,7 +372,7 @@ __device__ __forceinline__ f3 accel_f32(const StepParams& P, const FastConst& C,
                                         T c, T ez, float qm, float lpre, CellF32& cell) {
     f3 a = field_f32<FIELD>(P, C, p, c, ez, cell) * qm;
     if constexpr (COLL == COLL_DAMPING) {
-        const float g = (P.damping_model == 3) ? lpre / fmaxf(1e-6f, fast_sqrt(dot(v, v))) : lpre;
+        const float g = (P.damping_model == 3) ? lpre / fmaxf(1e-6f, fast_sqrt(dot<float>(v, v))) : lpre;
         if (g > 0.0f) {
             const f3 u = FLOW ? gas_velocity_f32(P, C, p) : f3{C.u_gas[0], C.u_gas[1], C.u_gas[2]};
             a = a - f3{v.x - u.x, v.y - u.y, v.z - u.z} * g;
@@ -364,58 +388,79 @@ __device__ __forceinline__ f3 accel_f32(const StepParams& P, const FastConst& C,
     return accel_f32<FIELD, COLL, FLOW>(P, C, p, v, c, ez, qm, lpre, cell);
 }
 
-// One RK4 or Boris push of the FP32 path: position and velocity increments of
-// the step from (p0, v0).
+// RF coefficient (or time) and axial field of stage S (0 start, 1 middle, 2 end):
+// FP64 for scaled field arrays (WIDE), rounded otherwise.
+template <bool WIDE, int S>
+__device__ __forceinline__ auto stage_c(const StepEntry& te) {
+    if constexpr (WIDE) return S == 0 ? te.c0 : S == 1 ? te.ch : te.c1;
+    else return S == 0 ? te.c0f : S == 1 ? te.chf : te.c1f;
+}
+template <bool WIDE, int S>
+__device__ __forceinline__ auto stage_e(const StepEntry& te) {
+    if constexpr (WIDE) return S == 0 ? te.e0 : S == 1 ? te.eh : te.e1;
+    else return S == 0 ? te.e0f : S == 1 ? te.ehf : te.e1f;
+}
+
+// The stages of RK4 along x (two = -2) or y (two = 2) of an RF field E = two p c(t).
+__device__ __forceinline__ void rk4_rf_axis(float p0, float v0, float two, const StepEntry& te, float qm, float dt,
+                                            float half_dt, float& dpos, float& dvel) {
+    const float k1a = two * p0 * te.c0f * qm;
+    const float k2v = fmaf(k1a, half_dt, v0);
+    const float k2a = two * fmaf(v0, half_dt, p0) * te.chf * qm;
+    const float k3v = fmaf(k2a, half_dt, v0);
+    const float k3a = two * fmaf(k2v, half_dt, p0) * te.chf * qm;
+    const float k4v = fmaf(k3a, dt, v0);
+    const float e4 = two * fmaf(k3v, dt, p0) * te.c1f;
+    dpos = fmaf(k3v, 2.0f, fmaf(k2v, 2.0f, v0)) + k4v;
+    dvel = fmaf(e4, qm, fmaf(k3a, 2.0f, fmaf(k2a, 2.0f, k1a)));
+}
+
+// One RK4 or Boris push of the FP32 path from (p0, v0).  The increments are
+// returned as apply_push_f32 takes them, RK4's in units of h6 = dt / 6, Boris'
+// position increment in units of dt.
 template <int INTEG, int FIELD, int COLL, bool FLOW = false>
 __device__ __forceinline__ void push_f32(const StepParams& P, const FastConst& C, const StepEntry& te, f3 p0, f3 v0,
-                                         float qm, float lp, float dt, float half_dt, float h6, CellF32& cell, f3& dpos,
+                                         float qm, float lp, float dt, float half_dt, CellF32& cell, f3& dpos,
                                          f3& dvel) {
+    constexpr bool X = FIELD == FIELD_ARRAY_X;
     if constexpr (INTEG == 0) {
         if constexpr (FIELD == FIELD_LINEAR && COLL != COLL_DAMPING) {
-            if (!P.has_rf) {
-                // E = (0, 0, E_z(t)) everywhere: the general stages below with
-                // x and y accelerations of zero, whose velocities stay v0
-                const float az1 = te.e0f * qm;
-                const float az2 = te.ehf * qm;
-                const float az4 = te.e1f * qm;
-                const float k2z = v0.z + az1 * half_dt;
-                const float k3z = v0.z + az2 * half_dt;
-                const float k4z = v0.z + az2 * dt;
-                dpos.x = (v0.x + v0.x * 2.0f + v0.x * 2.0f + v0.x) * h6;
-                dpos.y = (v0.y + v0.y * 2.0f + v0.y * 2.0f + v0.y) * h6;
-                dpos.z = (v0.z + k2z * 2.0f + k3z * 2.0f + k4z) * h6;
-                dvel = f3{0.0f, 0.0f, (az1 + az2 * 2.0f + az2 * 2.0f + az4) * h6};
-                return;
+            // E = (-2 x c(t), 2 y c(t), E_z(t)): the stages below by component, z first
+            const float az1 = te.e0f * qm, az2 = te.ehf * qm;
+            const float k2z = fmaf(az1, half_dt, v0.z), k3z = fmaf(az2, half_dt, v0.z), k4z = fmaf(az2, dt, v0.z);
+            f3 dp{0.0f, 0.0f, fmaf(k3z, 2.0f, fmaf(k2z, 2.0f, v0.z)) + k4z};
+            f3 dv{0.0f, 0.0f, fmaf(te.e1f, qm, fmaf(az2, 2.0f, fmaf(az2, 2.0f, az1)))};
+            if (P.has_rf) {
+                rk4_rf_axis(p0.x, v0.x, -2.0f, te, qm, dt, half_dt, dp.x, dv.x);
+                rk4_rf_axis(p0.y, v0.y, 2.0f, te, qm, dt, half_dt, dp.y, dv.y);
+            } else {   // no acceleration in x and y
+                dp.x = fmaf(v0.x, 2.0f, fmaf(v0.x, 2.0f, v0.x)) + v0.x;
+                dp.y = fmaf(v0.y, 2.0f, fmaf(v0.y, 2.0f, v0.y)) + v0.y;
             }
+            dpos = dp;
+            dvel = dv;
+            return;
         }
-        if constexpr (FIELD == FIELD_ARRAY_X) {   // stage times in FP64
-            const f3 k1a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, te.c0, te.e0, qm, lp, cell);
-            const f3 k2v = v0 + k1a * half_dt;
-            const f3 k2a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + v0 * half_dt, k2v, te.ch, te.eh, qm, lp, cell);
-            const f3 k3v = v0 + k2a * half_dt;
-            const f3 k3a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + k2v * half_dt, k3v, te.ch, te.eh, qm, lp, cell);
-            const f3 k4v = v0 + k3a * dt;
-            const f3 k4a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + k3v * dt, k4v, te.c1, te.e1, qm, lp, cell);
-            dpos = (v0 + k2v * 2.0f + k3v * 2.0f + k4v) * h6;
-            dvel = (k1a + k2a * 2.0f + k3a * 2.0f + k4a) * h6;
-        } else {
-            const f3 k1a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, te.c0f, te.e0f, qm, lp, cell);
-            const f3 k2v = v0 + k1a * half_dt;
-            const f3 k2a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + v0 * half_dt, k2v, te.chf, te.ehf, qm, lp, cell);
-            const f3 k3v = v0 + k2a * half_dt;
-            const f3 k3a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + k2v * half_dt, k3v, te.chf, te.ehf, qm, lp, cell);
-            const f3 k4v = v0 + k3a * dt;
-            const f3 k4a = accel_f32<FIELD, COLL, FLOW>(P, C, p0 + k3v * dt, k4v, te.c1f, te.e1f, qm, lp, cell);
-            dpos = (v0 + k2v * 2.0f + k3v * 2.0f + k4v) * h6;
-            dvel = (k1a + k2a * 2.0f + k3a * 2.0f + k4a) * h6;
-        }
-    } else {
-        f3 a;
-        if constexpr (FIELD == FIELD_ARRAY_X)
-            a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, te.c0, te.e0, qm, lp, cell);
+        const auto ch = stage_c<X, 1>(te), eh = stage_e<X, 1>(te), c1 = stage_c<X, 2>(te), e1 = stage_e<X, 2>(te);
+        const f3 k1a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, stage_c<X, 0>(te), stage_e<X, 0>(te), qm, lp, cell);
+        const f3 k2v = fma3(k1a, half_dt, v0);
+        const f3 k2a = accel_f32<FIELD, COLL, FLOW>(P, C, fma3(v0, half_dt, p0), k2v, ch, eh, qm, lp, cell);
+        const f3 k3v = fma3(k2a, half_dt, v0);
+        const f3 k3a = accel_f32<FIELD, COLL, FLOW>(P, C, fma3(k2v, half_dt, p0), k3v, ch, eh, qm, lp, cell);
+        const f3 k4v = fma3(k3a, dt, v0);
+        const f3 p4 = fma3(k3v, dt, p0);
+        const f3 a3 = fma3(k3a, 2.0f, fma3(k2a, 2.0f, k1a));
+        f3 a4;
+        // the last stage's field times q / m unrounded, without a damping force
+        if constexpr (COLL == COLL_DAMPING)
+            a4 = a3 + accel_f32<FIELD, COLL, FLOW>(P, C, p4, k4v, c1, e1, qm, lp, cell);
         else
-            a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, te.c0f, te.e0f, qm, lp, cell);
-        const f3 vm = v0 + a * half_dt;
+            a4 = fma3(field_f32<FIELD>(P, C, p4, c1, e1, cell), qm, a3);
+        dpos = fma3(k3v, 2.0f, fma3(k2v, 2.0f, v0)) + k4v;
+        dvel = a4;
+    } else {
+        const f3 a = accel_f32<FIELD, COLL, FLOW>(P, C, p0, v0, stage_c<X, 0>(te), stage_e<X, 0>(te), qm, lp, cell);
+        const f3 vm = fma3(a, half_dt, v0);
         f3 rot{0.0f, 0.0f, 0.0f};
         if (P.magnetic) {
             const f3 tv = f3{(float)P.B[0], (float)P.B[1], (float)P.B[2]} * (qm * half_dt);
@@ -424,8 +469,25 @@ __device__ __forceinline__ void push_f32(const StepParams& P, const FastConst& C
             rot = cross(vprime, tv * s_f);
         }
         // x += v+ dt, v = v+ + a dt/2 = v0 + a dt + rot (no cancellation)
-        dpos = (vm + rot) * dt;
-        dvel = a * dt + rot;
+        dpos = vm + rot;
+        dvel = fma3(a, dt, rot);
+    }
+}
+
+template <int INTEG>
+__device__ __forceinline__ void apply_push_f32(float hi[6], float lo[6], f3 dpos, f3 dvel, float dt, float h6) {
+    const float s = INTEG == 0 ? h6 : dt;
+    kahan_fma(hi[0], lo[0], dpos.x, s);
+    kahan_fma(hi[1], lo[1], dpos.y, s);
+    kahan_fma(hi[2], lo[2], dpos.z, s);
+    if constexpr (INTEG == 0) {
+        kahan_fma(hi[3], lo[3], dvel.x, s);
+        kahan_fma(hi[4], lo[4], dvel.y, s);
+        kahan_fma(hi[5], lo[5], dvel.z, s);
+    } else {
+        kahan_add(hi[3], lo[3], dvel.x);
+        kahan_add(hi[4], lo[4], dvel.y);
+        kahan_add(hi[5], lo[5], dvel.z);
     }
 }
 

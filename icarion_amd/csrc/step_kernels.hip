@@ -848,13 +848,8 @@ __device__ __forceinline__ void f32_ion(const StepParams& P, const IonPtrs& S, c
             const f3 p0{hi[0], hi[1], hi[2]};
             const f3 v0{hi[3], hi[4], hi[5]};
             f3 dpos, dvel;
-            push_f32<INTEG, FIELD, COLL, FLOW>(P, C, te, p0, v0, qm, lp, dt, half_dt, h6, cell, dpos, dvel);
-            kahan_add(hi[0], lo[0], dpos.x);
-            kahan_add(hi[1], lo[1], dpos.y);
-            kahan_add(hi[2], lo[2], dpos.z);
-            kahan_add(hi[3], lo[3], dvel.x);
-            kahan_add(hi[4], lo[4], dvel.y);
-            kahan_add(hi[5], lo[5], dvel.z);
+            push_f32<INTEG, FIELD, COLL, FLOW>(P, C, te, p0, v0, qm, lp, dt, half_dt, cell, dpos, dvel);
+            apply_push_f32<INTEG>(hi, lo, dpos, dvel, dt, h6);
             ++pushed;
             if constexpr (COLL != COLL_NONE) {
                 PhiloxStream rng(P.seed, i, P.step0 + k);
@@ -1009,13 +1004,8 @@ __device__ __forceinline__ void surr_ion(const StepParams& P, const IonPtrs& S, 
             const f3 p0{hi[0], hi[1], hi[2]};
             const f3 v0{hi[3], hi[4], hi[5]};
             f3 dpos, dvel;
-            push_f32<INTEG, FIELD, COLL_NONE>(P, C, te, p0, v0, qm, 0.f, dt, half_dt, h6, cell, dpos, dvel);
-            kahan_add(hi[0], lo[0], dpos.x);
-            kahan_add(hi[1], lo[1], dpos.y);
-            kahan_add(hi[2], lo[2], dpos.z);
-            kahan_add(hi[3], lo[3], dvel.x);
-            kahan_add(hi[4], lo[4], dvel.y);
-            kahan_add(hi[5], lo[5], dvel.z);
+            push_f32<INTEG, FIELD, COLL_NONE>(P, C, te, p0, v0, qm, 0.f, dt, half_dt, cell, dpos, dvel);
+            apply_push_f32<INTEG>(hi, lo, dpos, dvel, dt, h6);
             ++pushed;
             if (sigma > 0.0f) {
                 PhiloxStream rng(P.seed, i, P.step0 + k);
@@ -1023,16 +1013,15 @@ __device__ __forceinline__ void surr_ion(const StepParams& P, const IonPtrs& S, 
                 const float u3 = rng.uniform_f32(), u4 = rng.uniform_f32();
                 const float r1 = C.sigma_neutral * fast_sqrt(-2.0f * fast_ln(u1));
                 const float r2 = C.sigma_neutral * fast_sqrt(-2.0f * fast_ln(u3));
-                vn = f3{r1 * fast_cos_rev(u2) + C.u_gas[0], r1 * fast_sin_rev(u2) + C.u_gas[1],
-                        r2 * fast_cos_rev(u4) + C.u_gas[2]};
+                vn = f3{fmaf(r1, fast_cos_rev(u2), C.u_gas[0]), fmaf(r1, fast_sin_rev(u2), C.u_gas[1]),
+                        fmaf(r2, fast_cos_rev(u4), C.u_gas[2])};
                 const f3 v{hi[3], hi[4], hi[5]};
                 vrel = v - vn;
-                vm = fast_sqrt(dot(vrel, vrel));
+                vm = fast_sqrt(speed2_f32<INTEG>(vrel));
                 if (vm >= (float)kMinRelativeVelocity) {
                     // n dt of the step (the density ratio of a pressure waveform)
                     const float x = C.n_dt * te.nrelf * sigma * vm;
-                    const float Pc = x < 1e-3f ? x * (1.0f - 0.5f * x * (1.0f - x * (1.0f / 3.0f)))
-                                               : 1.0f - __builtin_amdgcn_exp2f(-x * 1.44269504089f);
+                    const float Pc = collision_probability_f32(x);
                     if (rng.uniform_f32() < Pc) {
                         coll = true;
                         const float uq = rng.uniform_f32();
@@ -1050,10 +1039,11 @@ __device__ __forceinline__ void surr_ion(const StepParams& P, const IonPtrs& S, 
         float out[3];
         if (mlp_eval(k, coll, in, out)) {
             if (coll) {
-                const float nrm = fast_sqrt(out[0] * out[0] + out[1] * out[1] + out[2] * out[2]);
+                const f3 o{out[0], out[1], out[2]};
+                const float nrm = fast_sqrt(dot(o, o));
                 float mu = nrm > 0.f ? -out[2] / nrm : 0.f;
                 mu = fminf(1.f, fmaxf(0.f, mu));
-                const float st = fast_sqrt(fmaxf(0.f, 1.f - mu * mu));
+                const float st = fast_sqrt(fmaxf(0.f, fmaf(-mu, mu, 1.f)));
                 const float inv = 1.0f / vm;
                 const f3 ax{vrel.x * inv, vrel.y * inv, vrel.z * inv};
                 const f3 a = fabsf(ax.x) < 0.9f ? f3{1.f, 0.f, 0.f} : f3{0.f, 1.f, 0.f};
@@ -1061,11 +1051,11 @@ __device__ __forceinline__ void surr_ion(const StepParams& P, const IonPtrs& S, 
                 t1 = t1 * (1.0f / fast_sqrt(dot(t1, t1)));
                 f3 t2 = cross(ax, t1);
                 t2 = t2 * (1.0f / fast_sqrt(dot(t2, t2)));
-                const f3 nvec = t1 * (st * in[1]) + t2 * (st * in[2]) + ax * (-mu);
-                const f3 vr = vrel - nvec * (2.0f * dot(vrel, nvec));
+                const f3 nvec = fma3(ax, -mu, fma3(t1, st * in[1], t2 * (st * in[2])));
+                const f3 vr = fma3(nvec, -2.0f * dot(vrel, nvec), vrel);
                 const f3 v{hi[3], hi[4], hi[5]};
-                const f3 Vcom = (v * m + vn * C.m_gas) * inv_m_plus;
-                const f3 vnew = Vcom + vr * (C.m_gas * inv_m_plus);
+                // centre of mass velocity + relative velocity times the neutral's share
+                const f3 vnew = fma3(fma3(v, m, vn * C.m_gas), inv_m_plus, vr * (C.m_gas * inv_m_plus));
                 hi[3] = vnew.x; hi[4] = vnew.y; hi[5] = vnew.z;
                 lo[3] = 0.f; lo[4] = 0.f; lo[5] = 0.f;
                 ++nc;
