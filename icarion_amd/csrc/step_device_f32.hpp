@@ -56,13 +56,15 @@ __device__ __forceinline__ float fast_sqrt(float x) { return __builtin_amdgcn_sq
 // more).  Gathering them at every stage, the RK4 kernel waited on four dependent
 // gathers per step: 1M ions x 2000 HSS steps on a 96 x 96 x 192 grid took 71 ms
 // of kernel time, now bound by vector issue and 29 ms; an in-cell test in place
-// of the cell search saves another 2 ms (3001 ions x 800: 3.69, 1.96, 1.61 ms).
+// of the cell search saves another 2 ms (3001 ions x 800: 3.69, 1.96, 1.61 ms),
+// the node's address formed for a new cell alone another 4 % (300,000 x 300: 1.58
+// and 1.51 ms).
 struct CellF32 {
     uint64_t node = ~0ull;   // the cell's first node
     f3 e[8];                 // corner 4 dx + 2 dy + dz
-    // the cell's indices for the in-cell test below; NaN (none passes it) while
-    // there is no cell and in the last cell of an axis, where positions past the
-    // grid are clamped
+    // the cell's indices for the in-cell test of field_f32; NaN (none passes it)
+    // while there is no cell and in the last cell of an axis, where positions
+    // past the grid are clamped
     f3 index{__builtin_nanf(""), 0.0f, 0.0f};
 };
 
@@ -96,13 +98,18 @@ __device__ __forceinline__ f3 field_f32(const StepParams& P, const FastConst& C,
     } else {
         // trilinear on float4 nodes; the axis search of the FP64 path on
         // non-uniform axes
-        // (branch-free: the clamped ends are selected over the interior value)
-        auto loc = [](float v, float v0, float vl, float inv_d, int n, int& i0, float& a) {
-            const float f = (v - v0) * inv_d;
-            const int i = min(static_cast<int>(f), n - 2);   // negative only below v0
+        // The cell (rounded down) and the coordinate in it of f = (v - v0) / spacing:
+        // the cell from the rounded product, the coordinate rounded once.
+        auto cell_of = [](float v, float v0, float inv_d, float& cell_i, float& a) {
+            cell_i = floorf((v - v0) * inv_d);
+            a = fmaf(v - v0, inv_d, -cell_i);
+        };
+        // clamped to the grid (branch-free: the ends are selected over the interior)
+        auto clamp_cell = [](float v, float v0, float vl, float inv_d, int n, float cell_i, int& i0, float& a) {
+            const int i = min(static_cast<int>(cell_i), n - 2);   // negative only below v0
             const bool below = v <= v0, above = v >= vl;
-            // (one rounding, written out: the in-cell shortcut takes the same value)
-            a = below ? 0.0f : above ? 1.0f : fmaf(v - v0, inv_d, -static_cast<float>(i));
+            const float in = static_cast<float>(i) < cell_i ? fmaf(v - v0, inv_d, -static_cast<float>(i)) : a;
+            a = below ? 0.0f : above ? 1.0f : in;
             i0 = below ? 0 : above ? n - 2 : i;
         };
         auto loc_axis = [](const float* __restrict__ ax, int n, float v, int& i0, float& a) {
@@ -123,51 +130,55 @@ __device__ __forceinline__ f3 field_f32(const StepParams& P, const FastConst& C,
         constexpr bool GEN = FIELD == FIELD_ARRAY_X;
         int ix = 0, iy = 0, iz = 0;
         float ax, ay, az;
-        // still in the kept cell: the cell coordinates minus the cell's indices,
-        // the values the search below gives, lie in [0, 1)
+        // Still in the kept cell?  The cell follows from the position alone, not from
+        // where the ion was before or where its launches begin.  (The coordinate
+        // against [0, 1) would decide otherwise within rounding of a face.)
         bool inside = false;
-        if constexpr (!GEN) {
-            ax = fmaf(p.x - C.fa_first[0], C.fa_inv[0], -cell.index.x);
-            ay = fmaf(p.y - C.fa_first[1], C.fa_inv[1], -cell.index.y);
-            az = fmaf(p.z - C.fa_first[2], C.fa_inv[2], -cell.index.z);
-            // (ax apart: min and max return the other operand for a NaN)
-            inside = ax >= 0.0f & ax < 1.0f & fminf(ay, az) >= 0.0f & fmaxf(ay, az) < 1.0f;
+        f3 at{0.0f, 0.0f, 0.0f};
+        if (!GEN || !P.axf_x) {
+            cell_of(p.x, C.fa_first[0], C.fa_inv[0], at.x, ax);
+            cell_of(p.y, C.fa_first[1], C.fa_inv[1], at.y, ay);
+            cell_of(p.z, C.fa_first[2], C.fa_inv[2], at.z, az);
         }
+        if constexpr (!GEN) inside = (at.x == cell.index.x) & (at.y == cell.index.y) & (at.z == cell.index.z);
+        f3 r{0.0f, 0.0f, 0.0f};
+        const size_t sy = static_cast<size_t>(P.nx), sz = static_cast<size_t>(P.nx) * P.ny;
         if (!inside) {
             if (GEN && P.axf_x) {
                 loc_axis(P.axf_x, P.nx, p.x, ix, ax);
                 loc_axis(P.axf_y, P.ny, p.y, iy, ay);
                 loc_axis(P.axf_z, P.nz, p.z, iz, az);
             } else {
-                loc(p.x, C.fa_first[0], C.fa_last[0], C.fa_inv[0], P.nx, ix, ax);
-                loc(p.y, C.fa_first[1], C.fa_last[1], C.fa_inv[1], P.ny, iy, ay);
-                loc(p.z, C.fa_first[2], C.fa_last[2], C.fa_inv[2], P.nz, iz, az);
+                clamp_cell(p.x, C.fa_first[0], C.fa_last[0], C.fa_inv[0], P.nx, at.x, ix, ax);
+                clamp_cell(p.y, C.fa_first[1], C.fa_last[1], C.fa_inv[1], P.ny, at.y, iy, ay);
+                clamp_cell(p.z, C.fa_first[2], C.fa_last[2], C.fa_inv[2], P.nz, at.z, iz, az);
+            }
+            if (!GEN || P.n_terms <= 1) {
+                // the cell's first node by two 32 x 32 -> 64-bit multiply-adds, the
+                // other three rows by one 64-bit add each; the second node of a
+                // row is an offset of the load
+                const uint32_t row = static_cast<uint32_t>(iy) + static_cast<uint32_t>(P.ny) * static_cast<uint32_t>(iz);
+                const uint64_t node = static_cast<uint64_t>(row) * static_cast<uint32_t>(P.nx) + static_cast<uint32_t>(ix);
+                const char* const p00 = reinterpret_cast<const char*>(P.fa_f32) + 16 * node;
+                if (node != cell.node) {
+                    cell.node = node;
+                    if constexpr (!GEN) {
+                        const bool last = ix == P.nx - 2 || iy == P.ny - 2 || iz == P.nz - 2;
+                        cell.index = f3{last ? __builtin_nanf("") : static_cast<float>(ix), static_cast<float>(iy),
+                                        static_cast<float>(iz)};
+                    }
+#pragma unroll
+                    for (int c4 = 0; c4 < 4; ++c4) {
+                        const float4* const q =
+                            reinterpret_cast<const float4*>(p00 + 16 * ((c4 >> 1) * sy + (c4 & 1) * sz));
+                        const float4 lo4 = q[0], hi4 = q[1];
+                        cell.e[c4] = f3{lo4.x, lo4.y, lo4.z};
+                        cell.e[4 + c4] = f3{hi4.x, hi4.y, hi4.z};
+                    }
+                }
             }
         }
-        f3 r{0.0f, 0.0f, 0.0f};
-        const size_t sy = static_cast<size_t>(P.nx), sz = static_cast<size_t>(P.nx) * P.ny;
         if (!GEN || P.n_terms <= 1) {
-            // the cell's first node by two 32 x 32 -> 64-bit multiply-adds, the
-            // other three rows by one 64-bit add each; the second node of a
-            // row is an offset of the load
-            const uint32_t row = static_cast<uint32_t>(iy) + static_cast<uint32_t>(P.ny) * static_cast<uint32_t>(iz);
-            const uint64_t node = static_cast<uint64_t>(row) * static_cast<uint32_t>(P.nx) + static_cast<uint32_t>(ix);
-            const char* const p00 = reinterpret_cast<const char*>(P.fa_f32) + 16 * node;
-            if (!inside && node != cell.node) {
-                cell.node = node;
-                if constexpr (!GEN) {
-                    const bool last = ix == P.nx - 2 || iy == P.ny - 2 || iz == P.nz - 2;
-                    cell.index = f3{last ? __builtin_nanf("") : static_cast<float>(ix), static_cast<float>(iy),
-                                    static_cast<float>(iz)};
-                }
-#pragma unroll
-                for (int c4 = 0; c4 < 4; ++c4) {
-                    const float4* const q = reinterpret_cast<const float4*>(p00 + 16 * ((c4 >> 1) * sy + (c4 & 1) * sz));
-                    const float4 lo4 = q[0], hi4 = q[1];
-                    cell.e[c4] = f3{lo4.x, lo4.y, lo4.z};
-                    cell.e[4 + c4] = f3{hi4.x, hi4.y, hi4.z};
-                }
-            }
 #pragma unroll
             for (int c8 = 0; c8 < 8; ++c8) {
                 const int dx = c8 >> 2, dy = (c8 >> 1) & 1, dzz = c8 & 1;
@@ -240,8 +251,10 @@ __device__ __forceinline__ f3 iso_dir_f32(PhiloxStream& rng) {
 }
 
 // FLOW: the neutrals move with ug (the gas velocity at the ion's position),
-// else with the constant gas velocity.
-template <int COLL, bool FLOW = false>
+// else with the constant gas velocity.  FIXED: the sums of the HSS collision after
+// a push by this integrator with their rounding written out (the field-array
+// kernels, single cloud and batch); -1: the compiler's choice.
+template <int COLL, bool FLOW = false, int FIXED = -1>
 __device__ __forceinline__ bool collide_f32(const StepParams& P, const FastConst& C,
                                             const SpeciesDev& sp, uint32_t sidx, float m,
                                             float inv_m_plus, float lpre, float kbt2_dt_over_m, f3& v,
@@ -321,17 +334,15 @@ __device__ __forceinline__ bool collide_f32(const StepParams& P, const FastConst
         const f3 vn{r1 * fast_cos_rev(u2) + u_gas.x, r1 * fast_sin_rev(u2) + u_gas.y,
                     r2 * fast_cos_rev(u4) + u_gas.z};
         const f3 vrel = v - vn;
-        const float vm2 = dot<float>(vrel, vrel);
-        const float vm = fast_sqrt(vm2);
+        const float vm = fast_sqrt(FIXED < 0 ? dot<float>(vrel, vrel) : speed2_f32<FIXED>(vrel));
         if (vm < (float)kMinRelativeVelocity) return false;
-        // P = 1 - exp(-x), evaluated as -expm1(-x) to keep small x accurate
-        const float x = n_dt * sigma * vm;
-        const float Pc = x < 1e-3f ? x * (1.0f - 0.5f * x * (1.0f - x * (1.0f / 3.0f)))
-                                   : 1.0f - __builtin_amdgcn_exp2f(-x * 1.44269504089f);
+        const float Pc = collision_probability_f32(n_dt * sigma * vm);
         if (rng.uniform_f32() >= Pc) return false;
         const f3 nd = iso_dir_f32(rng);
-        const f3 Vcom = (v * m + vn * C.m_gas) * inv_m_plus;
-        v = Vcom + nd * (vm * C.m_gas * inv_m_plus);
+        // centre of mass velocity + relative velocity times the neutral's share
+        const f3 share = nd * (vm * C.m_gas * inv_m_plus);
+        v = FIXED < 0 ? (v * m + vn * C.m_gas) * inv_m_plus + share
+                      : fma3(fma3(vn, C.m_gas, v * m), inv_m_plus, share);
         return true;
     } else if constexpr (COLL == COLL_DAMPING) {
         if (P.ou_kicks) {

@@ -864,8 +864,9 @@ __device__ __forceinline__ void f32_ion(const StepParams& P, const IonPtrs& S, c
                 uint32_t hits = 0;
                 const f3 ug = FLOW ? gas_velocity_f32(P, C, f3{hi[0], hi[1], hi[2]}) : f3{0.0f, 0.0f, 0.0f};
                 for (int s = 0; s < ns; ++s)
-                    hits += collide_f32<COLL, FLOW>(P, C, sp, sidx, m, inv_m_plus, lp, kbt2_dt_over_m * sub, v, rng,
-                                                    dtc * nrel, C.n_dt * sub * nrel, ug) ? 1u : 0u;
+                    hits += collide_f32<COLL, FLOW, FIELD == FIELD_ARRAY ? INTEG : -1>(
+                                P, C, sp, sidx, m, inv_m_plus, lp, kbt2_dt_over_m * sub, v, rng, dtc * nrel,
+                                C.n_dt * sub * nrel, ug) ? 1u : 0u;
                 if (COLL == COLL_HSS || COLL == COLL_HSS_MIX) {
                     if (hits) {
                         // a collision replaces the velocity: restart its compensation

@@ -271,7 +271,7 @@ def pinned_runs(kind):
     return out
 
 
-@pytest.mark.parametrize("kind", ["surrogate"])
+@pytest.mark.parametrize("kind", ["surrogate", "field_array"])
 def test_fp32_results_stay_the_same(kind):
     """The rounding of these kernels is written out, so that a change around it
     leaves the results as they were, bit for bit (tests/golden, made on an MI355X;
@@ -279,3 +279,41 @@ def test_fp32_results_stay_the_same(kind):
     with np.load(os.path.join(os.path.dirname(__file__), "golden", f"fp32_{kind}.npz"), allow_pickle=False) as want:
         for name, got in pinned_runs(kind).items():
             np.testing.assert_array_equal(got, want[name], err_msg=name)
+
+
+def test_field_array_cell_follows_from_the_position():
+    """Positions within rounding below a cell's face, whose cell coordinate as a
+    rounded product lies on the face: the next cell's, whether an ion is there
+    from the start or comes there from the cell before, which it has kept.  The
+    field is zero on the kept cell's nodes and 1 MV/m on the next one along x, so
+    that an ion with the wrong cell feels no force at all.  Boris in powers of two:
+    the second step begins exactly at the position."""
+    nx, spacing, first = 96, 1e-2 / 95, -5e-3
+    f32 = np.float32
+    x0, inv = f32(first), f32(1.0 / spacing)
+    p2 = []
+    for i in range(2, nx - 2, 3):   # faces between a zero cell and one that ends at a charged node
+        p = f32(first + i * spacing)
+        for _ in range(8):
+            p = np.nextafter(p, f32(-1.0))
+        for _ in range(16):
+            p = np.nextafter(p, f32(1.0))
+            d = f32(p - x0)
+            if f32(d * inv) >= i and float(d) * float(inv) < i and float(p) - 2.0**-14 == f32(p - f32(2.0**-14)):
+                p2.append(p)
+    assert len(p2) >= 8
+    E = np.zeros((5, 5, nx, 3), np.float32)
+    E[:, :, 3::3, 0] = 1e6
+    n = len(p2)
+    w = W.field_array_workload(n=1, grid=(2, 2, 2), seed=2)
+    w["physics"] = W.physics(_abi.INTEGRATOR_BORIS, _abi.COLLISION_NONE, precision=_abi.PRECISION_FP32_KAHAN, seed=2)
+    ens = W.gaussian_cloud(2 * n, 100.0, 1e-6, center=(0.0, 0.0, 20e-3), seed=6)
+    ens.vx[:] = ens.vy[:] = ens.vz[:] = 0.0
+    ens.x[:n] = ens.x[n:] = np.array(p2, np.float64)
+    ens.x[n:] -= 2.0**-14
+    ens.vx[n:] = 2.0**16
+    w.update(ensemble=ens, field=(E, (first, -5e-3, 0.0), (spacing, 2.5e-3, 1.25e-2)), dt=2.0**-30)
+    gpu_run(w, ens, 2)
+    there, coming = ens.vx[:n] / 2.0, ens.vx[n:] - 2.0**16   # two steps at the position, and one
+    assert (np.abs(there) > 1e-5).all()
+    np.testing.assert_allclose(coming, there, rtol=1e-4)
