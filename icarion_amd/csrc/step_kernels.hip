@@ -14,11 +14,19 @@
 // the reference's per-ion result.  Per-step wave-uniform values (engine time,
 // RF coefficient) come from a table read with scalar loads.  Counters are
 // reduced per wavefront before one atomic per wave.
+#include "launch_rules.hpp"
 #include "step_device.hpp"
 #include "step_device_f32.hpp"
 #include "surrogate.hpp"
 
 namespace icarion {
+
+// An index whose addresses are formed where it is used: hoisted out of the step
+// loop, the addresses of rare events take registers all along.
+__device__ __forceinline__ uint32_t here(uint32_t i) {
+    asm volatile("" : "+v"(i));
+    return i;
+}
 
 // The per-ion factor of the damping coefficient (DampingForce.cpp:150-177 / :269-271).
 __device__ __forceinline__ double damping_factor_f64(const StepParams& P, const SpeciesDev& sp, double m, double q) {
@@ -362,10 +370,13 @@ __global__ void __launch_bounds__(256) step_f64_quad_kernel(const StepParams P, 
 // What bounds it: FP64 issue in the atom loops and the chain of one collision.
 // Done once per collision, the orientation, the draws and the reflection were
 // two thirds of the instructions; a row of atoms was waited for at a time; and
-// 64 ions on every wavefront left SIMDs idle below 131,072 ions (launch_step
-// picks ions_per_wave).  Before and now: 701 ions x 200 steps 55.5 and 2.0 ms,
-// 9001 x 200 57.7 and 7.5 ms, 40,000 x 300 93 and 32 ms, 250,000 x 40 33.9 and
-// 26.2 ms.
+// 64 ions on every wavefront left SIMDs idle below 131,072 ions
+// (ehss_ions_per_wave).  Two wavefronts per SIMD hide the chain: birth, death and
+// arrival times stay in memory until their event and the table entry is read where
+// it is used, which leaves 256 registers and 4 spilled ones (with all of them in
+// registers 282, and one wavefront).  First, with one wavefront, and now:
+// 701 ions x 200 steps 56.0, 1.4 and 1.4 ms, 9001 x 200 59.6, 6.2 and 4.5 ms,
+// 40,000 x 100 33.3, 11.4 and 6.9 ms, 250,000 x 40 33.3, 25.2 and 16.2 ms.
 
 __device__ __forceinline__ uint32_t readlane_u32(uint32_t x, int lane) {
     return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), lane));
@@ -443,7 +454,8 @@ struct EhssDraws {
 };
 
 template <int INTEG, int FIELD>
-__global__ void __launch_bounds__(256) step_f64_ehss_kernel(const StepParams P, const IonPtrs S) {
+__global__ void __launch_bounds__(256, ehss_waves_per_simd(INTEG, FIELD == FIELD_ARRAY, FIELD == FIELD_ARRAY_X))
+    step_f64_ehss_kernel(const StepParams P, const IonPtrs S) {
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t G = P.ions_per_wave;
@@ -454,7 +466,7 @@ __global__ void __launch_bounds__(256) step_f64_ehss_kernel(const StepParams P, 
     const uint32_t i = first + lane;
     const bool have = lane < G && i < P.n_ions;
     d3 pos{0.0, 0.0, 0.0}, vel{0.0, 0.0, 0.0};
-    double m = 1.0, q = 0.0, birth = -INFINITY, death = -1.0, arrival = NAN;
+    double m = 1.0, q = 0.0;
     uint32_t sidx = 0, nc = 0;
     bool active = false, born = true;
     if (have) {
@@ -466,9 +478,6 @@ __global__ void __launch_bounds__(256) step_f64_ehss_kernel(const StepParams P, 
         const uint8_t flags = S.flags[i];
         active = flags & 1;
         born = (flags >> 1) & 1;
-        birth = S.birth ? S.birth[i] : -INFINITY;
-        death = S.death[i];
-        arrival = S.arrival[i];
         nc = S.ncoll[i];
     }
     const SpeciesDev sp = P.species[sidx];
@@ -479,18 +488,15 @@ __global__ void __launch_bounds__(256) step_f64_ehss_kernel(const StepParams P, 
     const double half_dt = dt * 0.5;
     __shared__ WaveAtoms s_atoms[4];   // 256 threads = 4 wavefronts
     WaveAtoms& lds = s_atoms[threadIdx.x >> 6];
-    // the next step's table entry is loaded one step ahead
-    StepEntry te_next = P.n_steps ? P.table[0] : StepEntry{};
     for (uint32_t k = 0; k < P.n_steps; ++k) {
         // unborn ions wait for their birth, live ones step; none left: the
         // whole wavefront leaves together
         if (__ballot(have && (!born || active)) == 0ull) break;
-        const StepEntry te = te_next;
-        if (k + 1 < P.n_steps) te_next = P.table[k + 1];
+        const StepEntry& te = P.table[k];
         const double t = te.t;
         bool live = false;
         if (have) {
-            if (!born && t >= birth) {
+            if (!born && (!S.birth || t >= S.birth[here(i)])) {
                 born = true;
                 active = true;
                 checked = false;
@@ -498,7 +504,7 @@ __global__ void __launch_bounds__(256) step_f64_ehss_kernel(const StepParams P, 
             if (born && active) {
                 if (!checked && !contains_f64(P, pos)) {
                     active = false;
-                    death = t;
+                    S.death[here(i)] = t;
                 } else {
                     live = true;
                 }
@@ -732,19 +738,19 @@ __global__ void __launch_bounds__(256) step_f64_ehss_kernel(const StepParams P, 
             }
         }
         if (live) {
-            if (P.detect && isnan(arrival)) {
-                if (z_before < P.det_z && pos.z >= P.det_z)
-                    arrival = t + dt * (P.det_z - z_before) / (pos.z - z_before);
+            if (P.detect && z_before < P.det_z && pos.z >= P.det_z) {
+                double& arrival = S.arrival[here(i)];
+                if (isnan(arrival)) arrival = t + dt * (P.det_z - z_before) / (pos.z - z_before);
             }
             if (!contains_f64(P, pos)) {
                 active = false;
-                death = t;
+                S.death[here(i)] = t;
             } else {
                 checked = true;
                 if (!(isfinite(pos.x) && isfinite(pos.y) && isfinite(pos.z) && isfinite(vel.x) &&
                       isfinite(vel.y) && isfinite(vel.z))) {
                     active = false;
-                    death = t;
+                    S.death[here(i)] = t;
                 }
             }
         }
@@ -753,8 +759,6 @@ __global__ void __launch_bounds__(256) step_f64_ehss_kernel(const StepParams P, 
         S.x[i] = pos.x; S.y[i] = pos.y; S.z[i] = pos.z;
         S.vx[i] = vel.x; S.vy[i] = vel.y; S.vz[i] = vel.z;
         S.flags[i] = static_cast<uint8_t>((active ? 1 : 0) | (born ? 2 : 0));
-        S.death[i] = death;
-        S.arrival[i] = arrival;
         S.ncoll[i] = nc;
     }
     add_counters(P, pushed, ncoll_launch);
@@ -935,13 +939,6 @@ __global__ void __launch_bounds__(256) step_f32_kernel(const StepParams P, const
 // instructions see every lane they need.  One ion per lane over P.n_steps
 // steps; with mlp_group_eval every lane of the workgroup calls it with the same
 // P.n_steps (lanes with i >= P.n_ions are carried along masked).
-// An index whose addresses are formed where it is used: hoisted out of the step
-// loop, the addresses of rare events take registers all along.
-__device__ __forceinline__ uint32_t here(uint32_t i) {
-    asm volatile("" : "+v"(i));
-    return i;
-}
-
 template <int INTEG, int FIELD, bool AHEAD, class MlpEval>
 __device__ __forceinline__ void surr_ion(const StepParams& P, const IonPtrs& S, uint32_t i,
                                          MlpEval&& mlp_eval, uint32_t& pushed, uint32_t& ncoll_launch) {
@@ -1533,17 +1530,6 @@ hipError_t launch_quad(KernelFn fn, const StepParams& P, const IonPtrs& S, hipSt
     return hipGetLastError();
 }
 
-// Ions per wavefront of the geometry EHSS kernel: two wavefronts per SIMD fit
-// (registers and LDS), 2048 on the chip.  A wavefront works through its
-// colliding ions one after another, so the ions are spread evenly over the
-// least number of full rounds of 2048 wavefronts.
-uint32_t ehss_ions_per_wave(uint32_t n_ions) {
-    const uint32_t slots = 2048;
-    const uint32_t rounds = (n_ions + 64 * slots - 1) / (64 * slots);
-    const uint32_t g = (n_ions + rounds * slots - 1) / (rounds * slots);
-    return g < 1 ? 1 : g > 64 ? 64 : g;
-}
-
 // Ions per wavefront of the surrogate kernel: up to 131,072 ions one or two
 // wavefronts per SIMD, evenly filled (a step lasts as long as the workgroup's
 // chain, which is shorter with fewer colliding ions: 30,000 ions x 1000 steps
@@ -1580,7 +1566,9 @@ hipError_t launch_step(int integrator, int field, int coll, int precision, int s
     static_assert(kSurrogateBlock == 256, "four wavefronts per workgroup");
     uint32_t grid = (P.n_ions + block - 1) / block;
     if (surrogate || coll == COLL_EHSS) {
-        P.ions_per_wave = surrogate ? surrogate_ions_per_wave(P.n_ions) : ehss_ions_per_wave(P.n_ions);
+        P.ions_per_wave = surrogate ? surrogate_ions_per_wave(P.n_ions)
+                                    : ehss_ions_per_wave(P.n_ions, ehss_waves_per_simd(integrator, field == FIELD_ARRAY,
+                                                                                       field == FIELD_ARRAY_X));
         block = 256;
         const uint32_t per_block = 4 * P.ions_per_wave;
         grid = (P.n_ions + per_block - 1) / per_block;

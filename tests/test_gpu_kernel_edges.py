@@ -40,8 +40,11 @@ COUNTS = (1, 2, 63, 64, 65, 128, 449, 511, 512, 513, 700)
 SPREAD = (0.0, 4e-9, 8e-10, 8e-10, 8e-10, 8e-10, 1.2e-9, 1.2e-9, 1.2e-9, 1.2e-9, 1.2e-9)
 
 
-@pytest.mark.parametrize("n", [1, 63, 2047, 2049, 5000])
-def test_geometry_ehss_rows_and_wavefronts(oracle, n):
+@pytest.mark.parametrize("n,steps", [(1, 25), (63, 25), (2047, 25), (2049, 25), (5000, 25),
+                                     # two and three passes of draws ahead (22 and 35 ions per
+                                     # wavefront), and a second round of wavefronts
+                                     (45001, 5), (70001, 4), (131073, 3)])
+def test_geometry_ehss_rows_and_wavefronts(oracle, n, steps):
     atoms, species = cluster_table(COUNTS, SPREAD, seed=5)
     w = W.ehss_surrogate_workload(n=1, seed=17, precision=_abi.PRECISION_FP64, ehss_mode=_abi.EHSS_GEOMETRY)
     rng = np.random.default_rng(n)
@@ -51,8 +54,8 @@ def test_geometry_ehss_rows_and_wavefronts(oracle, n):
     ens.species[:] = which
     w.update(species=species, atoms=atoms, ensemble=ens)
     g, o = ens.copy(), ens.copy()
-    sg = gpu_run(w, g, 25)
-    so = oracle_run(oracle, w, o, 25)
+    sg = gpu_run(w, g, steps)
+    so = oracle_run(oracle, w, o, steps)
     assert so.collisions > 0 or n < 63
     assert sg.collisions == so.collisions
     assert compare_ions(g, o, rtol=1e-9).all()
