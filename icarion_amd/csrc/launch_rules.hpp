@@ -1,5 +1,5 @@
-// launch_rules.hpp - how the geometry EHSS kernel spreads a cloud over the chip's 1024
-// SIMDs (host code, without HIP).
+// launch_rules.hpp - how the EHSS and surrogate kernels spread a cloud over the
+// chip's 1024 SIMDs (host code, without HIP).
 #pragma once
 
 #include <cstdint>
@@ -24,6 +24,23 @@ inline uint32_t ehss_ions_per_wave(uint32_t n_ions, uint32_t waves_per_simd) {
     if (rounds == 0) return 1;
     const uint64_t g = (n_ions + rounds * slots - 1) / (rounds * slots);
     return g > 64 ? 64u : static_cast<uint32_t>(g);
+}
+
+// The surrogate kernel's instantiation for large clouds (four wavefronts per SIMD
+// instead of three): from where the ions are more than two full wavefronts per SIMD.
+constexpr uint32_t kSurrogateLargeIons = 64 * 2 * kSimds;
+inline bool surrogate_large(uint32_t n_ions) { return n_ions > kSurrogateLargeIons; }
+
+// Ions per wavefront of the surrogate kernel: up to 131,072 ions one or two
+// wavefronts per SIMD, evenly filled (a step lasts as long as the workgroup's
+// chain, which is shorter with fewer colliding ions: 30,000 ions x 1000 steps
+// 5.7 ms with 64 per wavefront, 4.0 ms spread); above that full wavefronts, for
+// full MLP blocks.
+inline uint32_t surrogate_ions_per_wave(uint32_t n_ions) {
+    if (surrogate_large(n_ions)) return 64;
+    const uint32_t rounds = n_ions > 64 * kSimds ? 2 : 1;
+    const uint32_t g = (n_ions + rounds * kSimds - 1) / (rounds * kSimds);
+    return g < 1 ? 1 : g;
 }
 
 }  // namespace icarion

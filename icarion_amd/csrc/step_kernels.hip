@@ -1089,10 +1089,10 @@ __device__ __forceinline__ void surr_ion(const StepParams& P, const IonPtrs& S, 
     }
 }
 
-// OCC: wavefronts per SIMD.  Four (128 registers, 40 KB of LDS per workgroup)
-// run a large cloud faster, three a small one, whose one or two wavefronts per
-// SIMD gain from the registers instead: 1M ions x 4000 steps 151.8 and 141 ms,
-// 3001 x 2000 6.9 and 7.8 ms (three and four).
+// OCC: wavefronts per SIMD.  Four (128 registers and 4 spilled ones, 40 KB of LDS
+// per workgroup) run a large cloud faster, three a small one, whose one or two
+// wavefronts per SIMD gain from the registers instead (surrogate_large): 1M ions x
+// 4000 steps 151.8 and 134 ms, 3001 x 2000 6.9 and 7.8 ms (three and four).
 template <int INTEG, int FIELD, int OCC>
 __global__ void __launch_bounds__(kSurrogateBlock, OCC) step_surrogate_kernel(const StepParams P, const IonPtrs S) {
     __shared__ uint4 mlp_lds[kPackBytes / 16];
@@ -1496,20 +1496,17 @@ KernelFn pick_field(int field, int coll, int precision, bool sub) {
     }
 }
 
-template <int I, int OCC>
-KernelFn pick_surrogate_occ(int field) {
-    switch (field) {
-        case FIELD_ORBITRAP: return step_surrogate_kernel<I, FIELD_ORBITRAP, OCC>;
-        case FIELD_ARRAY: return step_surrogate_kernel<I, FIELD_ARRAY, OCC>;
-        case FIELD_ARRAY_X: return step_surrogate_kernel<I, FIELD_ARRAY_X, OCC>;
-        default: return step_surrogate_kernel<I, FIELD_LINEAR, OCC>;
-    }
-}
+// large: four wavefronts per SIMD; the field-array kernels, which keep a cell's
+// corners in registers, have three for every cloud.
 template <int I>
 KernelFn pick_surrogate(int field, bool large) {
-    // (the field-array kernels keep a cell's corners in registers: three)
-    const bool four = large && field != FIELD_ARRAY && field != FIELD_ARRAY_X;
-    return four ? pick_surrogate_occ<I, 4>(field) : pick_surrogate_occ<I, 3>(field);
+    switch (field) {
+        case FIELD_ORBITRAP:
+            return large ? step_surrogate_kernel<I, FIELD_ORBITRAP, 4> : step_surrogate_kernel<I, FIELD_ORBITRAP, 3>;
+        case FIELD_ARRAY: return step_surrogate_kernel<I, FIELD_ARRAY, 3>;
+        case FIELD_ARRAY_X: return step_surrogate_kernel<I, FIELD_ARRAY_X, 3>;
+        default: return large ? step_surrogate_kernel<I, FIELD_LINEAR, 4> : step_surrogate_kernel<I, FIELD_LINEAR, 3>;
+    }
 }
 
 // The four-lanes-per-ion kernel of a combination, or null.
@@ -1530,19 +1527,6 @@ hipError_t launch_quad(KernelFn fn, const StepParams& P, const IonPtrs& S, hipSt
     return hipGetLastError();
 }
 
-// Ions per wavefront of the surrogate kernel: up to 131,072 ions one or two
-// wavefronts per SIMD, evenly filled (a step lasts as long as the workgroup's
-// chain, which is shorter with fewer colliding ions: 30,000 ions x 1000 steps
-// 5.7 ms with 64 per wavefront, 4.0 ms spread); above that full wavefronts, for
-// full MLP blocks.
-uint32_t surrogate_ions_per_wave(uint32_t n_ions) {
-    const uint32_t waves = 1024;
-    const uint32_t rounds = (n_ions + 64 * waves - 1) / (64 * waves);
-    if (rounds > 2) return 64;
-    const uint32_t g = (n_ions + rounds * waves - 1) / (rounds * waves);
-    return g < 1 ? 1 : g;
-}
-
 // Returns hipSuccess, or hipErrorInvalidValue when the combination has no
 // kernel (the host maps that to ICARION_ERR_UNSUPPORTED).
 hipError_t launch_step(int integrator, int field, int coll, int precision, int surrogate,
@@ -1550,7 +1534,7 @@ hipError_t launch_step(int integrator, int field, int coll, int precision, int s
     StepParams P = params;
     KernelFn fn;
     if (surrogate) {
-        const bool large = surrogate_ions_per_wave(P.n_ions) == 64;
+        const bool large = surrogate_large(P.n_ions);
         fn = integrator == 1 ? pick_surrogate<1>(field, large) : pick_surrogate<0>(field, large);
     } else {
         // the extended instantiation: collision substeps or a parabolic flow
