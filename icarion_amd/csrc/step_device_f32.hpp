@@ -71,7 +71,7 @@ struct CellF32 {
 // c: the stage's RF coefficient (analytic fields) or the stage time (field
 // arrays, always in FP64); T: float where the caller holds rounded values.
 template <int FIELD, class T>
-__device__ __forceinline__ f3 field_f32(const StepParams& P, const FastConst& C, f3 p, T c, T ez, CellF32& cell) {
+__device__ __forceinline__ f3 field_f32(const StepParams& P, const FastConst& C, f3 p, T c, T ez, CellF32& kept) {
     if constexpr (FIELD == FIELD_LINEAR) {
         const float c_rf = (float)c;
         f3 E{0.0f, 0.0f, (float)ez};
@@ -128,6 +128,12 @@ __device__ __forceinline__ f3 field_f32(const StepParams& P, const FastConst& C,
             }
         };
         constexpr bool GEN = FIELD == FIELD_ARRAY_X;
+        // non-uniform axes and several terms gather the corners each time: the
+        // registers of a kept cell cost their kernels a wavefront per SIMD (300,000
+        // ions x 150 RK4 steps, one term: 4.7 ms with and 4.3 ms without; three
+        // terms, which read other nodes each time: 8.8 and 7.6 ms)
+        CellF32 fresh;
+        CellF32& cell = GEN ? fresh : kept;
         int ix = 0, iy = 0, iz = 0;
         float ax, ay, az;
         // Still in the kept cell?  The cell follows from the position alone, not from
