@@ -202,8 +202,10 @@ struct StateSlab {
             at += (width * n + 255) / 256 * 256;
         }
         off[kSlabArrays] = at;
-        if (dev.n < at) dev.resize(at);
-        if (host_cap < at) {
+        // kept from call to call while the need stays within a factor of four
+        // (repeated uploads allocate nothing), given back when it falls below
+        if (dev.n < at || dev.n / 4 > at) dev.resize(at);
+        if (host_cap < at || host_cap / 4 > at) {
             host.reset(new unsigned char[at]);   // pages are touched only where they are used
             host_cap = at;
         }
@@ -1893,6 +1895,14 @@ void do_upload(icarion_gpu* h, const icarion_ion_soa* ions, bool sync = true) {
     StateSlab& L = h->slab;
     h->have_state = false;   // until the new state is in place
     L.layout(n, true, h->has_birth);
+    // what a much larger cloud left behind
+    if (h->ord.n / 4 > n) {
+        h->ord.release(); h->ord_keys_a.release(); h->ord_keys_b.release(); h->ord_idx.release();
+        h->ord_temp.release();
+    }
+    if (h->r_err.n / 4 > n) {
+        h->r_err.release(); h->r_k1x.release(); h->r_k1y.release(); h->r_k1z.release(); h->r_fsal.release();
+    }
     h->x.view(L.dev_at(kX), n); h->y.view(L.dev_at(kY), n); h->z.view(L.dev_at(kZ), n);
     h->vx.view(L.dev_at(kVx), n); h->vy.view(L.dev_at(kVy), n); h->vz.view(L.dev_at(kVz), n);
     h->death.view(L.dev_at(kDeath), n); h->arrival.view(L.dev_at(kArrival), n);
