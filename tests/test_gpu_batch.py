@@ -1,8 +1,9 @@
 """Batched clouds in one persistent launch (icarion_gpu_batch_*): each cloud's
-result must be the one a handle of its own gives (same kernel bodies, same
-random streams) - to 1e-9 relative, the per-step bar of the single-cloud
-parity tests, since the batch kernel is a separate function the compiler
-contracts on its own (differences seen: ~1e-13) - and bit for bit the same
+result must be the one a handle of its own gives (same random streams and
+arithmetic) - to 1e-9 relative, the per-step bar of the single-cloud parity
+tests, since the batch kernel is a separate function the compiler contracts on
+its own, and FP64 clouds of up to 49,152 ions in a linear field run four lanes
+per ion on a handle but one in the batch (differences seen: ~1e-13) - and bit for bit the same
 whatever the tile / launch shape; the autotuner only picks among launch
 shapes.  Single-cloud runs are pinned against the oracle
 (test_gpu_parity.py), which carries that parity over to the batch."""

@@ -183,6 +183,51 @@ def test_lost_ions_leave_the_launches(precision):
         assert np.array_equal(getattr(a, f), getattr(b, f)), f
 
 
+@pytest.mark.parametrize("kind", ["hss", "mixture", "snapshots"])
+@pytest.mark.parametrize("precision", [_abi.PRECISION_FP64, _abi.PRECISION_FP32_KAHAN])
+def test_dropped_lanes_leave_no_trace(precision, kind):
+    """Half of the ions are outside the domain at the start, so that the first
+    count drops their lanes, and others arrive and leave later.  The same ions in
+    a cloud of one less than the rule's size run with every lane in place, in the
+    same launches: bit for bit the same, the snapshots during the run too."""
+    from icarion_amd import gpu
+    n = 262144
+    if kind == "mixture":
+        w = W.ims_mixture_workload(n=n, seed=12, precision=precision)
+    else:
+        w = W.ims_hss_workload(n=n, seed=12, precision=precision)
+    ens = w["ensemble"]
+    r = np.hypot(ens.x, ens.y)
+    w["domain"].radius_m = float(np.median(r))
+    w["domain"].detector_z_m = float(np.quantile(ens.z, 0.5)) + 1e-9    # crossed by some hundred ions
+    out = []
+    for size in (n, n - 1):
+        e = ens.subset(np.arange(size))
+        with gpu.Handle(steps_per_launch=40) as h:
+            h.set_domain(w["domain"], w["physics"])
+            h.set_species(w["species"])
+            if kind == "mixture":
+                h.set_gas_mixture(*w["mixture"])
+            h.upload_state(e)
+            if kind == "snapshots":
+                snaps, _, st = h.step_snapshots(0.0, w["dt"], 400, 70 * w["dt"])
+                assert len(snaps) >= 5
+            else:
+                snaps, st = [], h.step(0.0, w["dt"], 400)
+            h.download_state(e)
+        m = n - 1
+        assert st.alive == (e.active != 0).sum() < 0.55 * size and st.collisions == e.n_collisions.sum()
+        out.append((e.subset(np.arange(m)), [(x["step"], x["positions"][:m], x["velocities"][:m], x["flags"][:m])
+                                              for x in snaps]))
+    (a, sa), (b, sb) = out
+    assert np.isfinite(a.arrival_time_s).sum() > 100 and a.n_collisions.max() > 0
+    for f in ("x", "y", "z", "vx", "vy", "vz", "death_time_s", "arrival_time_s", "active", "born", "n_collisions"):
+        np.testing.assert_array_equal(getattr(a, f), getattr(b, f), err_msg=f)
+    assert len(sa) == len(sb)
+    for x, y in zip(sa, sb):
+        assert x[0] == y[0] and all(np.array_equal(p, q) for p, q in zip(x[1:], y[1:]))
+
+
 def test_all_ions_lost(precision=_abi.PRECISION_FP32_KAHAN):
     """Launches after the last ion is gone have nothing to run."""
     w = W.quadrupole_workload(n=262144, seed=8, precision=precision)
