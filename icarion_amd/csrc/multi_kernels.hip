@@ -8,7 +8,7 @@
 // domain lookup after the push starts with the domain's own span.  What bounds it
 // is the latency of the step's chain (100,000 ions are 1.5 wavefronts a SIMD).
 // With a record per lane every parameter was a vector load, the lookup a chain of
-// five dependent ones: 100,000 ions x 4000 steps in FP32 took 13.9 ms, now 12.8.
+// five dependent ones: 100,000 ions x 4000 steps in FP32 took 13.9 ms, then 12.6.
 // Per step and ion, the engine's domain logic (SimulationEngineLifecycle.cpp:
 // 72-195) around the same push and collision bodies as the single-domain kernels:
 //   prepare:  birth; the domain = DomainManager::find_domain_index of the

@@ -359,8 +359,9 @@ __device__ d3 ehss_f64(const StepParams& P, d3 v_ion, d3 v_n, double mi, double 
 }
 
 // The HSS collision's sums with the rounding written out: which product of a sum
-// of two goes into the fma is else the compiler's choice in each kernel, and a
-// batch's ions, one to a lane, have to equal a single cloud's, four lanes each.
+// of two goes into the fma is else the compiler's choice in each kernel, and with
+// it the batch's ions, one to a lane, differed from a single cloud's, four lanes
+// each, past what the pushes' rounding makes.
 __device__ __forceinline__ double speed_f64(d3 v) { return sqrt(fma(v.z, v.z, fma(v.y, v.y, v.x * v.x))); }
 
 // A component of the velocity after hss_collision: the centre of mass's plus the

@@ -179,8 +179,9 @@ __global__ void __launch_bounds__(256, (INTEG == 1 && FIELD == FIELD_ARRAY_X) ? 
 // ======================= FP64, four lanes per ion ============================
 //
 // The step of f64_ion for the analytic linear fields (no magnetic field) with
-// one ion on four lanes: lanes 0-2 hold the x, y and z components, lane 3
-// repeats z.  The draws of a step are four or five Philox blocks, three or four
+// one ion on four lanes: lanes 0-2 hold the x, y and z components.  Lane 3 starts
+// as z and serves the draws alone: after a collision its position and velocity
+// mean nothing, and nothing reads them.  The draws of a step are four or five Philox blocks, three or four
 // Box-Muller transforms and a direction: lane c takes block c, so one block, one
 // logarithm, one sine and cosine per lane replace them (lane 3 draws the
 // collision test and the direction).  Scalars of an ion (speeds, tests) are
@@ -1120,8 +1121,10 @@ __global__ void __launch_bounds__(kSurrogateBlock, OCC) step_surrogate_kernel(co
 // A fixed pool of workgroups pulls tiles from a queue until it is empty; the
 // host orders the tiles longest first, so the long clouds start first and the
 // short ones fill in at the end.  Every workgroup leaves the loop once the
-// queue index passes the tile count.  Each tile runs the same per-ion body as
-// the single-cloud kernels, so a cloud's result does not depend on the batch.
+// queue index passes the tile count.  Each tile runs the per-ion body of the
+// single-cloud kernels (f64_ion, f32_ion): a cloud's ions take the same course as
+// on a handle of their own, to rounding, where the compiler fuses other products,
+// or where the handle runs four lanes per ion (step_f64_quad_kernel).
 
 template <int PREC, bool SUB, int I, int F, int Cc>
 __device__ __forceinline__ void batch_ion(const StepParams& P, const IonPtrs& S, uint32_t i,
