@@ -163,7 +163,7 @@ __device__ __forceinline__ double log_unit(double u) {
     const double ed = static_cast<double>(e);
     // 2 s = f - s f; ln 2 in two parts, the first times e exact
     const double t = s * (f - 2.0 * (z * horner(pa, z)));
-    return fma(ed, 0.6931471805598903, f - fma(ed, -5.497923018708371e-14, t));
+    return fma(ed, 0.6931471805598903, f - fma(ed, -5.497924164543644e-14, t));
 }
 
 // Per-(ion, step) stream, counter = (block, ion, step_lo, step_hi), key =
