@@ -63,8 +63,9 @@ FLOPS_PER_ION_STEP = {"fp64": 86, "fp32": 122}
 EHSS_FLOPS_STEP = 115
 # HBM bytes per ion per launch of step_surrogate_kernel, measured with rocprofv3
 # FETCH_SIZE / WRITE_SIZE (calibrated on a 1 GiB copy) at 1M ions x 2000 steps:
-# 141.1 MB read + 70.0 MB written (state round trip + each ion's species row).
-EHSS_TRAFFIC_BYTES_PER_ION_LAUNCH = 211.1
+# 130.0 MB read + 67.4 MB written (the state, each ion's species row; event times
+# only where an event falls).
+EHSS_TRAFFIC_BYTES_PER_ION_LAUNCH = 197.4
 EHSS_FLOPS_COLLISION = 2 * (8 * 128 + 128 * 128 + 128 * 3) + 2 * 128 + 2 * 128 + 3 + 60
 # Field-array FP32 kernel (RK4 + trilinear + HSS), per ion-step: per stage the
 # cell location 9, corner weights 19, 8 corners x 3 components FMA 48, q/m 3
@@ -73,7 +74,7 @@ EHSS_FLOPS_COLLISION = 2 * (8 * 128 + 128 * 128 + 128 * 3) + 2 * 128 + 2 * 128 +
 FA_FLOPS_PER_ION_STEP = 476
 # HBM bytes per ion-step of that kernel in grid-brick order (rocprofv3
 # FETCH_SIZE + WRITE_SIZE, copy-calibrated, 4M ions x 2000 steps)
-FA_TRAFFIC_BYTES_PER_ION_STEP = 1.06
+FA_TRAFFIC_BYTES_PER_ION_STEP = 1.08
 
 
 def parse():
@@ -361,7 +362,7 @@ def bench_ehss(args):
             "unit": "TFLOP/s", "frac": achieved / MI355X_PEAK_BF16_TFLOPS,
             "traffic": EHSS_TRAFFIC_BYTES_PER_ION_LAUNCH * args.ions,
             "traffic_source": "rocprofv3 FETCH_SIZE + WRITE_SIZE per launch, copy-calibrated "
-                              "(profiles/step_surrogate_kernel_ehss_he_20td_1M.md)",
+                              "(profiles/step_kernels_cases.md)",
             "kernel": "step_surrogate_kernel<RK4, linear field>",
             "avg_launch_ms": avg_launch_s * 1e3, "launches": launches,
             "flops_per_ion_step": EHSS_FLOPS_STEP,
@@ -733,7 +734,7 @@ def bench_field_array(args):
     avg = fs.device_ms * 1e-3 / launches
     # the launches run in grid-brick order, so the corner gathers (4 stages x 8
     # corners x 16 B per ion-step) are served by the caches: rocprofv3 counts
-    # 1.06 B of HBM traffic per ion-step (FETCH_SIZE + WRITE_SIZE, copy-
+    # 1.08 B of HBM traffic per ion-step (FETCH_SIZE + WRITE_SIZE, copy-
     # calibrated) and 99 % L2 hits; the kernel is bound by vector issue, priced
     # against the FP32 vector peak
     tflops = FA_FLOPS_PER_ION_STEP * fs.ion_steps / launches / avg / 1e12
