@@ -26,15 +26,22 @@ constexpr double kGeomEpsilon = 1e-12;
 constexpr double kMinVoltage = 1e-12;
 
 // Keeps a wave-uniform branch a branch: without it the compiler computes both
-// sides in every step and selects.  A unit whose uniform records lie in memory
-// defines KEEP_BRANCH_READS_ONLY: its branches are held by a scheduling barrier that
-// nothing is bound by, since an asm statement counts as a write to memory and takes
-// the scalar loads away from every record read after it.
+// sides in every step and selects.  MEM: the kernel's uniform records lie in memory
+// (the general field arrays' axes and terms; everything in a unit that defines
+// KEEP_BRANCH_READS_ONLY): its branches are held by a scheduling barrier that nothing
+// is bound by, since an asm statement counts as a write to memory and takes the
+// scalar loads, and the loop's own constants, away from every record read after it
+// (RK4 steps of 300,000 ions in a field of three terms took 6 % longer).
 #ifdef KEEP_BRANCH_READS_ONLY
-__device__ __forceinline__ void keep_branch() { __builtin_amdgcn_sched_barrier(0x7ff); }
+constexpr bool kRecordsInMemory = true;
 #else
-__device__ __forceinline__ void keep_branch() { asm volatile(""); }
+constexpr bool kRecordsInMemory = false;
 #endif
+template <bool MEM = kRecordsInMemory>
+__device__ __forceinline__ void keep_branch() {
+    if constexpr (MEM) __builtin_amdgcn_sched_barrier(0x7ff);
+    else asm volatile("");
+}
 
 template <typename T>
 struct vec3 {

@@ -13,10 +13,11 @@ namespace icarion {
 
 using d3 = vec3<double>;
 
+template <bool MEM = kRecordsInMemory>
 __device__ __forceinline__ bool contains_f64(const StepParams& P, d3 p) {
     d3 l{p.x - P.origin[0], p.y - P.origin[1], p.z - P.origin[2]};
     if (!P.rot_identity) {
-        keep_branch();
+        keep_branch<MEM>();
         l = mat_mul(P.g2l, l);
     }
     if (P.instrument == 3) {

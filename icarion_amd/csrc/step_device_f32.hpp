@@ -220,12 +220,13 @@ __device__ __forceinline__ f3 field_f32(const StepParams& P, const FastConst& C,
 
 // Domain containment in FP32 (same predicates as contains_f64; the FP32
 // position is good to ~1e-7 relative, far finer than any domain feature).
+template <bool MEM = kRecordsInMemory>
 __device__ __forceinline__ bool contains_f32(const StepParams& P, const FastConst& C, float px,
                                              float py, float pz) {
     const f3 s{px - C.ox, py - C.oy, pz - C.oz};
     f3 l = s;
     if (!P.rot_identity) {
-        keep_branch();
+        keep_branch<MEM>();
         l = mat_mul(C.g2l, s);
     }
     const float r2 = fmaf(l.x, l.x, l.y * l.y);

@@ -83,7 +83,7 @@ __device__ __forceinline__ void f64_ion(const StepParams& P, const IonPtrs& S, c
             }
             if (state == 3u) {
                 state = 1u;
-                if (!contains_f64(P, pos)) {
+                if (!contains_f64<FIELD == FIELD_ARRAY_X>(P, pos)) {
                     state = 0u;
                     death = t;
                 }
@@ -146,11 +146,11 @@ __device__ __forceinline__ void f64_ion(const StepParams& P, const IonPtrs& S, c
             }
         }
         if (P.detect) {
-            keep_branch();
+            keep_branch<FIELD == FIELD_ARRAY_X>();
             if (isnan(arrival) && z_before < P.det_z && pos.z >= P.det_z)
                 arrival = t + dt * (P.det_z - z_before) / (pos.z - z_before);
         }
-        if (!(contains_f64(P, pos) & isfinite(pos.x) & isfinite(pos.y) & isfinite(pos.z) & isfinite(vel.x) &
+        if (!(contains_f64<FIELD == FIELD_ARRAY_X>(P, pos) & isfinite(pos.x) & isfinite(pos.y) & isfinite(pos.z) & isfinite(vel.x) &
               isfinite(vel.y) & isfinite(vel.z))) {
             state = 0u;
             death = t;
@@ -841,7 +841,7 @@ __device__ __forceinline__ void f32_ion(const StepParams& P, const IonPtrs& S, c
             }
             if (state == 3u) {
                 state = 1u;
-                if (!contains_f32(P, C, hi[0], hi[1], hi[2])) {
+                if (!contains_f32<FIELD == FIELD_ARRAY_X>(P, C, hi[0], hi[1], hi[2])) {
                     state = 0u;
                     death = t;
                 }
@@ -890,7 +890,7 @@ __device__ __forceinline__ void f32_ion(const StepParams& P, const IonPtrs& S, c
                 }
             }
             if (P.detect) {
-                keep_branch();
+                keep_branch<FIELD == FIELD_ARRAY_X>();
                 if (isnan(arrival)) {
                     const double zb = (double)z_before + (double)z_before_lo;
                     const double za = (double)hi[2] + (double)lo[2];
@@ -898,7 +898,7 @@ __device__ __forceinline__ void f32_ion(const StepParams& P, const IonPtrs& S, c
                         arrival = t + P.dt * (P.det_z - zb) / (za - zb);
                 }
             }
-            if (!(contains_f32(P, C, hi[0], hi[1], hi[2]) & isfinite(hi[0]) & isfinite(hi[1]) & isfinite(hi[2]) &
+            if (!(contains_f32<FIELD == FIELD_ARRAY_X>(P, C, hi[0], hi[1], hi[2]) & isfinite(hi[0]) & isfinite(hi[1]) & isfinite(hi[2]) &
                   isfinite(hi[3]) & isfinite(hi[4]) & isfinite(hi[5]))) {
                 state = 0u;
                 death = t;
@@ -990,7 +990,7 @@ __device__ __forceinline__ void surr_ion(const StepParams& P, const IonPtrs& S, 
             if (state == 2u && (!S.birth || t >= S.birth[here(ii)])) state = 3u;
             if (state == 3u) {
                 state = 1u;
-                if (!contains_f32(P, C, hi[0], hi[1], hi[2])) {
+                if (!contains_f32<FIELD == FIELD_ARRAY_X>(P, C, hi[0], hi[1], hi[2])) {
                     state = 0u;
                     S.death[here(ii)] = t;
                 }
@@ -1066,7 +1066,7 @@ __device__ __forceinline__ void surr_ion(const StepParams& P, const IonPtrs& S, 
         }
         if (live) {
             if (P.detect) {
-                keep_branch();
+                keep_branch<FIELD == FIELD_ARRAY_X>();
                 const double zb = (double)z_before + (double)z_before_lo;
                 const double za = (double)hi[2] + (double)lo[2];
                 if (zb < P.det_z && za >= P.det_z) {
@@ -1074,7 +1074,7 @@ __device__ __forceinline__ void surr_ion(const StepParams& P, const IonPtrs& S, 
                     if (isnan(arrival)) arrival = t + P.dt * (P.det_z - zb) / (za - zb);
                 }
             }
-            if (!(contains_f32(P, C, hi[0], hi[1], hi[2]) & isfinite(hi[0]) & isfinite(hi[1]) & isfinite(hi[2]) &
+            if (!(contains_f32<FIELD == FIELD_ARRAY_X>(P, C, hi[0], hi[1], hi[2]) & isfinite(hi[0]) & isfinite(hi[1]) & isfinite(hi[2]) &
                   isfinite(hi[3]) & isfinite(hi[4]) & isfinite(hi[5]))) {
                 state = 0u;
                 S.death[here(ii)] = t;
