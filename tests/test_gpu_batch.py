@@ -333,17 +333,16 @@ def surrogate_clouds(seed=4):
         w = W.ehss_surrogate_cloud(n, sigma, feat, counts, seed=50 + k, integrator=integ)
         clouds.append(dict(kind=f"ehss_surrogate_{k}", domain=w["domain"], physics=w["physics"],
                            species=w["species"], ensemble=w["ensemble"].copy(),
-                           ensemble0=w["ensemble"].copy(), t0=1e-9 * k,
+                           t0=1e-9 * k,
                            dt=w["dt"], n_steps=int(rng.integers(200, 600)), step_offset=11 * k))
     return clouds + mixed_clouds(seed)[:2]
 
 
 def test_batch_surrogate_clouds_equal_one_handle_per_cloud():
-    """The FP32 surrogate clouds run the single-cloud kernel's per-ion body,
-    but the compiler fuses multiply-adds differently in the two kernels, so
-    their FP32 trajectories differ by rounding, which the stochastic
-    collisions amplify: they are compared as ensembles (steps, collision
-    counts, mean drift); the ordinary clouds of the same batch ion by ion."""
+    """The surrogate clouds equal handles of their own bit for bit: the per-ion
+    body has its rounding written out, and an ion's MLP outputs do not depend on
+    the block it is evaluated in.  The ordinary clouds of the same batch ion by
+    ion."""
     params = np.load(SURROGATE_WEIGHTS)
     ref = surrogate_clouds()
     bat = copy_clouds(ref)
@@ -353,12 +352,8 @@ def test_batch_surrogate_clouds_equal_one_handle_per_cloud():
         assert a.t_end_s == b.t_end_s
         assert 0.0 < a.done_ms <= ms * 1.05 + 0.05
         if ca["kind"].startswith("ehss_surrogate"):
-            g, o, e0 = ca["ensemble"], cb["ensemble"], ca["ensemble0"]
-            assert a.ion_steps == b.ion_steps
-            assert a.collisions == pytest.approx(b.collisions, rel=0.02)
-            dz_g, dz_o = g.z - e0.z, o.z - e0.z
-            se = np.sqrt(dz_g.var() / g.n + dz_o.var() / o.n)
-            assert abs(dz_g.mean() - dz_o.mean()) < 4 * se, ca["kind"]
+            assert a.ion_steps == b.ion_steps and a.collisions == b.collisions
+            assert_same([ca], [cb])
         else:
             frac = close_fraction(ca["ensemble"], cb["ensemble"])
             assert frac >= 0.995, (ca["kind"], frac)
