@@ -165,11 +165,15 @@ __device__ __forceinline__ void f64_ion(const StepParams& P, const IonPtrs& S, c
     S.ncoll[i] = nc;
 }
 
-// Boris in general field arrays: two wavefronts per SIMD (256 registers and up to 30
-// spilled ones; with 282, one wavefront, 300,000 ions x 60 HSS steps took 1.89 ms,
-// now 1.38 ms).
+// Two wavefronts per SIMD where the compiler would take registers for one: Boris in
+// general field arrays (256 and up to 30 spilled; with 282 registers 300,000 ions x
+// 60 HSS steps took 1.89 ms, now 1.38 ms), EHSS with offline sets and over mixtures
+// in linear fields (256 and up to 12 spilled; 150,000 ions x 40 steps, offline sets
+// for one of three species 5.64 ms, now 4.24 ms).
 template <int INTEG, int FIELD, int COLL, bool SUB = false>
-__global__ void __launch_bounds__(256, (INTEG == 1 && FIELD == FIELD_ARRAY_X) ? 2 : 1) step_f64_kernel(const StepParams P, const IonPtrs S) {
+__global__ void __launch_bounds__(256, (FIELD == FIELD_LINEAR && (COLL == COLL_EHSS_TAB || COLL == COLL_EHSS_MIX)) ||
+                                       (INTEG == 1 && FIELD == FIELD_ARRAY_X) ? 2 : 1)
+    step_f64_kernel(const StepParams P, const IonPtrs S) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t pushed = 0, ncoll_launch = 0;
     if (i < P.n_ions) f64_ion<INTEG, FIELD, COLL, SUB, SUB>(P, S, P.order ? P.order[i] : i, pushed, ncoll_launch);

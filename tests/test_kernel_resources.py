@@ -1,6 +1,6 @@
 """Registers decide how many wavefronts a SIMD holds: the general field-array
-kernels (non-uniform axes, several terms) and the batch kernel with mixtures and
-arrays keep theirs."""
+kernels (non-uniform axes, several terms), the EHSS kernels and the batch kernel
+with mixtures and arrays keep theirs."""
 import os
 import re
 import shutil
@@ -37,7 +37,8 @@ def vgprs(tmp_path_factory):
 @pytest.mark.parametrize("kernel,waves", [
     ("step_f32_kernel<0, 3, 0, false>", 3), ("step_f32_kernel<0, 3, 1, false>", 3), ("step_f32_kernel<0, 3, 3, false>", 3),
     ("step_f32_kernel<1, 3, 0, false>", 3), ("step_f32_kernel<1, 3, 1, false>", 3), ("step_f32_kernel<1, 3, 3, false>", 3),
-    ("step_f64_kernel<1, 3, 1, false>", 2), ("step_f64_kernel<1, 3, 4, false>", 2), ("batch_kernel<1, true>", 3),
+    ("step_f64_kernel<1, 3, 1, false>", 2), ("step_f64_kernel<1, 3, 4, false>", 2), ("step_f64_kernel<0, 0, 5, false>", 2),
+    ("step_f64_kernel<0, 0, 6, false>", 2), ("batch_kernel<1, true>", 3),
     ("step_f64_ehss_kernel<0, 0>", 2), ("step_f64_ehss_kernel<1, 2>", 2)])
 def test_wavefronts_per_simd(vgprs, kernel, waves):
     assert 512 // (-(-vgprs[kernel] // 8) * 8) >= waves, vgprs[kernel]
